@@ -263,8 +263,8 @@ struct fsg_ctx {
     std::mutex mu;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    // interrupt flag the tile kernel reads at each refill: pinned host
-    // memory, written by the host while it waits for a tile
+    // interrupt flag that some waves of the tile kernel read at their refills:
+    // pinned host memory, written by the host while it waits for a tile
     uint32_t *stop_h = nullptr;
     const uint32_t *stop_d = nullptr;
     char *buf = nullptr;

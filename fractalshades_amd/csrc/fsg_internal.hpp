@@ -104,8 +104,9 @@ struct KArgs {
     // 1: the binary64 pass over the pixels whose stop_reason the binary32
     // pass set to REASON_UNSURE (every other pixel is skipped)
     int32_t redo; int32_t pad3;
-    // host-visible stop flag (pinned host memory) or null: once it is
-    // nonzero, lanes take no new pixel; the pixels in flight finish
+    // host-visible stop flag (pinned host memory) or null: once it is nonzero
+    // and a polling wave has seen it, lanes take no new pixel; the pixels in
+    // flight finish
     const uint32_t *stop;
 };
 

@@ -117,6 +117,9 @@ __device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) {
 // (a refill only once every lane is idle) within 1 % of 60.
 constexpr int REFILL_BATCH = 60;
 
+// added to a cursor, moves it past every slot of a launch
+constexpr unsigned long long CURSOR_DRAIN = 1ull << 44;
+
 template <class Model>
 __device__ __forceinline__ void tile_loop(const KArgs &a) {
     typename Model::State s;
@@ -141,6 +144,14 @@ __device__ __forceinline__ void tile_loop(const KArgs &a) {
     const unsigned xcd = blockIdx.x & 7u;
     const int gsh = min(14, max(6, 63 - __clzll((unsigned long long)max<int64_t>(a.npts >> 3, 1))));
     unsigned cur = 0;
+    // The interrupt flag is host memory, a read across PCIe: reads from every
+    // wave at every refill were served one after the other, 94 ns each (544 us
+    // for a 200x200 tile whose pixels take 35 us).  So one wave of every
+    // eighth block reads it, and only at a refill that writes finished pixels
+    // (the caller has just looked at the flag itself); when it is set, that
+    // wave drains every cursor, and no wave takes a new pixel.  The host call
+    // of the 200x200 tile: 973 -> 506 us.
+    const bool poller = a.stop != nullptr && xcd == 0u && __builtin_amdgcn_readfirstlane((int)threadIdx.x) < 64;
     bool active = false;      // iterating a pixel
     bool pending = false;     // holding a stopped pixel whose results are not written yet
     bool exhausted = false;   // every cursor is drained for this lane
@@ -155,6 +166,10 @@ __device__ __forceinline__ void tile_loop(const KArgs &a) {
         if (act == 0ull && want == 0ull) break;
         if (want != 0ull && (act == 0ull || 64 - __popcll(act) >= REFILL_BATCH)) {
             bool drained = false;     // this lane found the current cursor drained
+            if (poller && __ballot(pending) != 0ull) {
+                if (__hip_atomic_load(a.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0u && __lane_id() < 8)
+                    atomicAdd(cursors + 16 * __lane_id(), CURSOR_DRAIN);
+            }
             if (!active) {
                 if (pending) {
                     Model::finish(s, a, idx, reason);
@@ -169,19 +184,13 @@ __device__ __forceinline__ void tile_loop(const KArgs &a) {
                         (unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
                     const unsigned cx = (xcd + cur) & 7u;
                     unsigned long long base = 0;
-                    unsigned stop = 0;
-                    if ((int)__lane_id() == leader) {
+                    if ((int)__lane_id() == leader)
                         base = atomicAdd(cursors + 16 * cx, (unsigned long long)__popcll(mask));
-                        // the interrupt flag, read beside the cursor (its latency overlaps)
-                        if (a.stop) stop = __hip_atomic_load(a.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                    }
                     const unsigned lo = __builtin_amdgcn_readlane((unsigned)base, leader);
                     const unsigned hi = __builtin_amdgcn_readlane((unsigned)(base >> 32), leader);
                     const int64_t loc = (int64_t)(((unsigned long long)hi << 32) | lo) + rank;
                     idx = ((((loc >> gsh) << 3) + (int64_t)cx) << gsh) + (loc & ((1ll << gsh) - 1));
-                    if (__builtin_amdgcn_readlane(stop, leader) != 0u) {
-                        exhausted = true;          // interrupted: no new pixel
-                    } else if (idx < a.npts) {
+                    if (idx < a.npts) {
                         if (a.grid_w > 0) idx = grid_slot(idx, a.npts, a.grid_w);
                         // the binary64 pass takes only the pixels the binary32 one left unsure
                         if (!a.redo || a.stop_reason[idx] == REASON_UNSURE) {
