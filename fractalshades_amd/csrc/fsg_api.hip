@@ -256,6 +256,7 @@ struct fsg_ctx {
     int32_t zn_k_w = 0;
     double *xr_m = nullptr;
     double *M = nullptr, *r = nullptr;
+    int64_t *rk = nullptr;
     int64_t bla_len = 0;
     TablesX tx = {nullptr, nullptr, nullptr, nullptr, nullptr};
     int32_t stages = 0;
@@ -369,7 +370,7 @@ int fill_args(fsg_ctx *c, KArgs &a) {
     for (int q = 0; q < 4; q++) { t.bs[q] = c->bs[q]; t.bs_e[q] = c->bs_e[q]; }
     t.n_xr = c->d.n_xr; t.xr_idx = c->xr_idx; t.xr_m = c->xr_m; t.xr_e = c->xr_e;
     t.zn_k = c->zn_k; t.zn_k_w = c->zn_k_w;
-    t.M = c->M; t.r = c->r; t.stages_bla = c->stages; t.bla_on = c->d.bla_on;
+    t.M = c->M; t.r = c->r; t.rk = c->rk; t.stages_bla = c->stages; t.bla_on = c->d.bla_on;
     a.tx = c->tx;
     for (int q = 0; q < 4; q++) a.lin[q] = c->d.lin_mat[q];
     a.dx_m = c->d.dx_mant; a.dx_e = c->d.dx_exp;
@@ -678,14 +679,15 @@ int ctx_create(const fsg_ref_desc *desc, fsg_ctx *base, fsg_ctx **out) {
             if (hipMemsetAsync(c->M, 0, (size_t)(c->bla_len * dim) * sizeof(double), c->stream) != hipSuccess)
                 return cleanup(fail(FSG_E_HIP, "hipMemsetAsync BLA"));
         }
-        c->r = dalloc<double>((size_t)c->bla_len, err);
+        c->r = dalloc<double>((size_t)(2 * c->bla_len), err);     // the radii, then their keys
         if (err != hipSuccess) return cleanup(fail(FSG_E_NOMEM, "hipMalloc BLA"));
         c->owned.push_back(c->r);
         if (hipMemsetAsync(c->r, 0, (size_t)c->bla_len * sizeof(double), c->stream) != hipSuccess)
             return cleanup(fail(FSG_E_HIP, "hipMemsetAsync BLA"));
+        c->rk = reinterpret_cast<int64_t *>(c->r + c->bla_len);
         double kc = to_std(mkf(desc->kc_mant, desc->kc_exp));
         hipError_t be = launch_bla_build(desc->kind, c->d.degree, desc->flavor, c->Zn, c->L, kc,
-                                         desc->bla_eps, c->M, c->r, c->stages, c->stream, reuse_M);
+                                         desc->bla_eps, c->M, c->r, c->rk, c->stages, c->stream, reuse_M);
         if (be != hipSuccess) return cleanup(fail(FSG_E_HIP, std::string("BLA build: ") + hipGetErrorString(be)));
         if (hipStreamSynchronize(c->stream) != hipSuccess) return cleanup(fail(FSG_E_HIP, "BLA build sync"));
     }

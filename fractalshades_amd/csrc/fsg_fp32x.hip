@@ -685,7 +685,7 @@ struct BsF32 {
         const Tables &t = a.t;
         while (t.bla_on && (s.w & 7) == 0) {
             int32_t idx;
-            const int32_t st = bla_find(t, hypot2(s.xs, s.ys), s.w, idx);
+            const int32_t st = bla_find(t, hypot_key(s.xs, s.ys), s.w, idx);
             k.tries++;
             if (st == 0) break;
             {
@@ -777,7 +777,7 @@ __global__ void __launch_bounds__(1024) k_tile_lds_bsx(const KArgs a) {
     KArgs al = a;
     const int64_t K = p.K, KB = p.KB;
     al.t.Zn = stage<true>(lds, p.zn, a.t.Zn, K);
-    al.t.r = stage<true>(lds, p.r, a.t.r, KB);
+    al.t.rk = stage<true>(lds, p.r, a.t.rk, KB);
     al.t.M = stage<true>(lds, p.ax, a.t.M, KB * 8);     // the plan's ax slot: binary64 coefficients
     al.tx.ZRx = stage<true>(lds, p.zx, static_cast<const xsr *>(a.tx.ZRx), 2 * K);
     __syncthreads();

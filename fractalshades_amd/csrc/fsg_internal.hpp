@@ -41,7 +41,9 @@ struct Tables {
     // Xrange register's slot k - INT32_MIN
     const int32_t *zn_k;
     // BLA tree: 4 doubles (A, B complex) or 8 doubles (2x2 A, 2x2 B) per entry
-    const double *M; const double *r;
+    // (M), its radius (r) and the radius's key (rk, bla_key.hpp), which the
+    // binary64 lookups compare |z| with
+    const double *M; const double *r; const int64_t *rk;
     int32_t stages_bla; int32_t bla_on;
 };
 
@@ -124,8 +126,9 @@ int tile_lds_block(const LaunchCfg &cfg);        // lanes per block of select_ti
 bool lds_plan_full(const Tables &t, const LdsPlan &p);
 // radii_only: M already holds the coefficients (shared with another
 // context of the same orbit); write the radii r only
+// rk: the radii's keys, written after r
 hipError_t launch_bla_build(int kind, int degree, int flavor, const cplx *Zn, int32_t L,
-                            double kc, double eps, double *M, double *r, int32_t stages,
+                            double kc, double eps, double *M, double *r, int64_t *rk, int32_t stages,
                             hipStream_t stream, bool radii_only = false);
 int tile_kernel_blocks(const LaunchCfg &cfg);
 int grid_fill_blocks(const void *kernel);          // blocks filling the GPU at full occupancy

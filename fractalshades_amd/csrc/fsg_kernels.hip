@@ -148,6 +148,11 @@ __global__ void k_bla_merge(int32_t comp, int32_t stg, double kc, double eps, do
     }
 }
 
+__global__ void k_bla_keys(const double *r, int64_t n, int64_t *rk) {
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i < n) rk[i] = radius_key(r[i]);
+}
+
 // --------------------------------------------------------------------------
 // dispatch
 template <class Model> static tile_fn fn_of() { return k_tile<Model>; }
@@ -333,7 +338,7 @@ hipError_t launch_tile(const LaunchCfg &cfg, const KArgs &a, hipStream_t stream)
 
 template <bool RO>
 static hipError_t bla_build_t(int kind, int degree, int flavor, const cplx *Zn, int32_t L,
-                              double kc, double eps, double *M, double *r, int32_t stages,
+                              double kc, double eps, double *M, double *r, int64_t *rk, int32_t stages,
                               hipStream_t stream) {
     const int32_t comp = L >> 3;
     if (comp <= 0) return hipErrorInvalidValue;
@@ -366,14 +371,16 @@ static hipError_t bla_build_t(int kind, int degree, int flavor, const cplx *Zn, 
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    return hipSuccess;
+    const int64_t len = 2 * (int64_t)comp;
+    hipLaunchKernelGGL(k_bla_keys, dim3((unsigned)((len + tb - 1) / tb)), dim3(tb), 0, stream, r, len, rk);
+    return hipGetLastError();
 }
 
 hipError_t launch_bla_build(int kind, int degree, int flavor, const cplx *Zn, int32_t L,
-                            double kc, double eps, double *M, double *r, int32_t stages,
+                            double kc, double eps, double *M, double *r, int64_t *rk, int32_t stages,
                             hipStream_t stream, bool radii_only) {
-    return radii_only ? bla_build_t<true>(kind, degree, flavor, Zn, L, kc, eps, M, r, stages, stream)
-                      : bla_build_t<false>(kind, degree, flavor, Zn, L, kc, eps, M, r, stages, stream);
+    return radii_only ? bla_build_t<true>(kind, degree, flavor, Zn, L, kc, eps, M, r, rk, stages, stream)
+                      : bla_build_t<false>(kind, degree, flavor, Zn, L, kc, eps, M, r, rk, stages, stream);
 }
 
 }  // namespace fsg

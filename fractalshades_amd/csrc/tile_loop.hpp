@@ -4,6 +4,7 @@
 // from a pixel cursor.  Lanes that need work in the same wave share one
 // atomic: ballot + mbcnt hand out consecutive indices.
 #pragma once
+#include "bla_key.hpp"
 #include "fsg_internal.hpp"
 
 namespace fsg {
@@ -62,11 +63,8 @@ __device__ __forceinline__ int64_t grid_slot(int64_t s, int64_t n, int64_t w) {
 // start.  The highest valid stage is therefore found by bisection, with
 // about log2(stages) dependent loads instead of one per stage.
 // Returns the jump length (0 if no stage is valid) and the entry index.
-// SCALED: |z| = az 2^ez (the modulus of an extended-range mantissa and its
-// exponent); each radius is scaled by 2^-ez instead, which is exact.
-template <bool SCALED = false>
-__device__ __forceinline__ int32_t bla_find(const Tables &t, double az, int32_t w, int32_t &idx,
-                                            int32_t ez = 0) {
+// zk: the key of |z| (bla_key.hpp), compared with the radii's keys.
+__device__ __forceinline__ int32_t bla_find(const Tables &t, int64_t zk, int32_t w, int32_t &idx) {
     const int32_t it = w >> 3;
     const int32_t invalid_step = t.first_invalid - w;
     if (invalid_step <= 8) return 0;
@@ -78,14 +76,12 @@ __device__ __forceinline__ int32_t bla_find(const Tables &t, double az, int32_t 
         // the lowest stage first: invalid there, invalid at every stage (the
         // prefix property), which settles 40 % of the lookups of the 1e-300
         // frame in one read instead of about four (C2 -2.8 %)
-        const double r3 = t.r[2 * it];
-        if (!(az < (SCALED ? ldexp(r3, -ez) : r3))) return 0;
+        if (!(zk < t.rk[2 * it])) return 0;
         best = 3; lo = 4;
     }
     while (lo <= hi) {
         const int32_t mid = (lo + hi) >> 1;
-        const double r = t.r[2 * it + (1 << (mid - 3)) - 1];
-        if (az < (SCALED ? ldexp(r, -ez) : r)) { best = mid; lo = mid + 1; }
+        if (zk < t.rk[2 * it + (1 << (mid - 3)) - 1]) { best = mid; lo = mid + 1; }
         else hi = mid - 1;
     }
     if (best == 0) return 0;
@@ -298,7 +294,7 @@ __global__ void __launch_bounds__(BLOCK) k_tile_lds(const KArgs a) {
         t.bs_e[q] = stage<FULL>(lds, p.bs_e[q], a.t.bs_e[q], K);
     }
     t.zn_k = stage<FULL>(lds, p.zn_k, a.t.zn_k, K * a.t.zn_k_w);
-    t.r = stage<FULL>(lds, p.r, a.t.r, KB);
+    t.rk = stage<FULL>(lds, p.r, a.t.rk, KB);
     t.M = stage<FULL>(lds, p.M, a.t.M, KB * p.bla_dim);
     if ((FULL || p.dz >= 0) && a.t.dz) t.L = (int32_t)K;   // the wrapped dZndz value is staged at [K]
     __syncthreads();

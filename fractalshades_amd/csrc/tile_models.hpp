@@ -90,15 +90,15 @@ __device__ __forceinline__ void orbit_finish_bs(const OrbitRec<true> &o, const K
 // BLA lookup on binary64 |z| (ref_BLA_get, perturbation.py:2116-2170)
 __device__ __forceinline__ int32_t bla_lookup(const Tables &t, double zre, double zim,
                                               int32_t w, int32_t &idx) {
-    return bla_find(t, hypot2(zre, zim), w, idx);
+    return bla_find(t, hypot_key(zre, zim), w, idx);
 }
-// The same on an extended-range z: the modulus of its mantissa against the
-// radii scaled by 2^-e.  Where the binary64 copy of z is a normal number
+// The same on an extended-range z: the modulus of its mantissa scaled by
+// 2^e against the radii.  Where the binary64 copy of z is a normal number
 // this takes the decision hypot2 would (the prescale of hypot2 is the same
 // power of two); where that copy is subnormal or zero it keeps |z|'s
 // precision.
 __device__ __forceinline__ int32_t bla_lookup(const Tables &t, xl z, int32_t w, int32_t &idx) {
-    return bla_find<true>(t, sqrt(z.re * z.re + z.im * z.im), w, idx, z.e);
+    return bla_find(t, modulus_key(z.re * z.re + z.im * z.im, z.e), w, idx);
 }
 
 // The z^d + c step with the derivatives the launch computes (dz/dc when dc,
