@@ -113,6 +113,14 @@ __device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) {
 // (a refill only once every lane is idle) within 1 % of 60.
 constexpr int REFILL_BATCH = 60;
 
+// Models whose mantissas drift between renormalisations (LAZY) have them
+// renormalised every RENORM_TRIPS trips of the wave (one plain step of a lane
+// each, at most): a uniform branch, so the cost is the renormalisation's
+// divided by RENORM_TRIPS.
+constexpr unsigned RENORM_TRIPS = 8;
+template <class M, class = void> struct is_lazy { static constexpr bool value = false; };
+template <class M> struct is_lazy<M, decltype((void)M::LAZY)> { static constexpr bool value = M::LAZY; };
+
 // added to a cursor, moves it past every slot of a launch
 constexpr unsigned long long CURSOR_DRAIN = 1ull << 44;
 
@@ -148,6 +156,7 @@ __device__ __forceinline__ void tile_loop(const KArgs &a) {
     // wave drains every cursor, and no wave takes a new pixel.  The host call
     // of the 200x200 tile: 973 -> 506 us.
     const bool poller = a.stop != nullptr && xcd == 0u && __builtin_amdgcn_readfirstlane((int)threadIdx.x) < 64;
+    unsigned trips = 0;
     bool active = false;      // iterating a pixel
     bool pending = false;     // holding a stopped pixel whose results are not written yet
     bool exhausted = false;   // every cursor is drained for this lane
@@ -206,7 +215,10 @@ __device__ __forceinline__ void tile_loop(const KArgs &a) {
             // whole batch of slots without an unsure pixel) refill again on
             // the next trip
         }
+        trips++;
         if (active) {
+            if constexpr (is_lazy<Model>::value)
+                if (trips % RENORM_TRIPS == 0u) Model::renorm(s, a);
             reason = Model::step(s, a, k);
             if (reason >= 0) {
                 active = false;
