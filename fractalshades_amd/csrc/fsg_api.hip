@@ -682,7 +682,7 @@ int ctx_create(const fsg_ref_desc *desc, fsg_ctx *base, fsg_ctx **out) {
         c->r = dalloc<double>((size_t)(2 * c->bla_len), err);     // the radii, then their keys
         if (err != hipSuccess) return cleanup(fail(FSG_E_NOMEM, "hipMalloc BLA"));
         c->owned.push_back(c->r);
-        if (hipMemsetAsync(c->r, 0, (size_t)c->bla_len * sizeof(double), c->stream) != hipSuccess)
+        if (hipMemsetAsync(c->r, 0, (size_t)(2 * c->bla_len) * sizeof(double), c->stream) != hipSuccess)
             return cleanup(fail(FSG_E_HIP, "hipMemsetAsync BLA"));
         c->rk = reinterpret_cast<int64_t *>(c->r + c->bla_len);
         double kc = to_std(mkf(desc->kc_mant, desc->kc_exp));

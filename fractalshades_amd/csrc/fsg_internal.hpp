@@ -126,7 +126,7 @@ int tile_lds_block(const LaunchCfg &cfg);        // lanes per block of select_ti
 bool lds_plan_full(const Tables &t, const LdsPlan &p);
 // radii_only: M already holds the coefficients (shared with another
 // context of the same orbit); write the radii r only
-// rk: the radii's keys, written after r
+// rk: the radii's keys, written with r
 hipError_t launch_bla_build(int kind, int degree, int flavor, const cplx *Zn, int32_t L,
                             double kc, double eps, double *M, double *r, int64_t *rk, int32_t stages,
                             hipStream_t stream, bool radii_only = false);

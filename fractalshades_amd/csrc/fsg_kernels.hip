@@ -76,8 +76,13 @@ __device__ __forceinline__ HEntry load_h(const double *M, const double *r, int64
     HEntry e; e.A = mk(M[4 * i], M[4 * i + 1]); e.B = mk(M[4 * i + 2], M[4 * i + 3]); e.r = r[i];
     return e;
 }
-__device__ __forceinline__ void store_h(double *M, double *r, int64_t i, const HEntry &e) {
-    M[4 * i] = e.A.re; M[4 * i + 1] = e.A.im; M[4 * i + 2] = e.B.re; M[4 * i + 3] = e.B.im; r[i] = e.r;
+__device__ __forceinline__ void store_r(double *r, int64_t *rk, int64_t i, double v) {
+    r[i] = v;
+    rk[i] = radius_key(v);
+}
+__device__ __forceinline__ void store_h(double *M, double *r, int64_t *rk, int64_t i, const HEntry &e) {
+    M[4 * i] = e.A.re; M[4 * i + 1] = e.A.im; M[4 * i + 2] = e.B.re; M[4 * i + 3] = e.B.im;
+    store_r(r, rk, i, e.r);
 }
 __device__ __forceinline__ BEntry load_b(const double *M, const double *r, int64_t i) {
     BEntry e;
@@ -85,16 +90,16 @@ __device__ __forceinline__ BEntry load_b(const double *M, const double *r, int64
     e.r = r[i];
     return e;
 }
-__device__ __forceinline__ void store_b(double *M, double *r, int64_t i, const BEntry &e) {
+__device__ __forceinline__ void store_b(double *M, double *r, int64_t *rk, int64_t i, const BEntry &e) {
     for (int q = 0; q < 8; q++) M[8 * i + q] = e.M[q];
-    r[i] = e.r;
+    store_r(r, rk, i, e.r);
 }
 
 // RADII_ONLY: the coefficients M are already in place (a context sharing
 // another's orbit and BLA coefficients); only the radii, which depend on kc
 // and eps, are written
 template <int KIND, int DEG, bool RADII_ONLY>
-__global__ void k_bla0_holo(const cplx *Zn, int32_t comp, double kc, double eps, double *M, double *r) {
+__global__ void k_bla0_holo(const cplx *Zn, int32_t comp, double kc, double eps, double *M, double *r, int64_t *rk) {
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= comp) return;
     HEntry e[8];
@@ -108,12 +113,12 @@ __global__ void k_bla0_holo(const cplx *Zn, int32_t comp, double kc, double eps,
 #pragma unroll
     for (int j = 0; j < 2; j++) e[j] = merge(e[2 * j], e[2 * j + 1], kc, eps);
     const HEntry o = merge(e[0], e[1], kc, eps);
-    if constexpr (RADII_ONLY) r[2 * (int64_t)i] = o.r;
-    else store_h(M, r, 2 * (int64_t)i, o);
+    if constexpr (RADII_ONLY) store_r(r, rk, 2 * (int64_t)i, o.r);
+    else store_h(M, r, rk, 2 * (int64_t)i, o);
 }
 
 template <int FL, bool RADII_ONLY>
-__global__ void k_bla0_bs(const cplx *Zn, int32_t comp, double kc, double eps, double *M, double *r) {
+__global__ void k_bla0_bs(const cplx *Zn, int32_t comp, double kc, double eps, double *M, double *r, int64_t *rk) {
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= comp) return;
     BEntry e[8];
@@ -127,13 +132,13 @@ __global__ void k_bla0_bs(const cplx *Zn, int32_t comp, double kc, double eps, d
     for (int j = 0; j < 4; j++) e[j] = merge(e[2 * j], e[2 * j + 1], kc, eps);
     for (int j = 0; j < 2; j++) e[j] = merge(e[2 * j], e[2 * j + 1], kc, eps);
     const BEntry o = merge(e[0], e[1], kc, eps);
-    if constexpr (RADII_ONLY) r[2 * (int64_t)i] = o.r;
-    else store_b(M, r, 2 * (int64_t)i, o);
+    if constexpr (RADII_ONLY) store_r(r, rk, 2 * (int64_t)i, o.r);
+    else store_b(M, r, rk, 2 * (int64_t)i, o);
 }
 
 // one stored level: merge i in [0, floor(comp / 2^stg)) of stage stg
 template <bool BS, bool RADII_ONLY>
-__global__ void k_bla_merge(int32_t comp, int32_t stg, double kc, double eps, double *M, double *r) {
+__global__ void k_bla_merge(int32_t comp, int32_t stg, double kc, double eps, double *M, double *r, int64_t *rk) {
     const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     const int64_t step = 1LL << stg;
     if (t >= comp / step) return;
@@ -141,16 +146,11 @@ __global__ void k_bla_merge(int32_t comp, int32_t stg, double kc, double eps, do
     const int64_t i1 = 2 * i + (step / 2 - 1), i2 = 2 * ii + (step / 2 - 1), ir = 2 * i + (step - 1);
     if constexpr (BS) {
         const BEntry o = merge(load_b(M, r, i1), load_b(M, r, i2), kc, eps);
-        if constexpr (RADII_ONLY) r[ir] = o.r; else store_b(M, r, ir, o);
+        if constexpr (RADII_ONLY) store_r(r, rk, ir, o.r); else store_b(M, r, rk, ir, o);
     } else {
         const HEntry o = merge(load_h(M, r, i1), load_h(M, r, i2), kc, eps);
-        if constexpr (RADII_ONLY) r[ir] = o.r; else store_h(M, r, ir, o);
+        if constexpr (RADII_ONLY) store_r(r, rk, ir, o.r); else store_h(M, r, rk, ir, o);
     }
-}
-
-__global__ void k_bla_keys(const double *r, int64_t n, int64_t *rk) {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i < n) rk[i] = radius_key(r[i]);
 }
 
 // --------------------------------------------------------------------------
@@ -344,17 +344,17 @@ static hipError_t bla_build_t(int kind, int degree, int flavor, const cplx *Zn, 
     if (comp <= 0) return hipErrorInvalidValue;
     const int tb = 128;
     dim3 g0((comp + tb - 1) / tb);
-    if (kind == KIND_M2) hipLaunchKernelGGL((k_bla0_holo<KIND_M2, 2, RO>), g0, dim3(tb), 0, stream, Zn, comp, kc, eps, M, r);
+    if (kind == KIND_M2) hipLaunchKernelGGL((k_bla0_holo<KIND_M2, 2, RO>), g0, dim3(tb), 0, stream, Zn, comp, kc, eps, M, r, rk);
     else if (kind == KIND_MN) {
         switch (degree) {
-#define FSG_MN(D) case D: hipLaunchKernelGGL((k_bla0_holo<KIND_MN, D, RO>), g0, dim3(tb), 0, stream, Zn, comp, kc, eps, M, r); break;
+#define FSG_MN(D) case D: hipLaunchKernelGGL((k_bla0_holo<KIND_MN, D, RO>), g0, dim3(tb), 0, stream, Zn, comp, kc, eps, M, r, rk); break;
             FSG_MN(2) FSG_MN(3) FSG_MN(4) FSG_MN(5) FSG_MN(6) FSG_MN(7) FSG_MN(8)
 #undef FSG_MN
             default: return hipErrorInvalidValue;
         }
     } else {
         switch (flavor) {
-#define FSG_BS(F) case F: hipLaunchKernelGGL((k_bla0_bs<F, RO>), g0, dim3(tb), 0, stream, Zn, comp, kc, eps, M, r); break;
+#define FSG_BS(F) case F: hipLaunchKernelGGL((k_bla0_bs<F, RO>), g0, dim3(tb), 0, stream, Zn, comp, kc, eps, M, r, rk); break;
             FSG_BS(1) FSG_BS(2) FSG_BS(3) FSG_BS(4) FSG_BS(5)
 #undef FSG_BS
             default: return hipErrorInvalidValue;
@@ -366,14 +366,12 @@ static hipError_t bla_build_t(int kind, int degree, int flavor, const cplx *Zn, 
         int64_t nm = comp >> stg;
         if (nm <= 0) break;
         dim3 g((unsigned)((nm + tb - 1) / tb));
-        if (kind == KIND_BS) hipLaunchKernelGGL((k_bla_merge<true, RO>), g, dim3(tb), 0, stream, comp, stg, kc, eps, M, r);
-        else hipLaunchKernelGGL((k_bla_merge<false, RO>), g, dim3(tb), 0, stream, comp, stg, kc, eps, M, r);
+        if (kind == KIND_BS) hipLaunchKernelGGL((k_bla_merge<true, RO>), g, dim3(tb), 0, stream, comp, stg, kc, eps, M, r, rk);
+        else hipLaunchKernelGGL((k_bla_merge<false, RO>), g, dim3(tb), 0, stream, comp, stg, kc, eps, M, r, rk);
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    const int64_t len = 2 * (int64_t)comp;
-    hipLaunchKernelGGL(k_bla_keys, dim3((unsigned)((len + tb - 1) / tb)), dim3(tb), 0, stream, r, len, rk);
-    return hipGetLastError();
+    return hipSuccess;
 }
 
 hipError_t launch_bla_build(int kind, int degree, int flavor, const cplx *Zn, int32_t L,
