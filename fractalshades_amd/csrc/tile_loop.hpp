@@ -156,6 +156,9 @@ __device__ __forceinline__ void tile_loop(const KArgs &a) {
     // wave drains every cursor, and no wave takes a new pixel.  The host call
     // of the 200x200 tile: 973 -> 506 us.
     const bool poller = a.stop != nullptr && xcd == 0u && __builtin_amdgcn_readfirstlane((int)threadIdx.x) < 64;
+    // an escape radius past 2^30 lets one step multiply a mantissa further:
+    // renormalised on every trip there
+    const unsigned renorm_mask = a.M2 > 0x1p60 ? 0u : RENORM_TRIPS - 1u;
     unsigned trips = 0;
     bool active = false;      // iterating a pixel
     bool pending = false;     // holding a stopped pixel whose results are not written yet
@@ -218,7 +221,7 @@ __device__ __forceinline__ void tile_loop(const KArgs &a) {
         trips++;
         if (active) {
             if constexpr (is_lazy<Model>::value)
-                if (trips % RENORM_TRIPS == 0u) Model::renorm(s, a);
+                if ((trips & renorm_mask) == 0u) Model::renorm(s, a);
             reason = Model::step(s, a, k);
             if (reason >= 0) {
                 active = false;

@@ -267,24 +267,28 @@ struct HoloStd {
 // rounding, so every operation rounds exactly like the reference's Xrange
 // record.
 //
-// z^2 + c (LAZY): the mantissas of z, dz/dc and dz/dz drift freely between
+// LAZY: the mantissas of z, dz/dc and dz/dz drift freely between
 // renormalisations, which the tile loop asks for every RENORM_TRIPS trips
 // (and the BLA jump and the rebase for what they read); each keeps one
 // exponent, and a sum shifts its other operand -- c, or the path's term -- to
-// that exponent instead of aligning both on the larger one.  Z + z and z + 2 Z
-// are formed in binary64 from z's binary64 copy: Z is in range, so a z that
-// underflows there is far below the rounding of the sum.  Two exceptions
+// that exponent instead of aligning both on the larger one.  z^2 + c: Z + z
+// and z + 2 Z are formed in binary64 from z's binary64 copy: Z is in range,
+// so a z that underflows there is far below the rounding of the sum.
+// z^d + c: the same for the factors of every binomial term.  Two exceptions
 // leave the straight line: an orbit point below 2^LOW_Z (zero, the Xrange
-// register), whose sums are aligned as the general extended-range sum does,
-// and an operand so much larger than the quantity it is added to (|shift| >
-// FAR: a quantity that is still zero, mostly) that the exponent moves to the
-// operand's first.  A mantissa then stays within 2^+-700: a step multiplies it
-// by at least 2^-73 (|Z| >= 2^-20, 53 bits of cancellation) and at most
-// 2 |Z + z|, and adds no more than 2^FAR times the operand's mantissa.
-// The loop is bound by vector instruction issue: a step takes 104 instructions
-// (dz/dc and dz/dz on; 58 are the algorithmic flops) where normalising every
-// result and aligning every sum took 174.  2048x2048 frames with it: 1e-300
-// 999 -> 792 us, 1e-2000 1212 -> 1027 us, interior-dominated 24.7 -> 22.3 ms.
+// register) or above 2^HIGH_Z, with which the factors take the exponent of
+// the larger of Z and z; and an operand so much larger than the quantity it
+// is added to (shift > FAR: a quantity that is still zero, mostly) that the
+// exponent moves to the operand's first.  A mantissa then stays within
+// 2^+-700: a step multiplies it by at least 2^(LOW_Z (d - 1)) but for
+// cancellation and at most d |Z + z|^(d - 1), and adds no more than 2^FAR
+// times the operand's mantissa.
+// The loop is bound by vector instruction issue: a z^2 + c step takes 104
+// instructions (dz/dc and dz/dz on; 58 are the algorithmic flops) where
+// normalising every result and aligning every sum took 174.  2048x2048 frames
+// with it: 1e-300 999 -> 792 us, 1e-2000 1212 -> 1027 us, interior-dominated
+// 24.7 -> 22.3 ms; 1920x1080 at 1e-800: z^3 + c 850 -> 729 us, z^6 + c 868 ->
+// 666 us.
 // DER >= 0 fixes the derivatives at compile time (bit 0: dz/dc, bit 1:
 // dz/dz): the step is then one block of straight-line code, which the
 // compiler schedules across the z, dz/dc and dz/dz recurrences; DER = -1
@@ -294,8 +298,34 @@ struct HoloXr {
     __device__ static bool DC_ON(const KArgs &a) { if constexpr (DER >= 0) return (DER & 1) != 0; else return a.calc_dc != 0; }
     __device__ static bool DZ_ON(const KArgs &a) { if constexpr (DER >= 0) return (DER & 2) != 0; else return a.calc_dz != 0; }
     struct State { xl z, d, h, c; cplx zs; int32_t w, n; bool dyn, nul; OrbitRec<ORB> orb; };
-    static constexpr bool LAZY = KIND == KIND_M2;
-    static constexpr int32_t LOW_Z = -20, FAR = 256;
+    static constexpr bool LAZY = true;
+    static constexpr int32_t LOW_Z = (KIND == KIND_M2) ? -20 : -60 / (DEG - 1), HIGH_Z = 60, FAR = 256;
+
+    // The z^d + c derivative recurrence of one quantity: its delta v 2^e, the
+    // orbit's value Z 2^eG, and the running term t 2^e (times 2^(q eK)).  The
+    // inner sum is in the orbit value's scale, far above the delta's: s1
+    // takes v's scale there, s2 the product with z back.
+    struct Deriv {
+        cplx v, Z, t;
+        int32_t e, eG, s1, s2;
+        __device__ void set(const xl &d, const xz &Zp, int32_t et) {
+            v = mk(d.re, d.im); e = d.e; Z = mk(Zp.re, Zp.im);
+            eG = Zp.e < XL_ZERO_E / 2 ? e : Zp.e;          // a zero value has no scale of its own
+            s1 = e - eG; s2 = et - s1;
+        }
+        // the exponents moved together where a shift is out of range
+        __device__ void near(int32_t et) {
+            if (s1 > FAR) { Z = mk(ldexp(Z.re, -s1), ldexp(Z.im, -s1)); eG = e; s1 = 0; s2 = et; }
+            if (s2 > FAR) { v = mk(ldexp(v.re, -s2), ldexp(v.im, -s2)); e += s2; s1 = e - eG; s2 = et - s1; }
+        }
+        // t <- v mul + z (t + C dZ), t = v at the first term
+        __device__ void term(cplx z, cplx mul, cplx CdZ, bool first) {
+            const cplx u = first ? v : t;
+            const cplx g = z * (mk(ldexp(u.re, s1), ldexp(u.im, s1)) + CdZ);
+            const cplx p = v * mul;
+            t = mk(p.re + ldexp(g.re, s2), p.im + ldexp(g.im, s2));
+        }
+    };
 
     __device__ static void renorm(State &s, const KArgs &a) {
         s.z = xl_of(as_z(s.z));
@@ -332,7 +362,7 @@ struct HoloXr {
 
     __device__ static int step(State &s, const KArgs &a, Counters &k) {
         const Tables &t = a.t;
-        if (LAZY && t.bla_on && (s.w & 7) == 0) s.z = xl_of(as_z(s.z));
+        if (t.bla_on && (s.w & 7) == 0) s.z = xl_of(as_z(s.z));
         while (t.bla_on && (s.w & 7) == 0) {
             int32_t idx;
             int32_t st = bla_lookup(t, s.z, s.w, idx);
@@ -345,8 +375,8 @@ struct HoloXr {
                 s.w += st;
                 // a coefficient can be near the end of the binary64 range: it
                 // multiplies normalised mantissas only
-                if (LAZY && DC_ON(a)) s.d = xl_of(as_z(s.d));
-                if (LAZY && DZ_ON(a)) s.h = xl_of(as_z(s.h));
+                if (DC_ON(a)) s.d = xl_of(as_z(s.d));
+                if (DZ_ON(a)) s.h = xl_of(as_z(s.h));
                 s.z = add_n(as_z(s.z) * A, as_z(s.c) * B);
                 s.zs = to_std(s.z);
                 if (DC_ON(a)) s.d = mul_n(as_z(s.d), A);
@@ -364,15 +394,12 @@ struct HoloXr {
         const int32_t k0 = t.zn_k[s.w];
         const cplx Z0 = t.Zn[s.w], Z1 = t.Zn[w1];
         xz Zd = xz_zero(), Zh = xz_zero(), H1 = xz_zero();
-        if (DC_ON(a)) {
-            Zd = DCz(t, s.w);
-            if constexpr (!LAZY) Zd = s.dyn ? xz_zero() : Zd;
-        }
+        if (DC_ON(a)) Zd = DCz(t, s.w);
         if (DZ_ON(a)) {
             Zh = DZz(t, s.nul ? 0 : s.w);
             if constexpr (KIND == KIND_M2) H1 = DZz(t, s.nul ? 0 : (s.n == t.order ? t.L : w1));
         }
-        if constexpr (LAZY) {
+        if constexpr (KIND == KIND_M2) {
             // mandelbrot_M2.py:607-622: z (z + 2 Z) + c, 2 ((Z + z) d + Zd z)
             cplx A = s.zs + Z0;                                      // Z + z
             cplx W = mk(__builtin_fma(2., Z0.re, s.zs.re), __builtin_fma(2., Z0.im, s.zs.im));   // z + 2 Z
@@ -383,6 +410,7 @@ struct HoloXr {
                     const xl Zr = ZRv(t, k0, Z0);
                     s.z = xl_of(as_z(s.z));
                     eK = max(Zr.e, s.z.e);
+                    if (eK < XL_ZERO_E / 2) eK = 0;              // Z = z = 0
                     const int32_t sZ = shift_of(Zr.e, eK), sz = shift_of(s.z.e, eK);
                     const cplx Zk = mk(ldexp(Zr.re, sZ), ldexp(Zr.im, sZ)), zk = mk(ldexp(s.z.re, sz), ldexp(s.z.im, sz));
                     A = Zk + zk;
@@ -412,28 +440,69 @@ struct HoloXr {
             s.z.re = u.re + ldexp(s.c.re, sz); s.z.im = u.im + ldexp(s.c.im, sz); s.z.e = ez;
             s.zs = mk(ldexp(s.z.re, ez), ldexp(s.z.im, ez));
         } else {
-            const xz Zr = as_z(ZRv(t, k0, Z0));
-            const xz z0 = as_z(s.z);
-            // the last sums normalised at once (add_n: no zero test of their own)
-            s.z = mn_step<DEG>(z0, Zr, as_z(s.c), DC_ON(a), DZ_ON(a), s.d, s.h, as_z(s.d), as_z(s.h),
-                               Zd, Zh, [](xz u, xz v) { return add_n(u, v); });
-        }
-        if constexpr (KIND == KIND_MN) {
+            // mandelbrot_Mn.py:646-729 (p_zn_derivs of models.hpp).  zk, Zk: z
+            // and Z in units of 2^eK; the running factor mul of term q is then
+            // in units of 2^(q eK), and tmp = z mul on z's mantissa comes back
+            // to that scale with the shift et.
+            cplx Zk = Z0, zk = s.zs;
+            int32_t eK = 0;
+            const bool far_z = (uint32_t)(k0 - LOW_Z) > (uint32_t)(HIGH_Z - LOW_Z);
+            if (far_z || s.dyn) {
+                if (s.dyn) Zd = xz_zero();
+                if (far_z) {
+                    const xl Zr = ZRv(t, k0, Z0);
+                    s.z = xl_of(as_z(s.z));
+                    eK = max(Zr.e, s.z.e);
+                    if (eK < XL_ZERO_E / 2) eK = 0;              // Z = z = 0
+                    const int32_t sZ = shift_of(Zr.e, eK), sz = shift_of(s.z.e, eK);
+                    Zk = mk(ldexp(Zr.re, sZ), ldexp(Zr.im, sZ));
+                    zk = mk(ldexp(s.z.re, sz), ldexp(s.z.im, sz));
+                }
+            }
+            const int32_t et = s.z.e - eK;
+            int32_t ez = s.z.e + (DEG - 1) * eK, sz = s.c.e - ez;
+            Deriv D[2];
+            if (DC_ON(a)) D[0].set(s.d, Zd, et);
+            if (DZ_ON(a)) D[1].set(s.h, Zh, et);
+            int32_t far = sz;
+            if (DC_ON(a)) far = max(far, max(D[0].s1, D[0].s2));
+            if (DZ_ON(a)) far = max(far, max(D[1].s1, D[1].s2));
+            int32_t cut = 0;
+            if (far > FAR) {
+                if (sz > FAR) { cut = -sz; ez += sz; sz = 0; }
+                if (DC_ON(a)) D[0].near(et);
+                if (DZ_ON(a)) D[1].near(et);
+            }
+            const cplx z = mk(s.z.re, s.z.im);
+            cplx mul = zk + scale(cbinom(DEG, 1), Zk);
+            cplx tmp = z * mul;
+            if (DC_ON(a)) D[0].term(z, mul, scale(cbinom(DEG, 1), D[0].Z), true);
+            if (DZ_ON(a)) D[1].term(z, mul, scale(cbinom(DEG, 1), D[1].Z), true);
+            cplx Zpk = Zk;
+#pragma unroll
+            for (int q = 2; q < DEG; q++) {
+                const cplx qZ = scale((double)q, Zpk);
+                Zpk = Zpk * Zk;
+                mul = mk(ldexp(tmp.re, et), ldexp(tmp.im, et)) + scale(cbinom(DEG, q), Zpk);
+                if (DC_ON(a)) D[0].term(z, mul, scale(cbinom(DEG, q), qZ * D[0].Z), false);
+                if (DZ_ON(a)) D[1].term(z, mul, scale(cbinom(DEG, q), qZ * D[1].Z), false);
+                tmp = z * mul;
+            }
+            if (cut != 0) tmp = mk(ldexp(tmp.re, cut), ldexp(tmp.im, cut));
+            if (DC_ON(a)) { s.d.re = D[0].t.re; s.d.im = D[0].t.im; s.d.e = D[0].e + (DEG - 1) * eK; }
+            if (DZ_ON(a)) { s.h.re = D[1].t.re; s.h.im = D[1].t.im; s.h.e = D[1].e + (DEG - 1) * eK; }
+            s.z.re = tmp.re + ldexp(s.c.re, sz); s.z.im = tmp.im + ldexp(s.c.im, sz); s.z.e = ez;
+            s.zs = mk(ldexp(s.z.re, ez), ldexp(s.z.im, ez));
             if (DZ_ON(a)) H1 = DZz(t, s.nul ? 0 : (s.n == t.order ? t.L : w1));
         }
-        if constexpr (!LAZY) s.zs = to_std(s.z);
         s.w = w1;
         // the stop and rebase tests evaluated together, as in HoloStd
         bool t_int = false;
-        if constexpr (LAZY) {
-            if (DZ_ON(a)) {
-                // in binary64: what underflows or overflows there lies far on
-                // one side of eps
-                const cplx q = mk(ldexp(s.h.re, s.h.e) + ldexp(H1.re, H1.e), ldexp(s.h.im, s.h.e) + ldexp(H1.im, H1.e));
-                t_int = q.re * q.re + q.im * q.im < a.eps2;
-            }
-        } else {
-            t_int = DZ_ON(a) && abs2_lt(add_raw(as_z(s.h), H1), a.eps2);
+        if (DZ_ON(a)) {
+            // in binary64: what underflows or overflows there lies far on one
+            // side of eps
+            const cplx q = mk(ldexp(s.h.re, s.h.e) + ldexp(H1.re, H1.e), ldexp(s.h.im, s.h.e) + ldexp(H1.im, H1.e));
+            t_int = q.re * q.re + q.im * q.im < a.eps2;
         }
         const cplx ZZ = s.zs + Z1;
         const bool t_esc = ZZ.re * ZZ.re + ZZ.im * ZZ.im > a.M2;
@@ -453,7 +522,7 @@ struct HoloXr {
         if (!reb_div) {
             s.dyn = dyn;
             if (s.dyn) {
-                if constexpr (LAZY) s.z = xl_of(as_z(s.z));
+                s.z = xl_of(as_z(s.z));
                 ZZx = s.z + ZRv(t, t.zn_k[w1], Z1);
                 reb = le_abs2(ZZx, s.z);
             }
@@ -462,12 +531,9 @@ struct HoloXr {
             if (reb_div) { s.zs = ZZ; s.z = xl_of(ZZ); }
             else { s.z = ZZx; s.zs = to_std(ZZx); }
             // the path values unnormalised: the sum's normalisation covers them
-            if constexpr (LAZY) {
-                if (DC_ON(a)) s.d = xl_of(as_z(s.d));
-                if (DZ_ON(a)) s.h = xl_of(as_z(s.h));
-            }
-            if (DC_ON(a)) s.d = add_n(as_z(s.d), DCz(t, s.w));
+            if (DC_ON(a)) s.d = add_n(as_z(xl_of(as_z(s.d))), DCz(t, s.w));
             if (DZ_ON(a)) {
+                s.h = xl_of(as_z(s.h));
                 if (!s.nul) s.h = add_n(as_z(s.h), H1);   // dZndz at w (at L after a full period)
                 s.nul = true;
             }
@@ -479,7 +545,7 @@ struct HoloXr {
 
     __device__ static void finish(State &s, const KArgs &a, int64_t i, int reason) {
         const int64_t n = a.ld;
-        if constexpr (LAZY) renorm(s, a);
+        renorm(s, a);
         cplx z = to_std(s.z) + a.t.Zn[s.w];
         a.Z[2 * i] = z.re; a.Z[2 * i + 1] = z.im;
         int f = 1;
