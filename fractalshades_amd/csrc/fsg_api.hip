@@ -524,9 +524,11 @@ int tile_staged(fsg_ctx *c, const double *c_pix, int64_t n, int64_t grid_w, doub
 // copy for the life of the process, and no call allocates.  Its address on a
 // device comes from hipGetSymbolAddress, taken once per device with that
 // device current; host code uses that address, never the array's name.
-constexpr size_t NOALLOC_WORK_BYTES = 4096;      // cursors and counters, then the tile staging
-static_assert(NOALLOC_WORK_BYTES >= WORK_WORDS * sizeof(unsigned long long), "workspace does not fit");
-static __device__ __align__(256) unsigned char scratch[FSG_NOALLOC_SCRATCH_BYTES];
+// The cursors and counters lie past the FSG_NOALLOC_SCRATCH_BYTES of the tile
+// staging, of which NOALLOC_RESERVED stay unused: the limit on a tile counts
+// them.
+constexpr size_t NOALLOC_RESERVED = 4096;
+static __device__ __align__(256) unsigned char scratch[FSG_NOALLOC_SCRATCH_BYTES + WORK_WORDS * sizeof(unsigned long long)];
 
 struct ScratchDev {
     std::once_flag once;
@@ -819,7 +821,7 @@ int fsg_tile_grid_noalloc(fsg_ctx *c, const double *c_pix, int64_t n, int64_t gr
     if (n < 0 || (n > 0 && (!c_pix || !Z || !U || !stop_reason || !stop_iter)))
         return fail(FSG_E_INVALID, "bad tile buffers");
     if (grid_w < 0) return fail(FSG_E_INVALID, "negative grid width");
-    const size_t need = NOALLOC_WORK_BYTES + staging_bytes(c, n);
+    const size_t need = NOALLOC_RESERVED + staging_bytes(c, n);
     if (need > FSG_NOALLOC_SCRATCH_BYTES)
         return fail(FSG_E_RANGE, "fsg_tile_grid_noalloc: a tile of " + std::to_string(n) + " pixels needs " +
                                  std::to_string(need) + " bytes of device staging, above the " +
@@ -834,7 +836,7 @@ int fsg_tile_grid_noalloc(fsg_ctx *c, const double *c_pix, int64_t n, int64_t gr
     std::lock_guard<std::mutex> lk_dev(g_scratch[c->device].mu);
     std::lock_guard<std::mutex> lk(c->mu);
     return tile_staged(c, c_pix, n, grid_w, Z, U, stop_reason, stop_iter, interrupted, stats,
-                       base + NOALLOC_WORK_BYTES, reinterpret_cast<unsigned long long *>(base));
+                       base, reinterpret_cast<unsigned long long *>(base + FSG_NOALLOC_SCRATCH_BYTES));
 }
 
 int fsg_tile_device(fsg_ctx *c, const double *d_c_pix, int64_t n, double *d_Z, int32_t *d_U,

@@ -504,23 +504,23 @@ struct HoloS32 {
         return -1;
     }
 
-    __device__ static void finish(const State &s, const KArgs &a, int64_t i, int reason) {
-        a.stop_reason[i] = (int8_t)reason;
+    __device__ static void finish(const State &s, const KArgs &a, const KArgs &g, int64_t i, int reason) {
+        g.stop_reason[i] = (int8_t)reason;
         if (reason == REASON_UNSURE) return;        // the binary64 pass writes this pixel
-        const int64_t n = a.ld;
+        const int64_t n = g.ld;
         const cplx z = zd(s) + a.t.Zn[s.w];
-        a.Z[2 * i] = z.re; a.Z[2 * i + 1] = z.im;
+        g.Z[2 * i] = z.re; g.Z[2 * i + 1] = z.im;
         int f = 1;
         if (a.calc_dz) {
             const cplx h = xs_to_d(xs_norm(s.h.x, s.h.y, s.h.e));
-            a.Z[2 * (n + i)] = h.re; a.Z[2 * (n + i) + 1] = h.im;
+            g.Z[2 * (n + i)] = h.re; g.Z[2 * (n + i) + 1] = h.im;
             f = 2;
         }
         if (a.calc_dc) {
             const cplx d = xs_to_d(xs_norm(s.d.x, s.d.y, s.d.e) + ((const xs *)a.tx.DCx)[s.w]);
-            a.Z[2 * (f * n + i)] = d.re; a.Z[2 * (f * n + i) + 1] = d.im;
+            g.Z[2 * (f * n + i)] = d.re; g.Z[2 * (f * n + i) + 1] = d.im;
         }
-        a.U[i] = s.w; a.stop_iter[i] = s.n;
+        g.U[i] = s.w; g.stop_iter[i] = s.n;
     }
 };
 
@@ -753,13 +753,13 @@ struct BsF32 {
         return -1;
     }
 
-    __device__ static void finish(const State &s, const KArgs &a, int64_t i, int reason) {
-        const int64_t n = a.ld;
+    __device__ static void finish(const State &s, const KArgs &a, const KArgs &g, int64_t i, int reason) {
+        const int64_t n = g.ld;
         const cplx R = a.t.Zn[s.w];
-        a.Z[i] = s.xs + R.re; a.Z[n + i] = s.ys + R.im;
+        g.Z[i] = s.xs + R.re; g.Z[n + i] = s.ys + R.im;
         if (a.calc_dc)
-            for (int q = 0; q < 4; q++) a.Z[(2 + q) * n + i] = xsr_to_d(s.P[q] + PATH(a, q, s.w));
-        a.U[i] = s.w; a.stop_iter[i] = s.n; a.stop_reason[i] = (int8_t)reason;
+            for (int q = 0; q < 4; q++) g.Z[(2 + q) * n + i] = xsr_to_d(s.P[q] + PATH(a, q, s.w));
+        g.U[i] = s.w; g.stop_iter[i] = s.n; g.stop_reason[i] = (int8_t)reason;
     }
 };
 

@@ -10,11 +10,14 @@ enum Kind { KIND_M2 = 0, KIND_MN = 1, KIND_BS = 2 };
 constexpr int32_t ZK_REGISTER = -(1 << 28);
 
 // Workspace of a tile launch (KArgs::work), 64-bit words: [1..5] step
-// counters, [6] unsure pixels, then the pixel cursors, one per XCD, each in
-// a 128-byte line of its own: word WORK_CURSORS + 16 x for the first pass,
-// WORK_CURSORS + 128 + 16 x for the binary64 pass over the unsure pixels.
-constexpr int WORK_CURSORS = 16;
-constexpr int WORK_WORDS = WORK_CURSORS + 2 * 8 * 16;
+// counters, [6] unsure pixels; the words of drained cursors and the WORK_NC
+// pixel cursors, each in a 128-byte line of its own, of the first pass
+// (WORK_DRAINED, WORK_CURSORS + 16 x) and of the binary64 pass over the unsure
+// pixels (WORK_DRAINED + 16, WORK_CURSORS + 16 (WORK_NC + x)).
+constexpr int WORK_NC = 16;
+constexpr int WORK_DRAINED = 16;
+constexpr int WORK_CURSORS = 48;
+constexpr int WORK_WORDS = WORK_CURSORS + 2 * WORK_NC * 16;
 // LDS the tile loop declares itself (its counters' block sums), kept out of
 // the budget for staged tables
 constexpr int TILE_STATIC_LDS = 1024;

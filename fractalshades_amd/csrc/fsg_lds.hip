@@ -14,7 +14,7 @@ template <class Model> static tile_fn fn_lds512(bool full) {
     return full ? k_tile_lds<Model, true, 512> : k_tile_lds<Model, false, 512>;
 }
 
-int tile_lds_block(const LaunchCfg &c) { return (c.kind == KIND_MN && c.xr && c.degree >= 6) ? 512 : 1024; }
+int tile_lds_block(const LaunchCfg &c) { return 1024; }
 
 // z^2 + c in extended range, the headline case: one instantiation per
 // combination of derivatives (der: bit 0 dz/dc, bit 1 dz/dz)

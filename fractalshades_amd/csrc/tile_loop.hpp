@@ -1,15 +1,15 @@
 // tile_loop.hpp -- the persistent, work-stealing tile kernel, generic over a
-// pixel model (State / init / step / finish).  Each lane owns one pixel at a
-// time; when it stops, the lane writes its outputs and takes the next index
-// from a pixel cursor.  Lanes that need work in the same wave share one
-// atomic: ballot + mbcnt hand out consecutive indices.
+// pixel model (State / init / step / finish).  A wave takes 64 pixels at a
+// time, one per lane, from its own first slots, then from pixel cursors that
+// the launch's waves share.
 #pragma once
 #include "bla_key.hpp"
 #include "fsg_internal.hpp"
 
 namespace fsg {
 
-struct Counters { unsigned long long plain, bla, bla_it, reb, tries; };
+// a lane's counts (a lane's plain steps stay far below 2^32: 2000 s of them)
+struct Counters { unsigned plain, bla, reb, tries; unsigned long long bla_it; };
 
 // Stop reason of a pixel whose binary32 result may differ from the binary64
 // loop's (a decision taken within the pixel's error bound): set by the
@@ -97,22 +97,6 @@ __device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) {
     return v;
 }
 
-// A lane whose pixel stops goes idle; the results are written and new
-// pixels taken only once REFILL_BATCH lanes of the wave are idle (or all of
-// them).  Writing a pixel's results and starting the next one costs about as
-// much as a few iterations plus two dependent memory round trips (the
-// cursor atomic, then the pixel offsets), and under SIMT a wave pays it for
-// every trip on which any lane switches -- about one switch per trip when
-// each lane switches on its own.  Batching the switches trades idle lanes for
-// that cost; measured on the 2048x2048 1e-300 frame: batch 8 -> 2.51 ms,
-// 16 -> 2.19, 24 -> 2.09, 32 -> 2.02, 40 -> 1.96, 48 -> 1.96.  Re-measured
-// once the refill's atomics were spread over the XCDs and the step's tests
-// taken together, against 40 (1e-300 frame / interior-dominated frame at
-// 5e-601 / z^3 + c at 1e-800): 24: +1 / +15 / +5 %, 32: +1 / +7 / +2 %,
-// 48: -2 / -5 / -1 %, 56: -2 / -9 / -2.5 %, 60: -3 / -10 / -2 %; 62 and 64
-// (a refill only once every lane is idle) within 1 % of 60.
-constexpr int REFILL_BATCH = 60;
-
 // Models whose mantissas drift between renormalisations (LAZY) have them
 // renormalised every RENORM_TRIPS trips of the wave (one plain step of a lane
 // each, at most): a uniform branch, so the cost is the renormalisation's
@@ -123,110 +107,198 @@ template <class M> struct is_lazy<M, decltype((void)M::LAZY)> { static constexpr
 
 // added to a cursor, moves it past every slot of a launch
 constexpr unsigned long long CURSOR_DRAIN = 1ull << 44;
+constexpr int NC = WORK_NC;
+static_assert(NC <= 16, "the cursors' bits are rotated within a 32-bit word");
+constexpr unsigned ALL_CURSORS = (1u << NC) - 1u;
+constexpr unsigned HAND_STARTED = 1u << 31, HAND_DONE = HAND_STARTED | (ALL_CURSORS << 8);
 
+// The kernel's arguments (its one KArgs), read anew at each use: the compiler
+// cannot keep what is read through this reference in scalar registers from
+// one use to the next.
+__device__ __forceinline__ const KArgs &cold_args() {
+    uint64_t p = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const KArgs *)(const __attribute__((address_space(4))) KArgs *)p;
+}
+
+// Index of slot base + lane, base a multiple of 64 (uniform over the wave): in
+// the blocks' part of a grid the 64 slots are one 8x8 block, found with one
+// division; elsewhere each lane maps its own slot.
+__device__ __forceinline__ int64_t batch_slot(int64_t base, int64_t n, int64_t w) {
+    const unsigned lane = __lane_id();
+    if (w <= 0) return base + lane;
+    if (n <= 0xffffffffll) {
+        const uint32_t w32 = (uint32_t)w, per_row = w32 >> 3, h8 = ((uint32_t)n / w32) & ~7u;
+        const uint32_t blk = (uint32_t)(base >> 6);
+        if ((uint64_t)blk * 64u < (uint64_t)h8 * (w32 & ~7u)) {
+            const uint32_t by = blk / per_row, bx = blk - by * per_row;
+            return (int64_t)(((by << 3) + (lane >> 3)) * w32 + (bx << 3) + (lane & 7u));
+        }
+    }
+    const int64_t s = base + lane;
+    return s < n ? grid_slot(s, n, w) : s;
+}
+
+// One wave takes 64 pixels at a time, iterates them until the last of them has
+// stopped, writes their results and takes the next 64.  Switching a lane to a
+// new pixel as soon as its own stops would cost the wave the write, two
+// dependent memory round trips and the set-up on every trip on which any lane
+// switches; the 64 pixels of an 8x8 block stop at about the same trip, and
+// waiting for 60 idle lanes instead of all 64 measured within 1 %, on the
+// interior-dominated frame too.  The loop over a pixel's trips then is an
+// ordinary divergent loop, without a test for idle lanes.
 template <class Model>
 __device__ __forceinline__ void tile_loop(const KArgs &a) {
     typename Model::State s;
     Counters k = {0, 0, 0, 0, 0};
-    unsigned long long unsure = 0;
-    int64_t idx = -1;
-    int reason = 0;
-    // Pixel cursors, one per XCD.  A launch's blocks go to the 8 XCDs round
-    // robin, and an atomic on one address from every XCD is serialised across
-    // the dies: with one cursor all 4096 waves of a launch queue on it at the
-    // start (about 0.3 ms) and at every refill after.  The slots form groups
-    // of 2^gsh (at most 16384 -- 256 8x8 blocks -- and at least 64, with 8
-    // groups or more when the launch has 512 slots or more); cursor x hands
-    // out the groups g with g % 8 == x, in order.  A wave draws from its own
-    // XCD's cursor, then, once that one is drained, from the next ones in turn
-    // (work stealing), so that every slot is taken exactly once whatever the
-    // block-to-XCD placement.  cur is uniform over the wave.  Group sizes
-    // measured against one cursor: 64 slots -5 %, 4096 -7 %, 16384 -7 % on
-    // the 2048x2048 frame at 1e-300, -15 % on z^3 + c at 1e-800; the
+    unsigned unsure = 0;
+    // Slots.  Wave g's first 64 slots are [64 g, 64 g + 64), without an atomic;
+    // a launch with no more slots than lanes needs no other.  The slots past
+    // those of all waves are handed out, 64 at a draw, by NC pixel cursors,
+    // each in its own 128-byte line: an atomic takes 12-15 ns on its address
+    // whichever wave it comes from, so one cursor serves a draw per 12 ns and
+    // 16 one per 1 ns.
+    // The slots form groups of 2^gsh (at most 16384 -- 256 8x8 blocks -- and at
+    // least 64); cursor x hands out the groups g with g % NC == x, in order.
+    // A wave draws from its block's cursor (the blocks of one cursor are on
+    // one XCD: they go to the 8 XCDs round robin), then, once that one is
+    // drained, from the next one in turn that is not (work stealing), so that
+    // every slot is taken exactly once whatever the block-to-XCD placement.
+    // The first wave that finds a cursor drained marks it in a global word;
+    // every one takes the marks of that word and passes them to its block in
+    // LDS: no wave tries the cursors in turn (a read of a cursor's line costs
+    // as much as a draw).  Before (eight cursors; every wave drew its first slots too,
+    // and at the end from each cursor in turn): 512x512 pixels of one
+    // iteration 67 us, now 14; 2048x2048 198, now 105.
+    // Group sizes measured against one cursor: 64 slots -5 %, 4096 -7 %, 16384
+    // -7 % on the 2048x2048 frame at 1e-300, -15 % on z^3 + c at 1e-800; the
     // interior-dominated frame lost 9 %, 3.5 % and 0.8 %.
-    unsigned long long *const cursors = a.work + WORK_CURSORS + (a.redo ? 128 : 0);
-    const unsigned xcd = blockIdx.x & 7u;
-    const int gsh = min(14, max(6, 63 - __clzll((unsigned long long)max<int64_t>(a.npts >> 3, 1))));
-    unsigned cur = 0;
-    // The interrupt flag is host memory, a read across PCIe: reads from every
-    // wave at every refill were served one after the other, 94 ns each (544 us
-    // for a 200x200 tile whose pixels take 35 us).  So one wave of every
-    // eighth block reads it, and only at a refill that writes finished pixels
-    // (the caller has just looked at the flag itself); when it is set, that
-    // wave drains every cursor, and no wave takes a new pixel.  The host call
-    // of the 200x200 tile: 973 -> 506 us.
-    const bool poller = a.stop != nullptr && xcd == 0u && __builtin_amdgcn_readfirstlane((int)threadIdx.x) < 64;
+    //
+    // hand: the wave's cursor (low 8 bits), the cursors it knows drained
+    // (ALL_CURSORS << 8) and whether it has taken its first slots (STARTED),
+    // uniform over the wave.  Everything else it needs between two batches it
+    // takes from the kernel's arguments again (cold_args): held in scalar
+    // registers over the loop, that spilled scalar registers the step uses.
+    __shared__ unsigned block_seen;                 // cursors known drained to the block
+    const unsigned wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    unsigned hand = blockIdx.x % NC;
+    if (threadIdx.x == 0) block_seen = 0u;
+    __syncthreads();
     // an escape radius past 2^30 lets one step multiply a mantissa further:
     // renormalised on every trip there
     const unsigned renorm_mask = a.M2 > 0x1p60 ? 0u : RENORM_TRIPS - 1u;
-    unsigned trips = 0;
-    bool active = false;      // iterating a pixel
-    bool pending = false;     // holding a stopped pixel whose results are not written yet
-    bool exhausted = false;   // every cursor is drained for this lane
+    // the binary64 pass: slots of the last batch drawn that are still to take
+    unsigned long long rest = 0;
+    int64_t rest_idx = 0;
     for (;;) {
-        const unsigned long long act = __ballot(active);
-        // idle lanes with something to do at a refill: a stopped pixel to
-        // write, or cursors not all found drained.  Once there are none, the
-        // wave only steps its remaining pixels (a launch's last, longest
-        // ones) without the refill's ballots, and leaves the loop when none
-        // is left: every result is then written.
-        const unsigned long long want = __ballot(!active && (pending || !exhausted));
-        if (act == 0ull && want == 0ull) break;
-        if (want != 0ull && (act == 0ull || 64 - __popcll(act) >= REFILL_BATCH)) {
-            bool drained = false;     // this lane found the current cursor drained
-            if (poller && __ballot(pending) != 0ull) {
-                if (__hip_atomic_load(a.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0u && __lane_id() < 8)
-                    atomicAdd(cursors + 16 * __lane_id(), CURSOR_DRAIN);
-            }
-            if (!active) {
-                if (pending) {
-                    Model::finish(s, a, idx, reason);
-                    unsure += (reason == REASON_UNSURE);
-                    pending = false;
-                }
-                if (!exhausted) {
-                    // idle lanes take consecutive indices from one atomic
-                    const unsigned long long mask = __ballot(1);
-                    const int leader = __ffsll((long long)mask) - 1;
-                    const unsigned rank = __builtin_amdgcn_mbcnt_hi(
-                        (unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
-                    const unsigned cx = (xcd + cur) & 7u;
-                    unsigned long long base = 0;
-                    if ((int)__lane_id() == leader)
-                        base = atomicAdd(cursors + 16 * cx, (unsigned long long)__popcll(mask));
-                    const unsigned lo = __builtin_amdgcn_readlane((unsigned)base, leader);
-                    const unsigned hi = __builtin_amdgcn_readlane((unsigned)(base >> 32), leader);
-                    const int64_t loc = (int64_t)(((unsigned long long)hi << 32) | lo) + rank;
-                    idx = ((((loc >> gsh) << 3) + (int64_t)cx) << gsh) + (loc & ((1ll << gsh) - 1));
-                    if (idx < a.npts) {
-                        if (a.grid_w > 0) idx = grid_slot(idx, a.npts, a.grid_w);
-                        // the binary64 pass takes only the pixels the binary32 one left unsure
-                        if (!a.redo || a.stop_reason[idx] == REASON_UNSURE) {
-                            Model::init(s, a, a.pix[2 * idx], a.pix[2 * idx + 1]);
-                            active = true;
-                        }
-                    } else {
-                        drained = true;
-                        // cur >= 7: the wave has found every cursor drained
-                        // (cur counts the cursors found drained, in turn)
-                        exhausted = (cur >= 7u);
+        const KArgs &g = cold_args();
+        int64_t idx = 0;
+        unsigned filled = 0;              // lanes [0, filled) have a pixel
+        while (filled < 64u) {
+            if (rest == 0ull) {
+                // the next 64 slots, base .. base + 63
+                const unsigned waves = blockDim.x >> 6;
+                const int64_t held = 64 * (int64_t)(gridDim.x * waves);      // the waves' first slots
+                const int64_t left = g.npts - held;                          // the cursors' slots
+                int64_t base = -1;
+                if ((hand & HAND_STARTED) == 0u) {
+                    base = 64 * (int64_t)(blockIdx.x * waves + wave);
+                    hand |= left > 0 ? HAND_STARTED : HAND_DONE;
+                } else {
+                    unsigned long long *const cursors = g.work + WORK_CURSORS + (g.redo ? 16 * NC : 0);
+                    unsigned *const drained = reinterpret_cast<unsigned *>(g.work + WORK_DRAINED + (g.redo ? 16 : 0));
+                    // The interrupt flag is host memory, a read across PCIe:
+                    // reads from every wave at every refill were served one
+                    // after the other, 94 ns each (544 us for a 200x200 tile
+                    // whose pixels take 35 us).  So one wave of every eighth
+                    // block reads it, when it has finished a batch (the caller
+                    // has just looked at the flag itself); when it is set,
+                    // that wave drains every cursor, and no wave takes a new
+                    // pixel.  The host call of the 200x200 tile: 973 -> 506 us.
+                    if (g.stop != nullptr && (blockIdx.x & 7u) == 0u && wave == 0u && __lane_id() < NC &&
+                        __hip_atomic_load(g.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0u) {
+                        atomicAdd(cursors + 16 * __lane_id(), CURSOR_DRAIN);
+                        atomicOr(drained, ALL_CURSORS);
                     }
+                    const int gsh = min(14, max(6, 63 - __clzll((unsigned long long)(left / NC | 1))));
+                    const int64_t low = (1ll << gsh) - 1;
+                    unsigned seen = (hand >> 8) & ALL_CURSORS, cur = hand & 0xffu;
+                    while (seen != ALL_CURSORS) {
+                        seen |= (unsigned)__builtin_amdgcn_readfirstlane((int)__hip_atomic_load(
+                            &block_seen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+                        if (seen == ALL_CURSORS) break;
+                        // the first cursor from the wave's on that is not known drained
+                        const unsigned open = ~seen & ALL_CURSORS;
+                        cur = (cur + (unsigned)__builtin_ctz(open >> cur | open << (NC - cur))) % NC;
+                        unsigned long long v = 0;
+                        if (__lane_id() == 0) v = atomicAdd(cursors + 16 * cur, 64ull);
+                        const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
+                        const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+                        const int64_t loc = (int64_t)(((unsigned long long)hi << 32) | lo);
+                        // the cursor's positions: its whole groups, and the last, short one
+                        const int64_t ng = left >> gsh;
+                        const int64_t end = (((ng + NC - 1 - (int64_t)cur) / NC) << gsh) +
+                                            (ng % NC == (int64_t)cur ? left & low : 0);
+                        if (loc < end) {
+                            base = held + ((((loc >> gsh) * NC + (int64_t)cur) << gsh) | (loc & low));
+                            break;
+                        }
+                        // the first draw past the cursor's end marks it; every
+                        // one takes the marks (a read: an atomic of each wave
+                        // on this one word would queue them)
+                        unsigned known = 0;
+                        if (__lane_id() == 0) {
+                            known = loc - end < 64 ? atomicOr(drained, 1u << cur)
+                                                   : __hip_atomic_load(drained, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        }
+                        seen |= (unsigned)__builtin_amdgcn_readfirstlane((int)known) | (1u << cur);
+                        if (__lane_id() == 0) atomicOr(&block_seen, seen);
+                    }
+                    hand = cur | (seen << 8) | HAND_STARTED;
                 }
+                if (base < 0) break;
+                rest_idx = batch_slot(base, g.npts, g.grid_w);
+                bool take = base + (int64_t)__lane_id() < g.npts;
+                // the binary64 pass takes only the pixels the binary32 one left unsure
+                if (g.redo) take = take && g.stop_reason[take ? rest_idx : 0] == REASON_UNSURE;
+                rest = __builtin_amdgcn_ballot_w64(take);
+                if (!g.redo) {
+                    idx = rest_idx;
+                    filled = (unsigned)__popcll(rest);        // the first lanes
+                    rest = 0ull;
+                    break;
+                }
+            } else {
+                // the batch's unsure slots go to the free lanes, in order
+                // (without it a wave iterated only its 44 to 88 % of lanes
+                // that drew one); the other lanes complete the permutation
+                const auto below = [](unsigned long long m) {
+                    return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+                };
+                const bool goes = ((rest >> __lane_id()) & 1ull) != 0ull && filled + below(rest) < 64u;
+                const unsigned long long sent = __builtin_amdgcn_ballot_w64(goes);
+                const unsigned rank = below(sent), end = filled + (unsigned)__popcll(sent);
+                const int to = (int)(4u * ((goes ? filled + rank : end + __lane_id() - rank) & 63u));
+                const int lo = __builtin_amdgcn_ds_permute(to, (int)(uint32_t)rest_idx);
+                const int hi = __builtin_amdgcn_ds_permute(to, (int)(uint32_t)((uint64_t)rest_idx >> 32));
+                if (__lane_id() >= filled && __lane_id() < end) idx = (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+                rest &= ~sent;
+                filled = end;
             }
-            if (__ballot(drained) != 0ull) cur++;
-            // lanes still idle after the refill (the binary64 pass can draw a
-            // whole batch of slots without an unsure pixel) refill again on
-            // the next trip
         }
-        trips++;
-        if (active) {
-            if constexpr (is_lazy<Model>::value)
-                if ((trips & renorm_mask) == 0u) Model::renorm(s, a);
-            reason = Model::step(s, a, k);
-            if (reason >= 0) {
-                active = false;
-                pending = true;
-            }
+        if (filled == 0u) break;
+        if (__lane_id() < filled) {
+            Model::init(s, g, g.pix[2 * idx], g.pix[2 * idx + 1]);
+            unsigned trips = 0;
+            int reason;
+            do {
+                if constexpr (is_lazy<Model>::value) {
+                    if ((++trips & renorm_mask) == 0u) Model::renorm(s, a);
+                }
+                reason = Model::step(s, a, k);
+            } while (reason < 0);
+            Model::finish(s, a, cold_args(), idx, reason);
+            unsure += (reason == REASON_UNSURE);
         }
     }
     // All lanes have left the loop.  The block's waves add up their counters

@@ -66,25 +66,25 @@ __device__ __forceinline__ void bs_full(double &x, double &y, double A, double B
 // orbit finish (perturbation.py:1390-1396): from the last-but-one record to
 // n - backshift with c + Zn_path[1]
 template <int KIND, int DEG>
-__device__ __forceinline__ void orbit_finish_holo(const OrbitRec<true> &o, const KArgs &a, int32_t n,
+__device__ __forceinline__ void orbit_finish_holo(const OrbitRec<true> &o, const KArgs &a, const KArgs &g, int32_t n,
                                                   cplx c, int64_t i) {
     cplx zo = mk(o.x2, o.y2);
     const cplx CC = c + a.t.Zn[1];
     for (int32_t k = o.i2; k < n - a.backshift; k++) zo = zn_full<KIND, DEG>(zo, CC);
     const int64_t fo = 1 + a.calc_dz + a.calc_dc;
-    a.Z[2 * (fo * a.ld + i)] = zo.re; a.Z[2 * (fo * a.ld + i) + 1] = zo.im;
+    g.Z[2 * (fo * g.ld + i)] = zo.re; g.Z[2 * (fo * g.ld + i) + 1] = zo.im;
 }
 // the same for the burning ship (perturbation.py:1778-1787); the second
 // constant is b + Im Zn_path[1], as the reference has it
 template <int FL>
-__device__ __forceinline__ void orbit_finish_bs(const OrbitRec<true> &o, const KArgs &a, int32_t n,
+__device__ __forceinline__ void orbit_finish_bs(const OrbitRec<true> &o, const KArgs &a, const KArgs &g, int32_t n,
                                                 double ca, double cb, int64_t i) {
     double x = o.x2, y = o.y2;
     const cplx R1 = a.t.Zn[1];
     const double AA = ca + R1.re, BB = cb + R1.im;
     for (int32_t k = o.i2; k < n - a.backshift; k++) bs_full<FL>(x, y, AA, BB);
     const int64_t fo = 2 + (a.calc_dc ? 4 : 0);
-    a.Z[fo * a.ld + i] = x; a.Z[(fo + 1) * a.ld + i] = y;
+    g.Z[fo * g.ld + i] = x; g.Z[(fo + 1) * g.ld + i] = y;
 }
 
 // BLA lookup on binary64 |z| (ref_BLA_get, perturbation.py:2116-2170)
@@ -247,18 +247,18 @@ struct HoloStd {
         return -1;
     }
 
-    __device__ static void finish(const State &s, const KArgs &a, int64_t i, int reason) {
-        const int64_t n = a.ld;
+    __device__ static void finish(const State &s, const KArgs &a, const KArgs &g, int64_t i, int reason) {
+        const int64_t n = g.ld;
         cplx z = s.z + a.t.Zn[s.w];
-        a.Z[2 * i] = z.re; a.Z[2 * i + 1] = z.im;
+        g.Z[2 * i] = z.re; g.Z[2 * i + 1] = z.im;
         int f = 1;
-        if (DZ_ON(a)) { a.Z[2 * (n + i)] = s.h.re; a.Z[2 * (n + i) + 1] = s.h.im; f = 2; }
+        if (DZ_ON(a)) { g.Z[2 * (n + i)] = s.h.re; g.Z[2 * (n + i) + 1] = s.h.im; f = 2; }
         if (DC_ON(a)) {
             cplx d = s.d + a.t.dc[s.w];
-            a.Z[2 * (f * n + i)] = d.re; a.Z[2 * (f * n + i) + 1] = d.im;
+            g.Z[2 * (f * n + i)] = d.re; g.Z[2 * (f * n + i) + 1] = d.im;
         }
-        if constexpr (ORB) orbit_finish_holo<KIND, DEG>(s.orb, a, s.n, s.c, i);
-        a.U[i] = s.w; a.stop_iter[i] = s.n; a.stop_reason[i] = (int8_t)reason;
+        if constexpr (ORB) orbit_finish_holo<KIND, DEG>(s.orb, a, g, s.n, s.c, i);
+        g.U[i] = s.w; g.stop_iter[i] = s.n; g.stop_reason[i] = (int8_t)reason;
     }
 };
 
@@ -543,21 +543,21 @@ struct HoloXr {
         return -1;
     }
 
-    __device__ static void finish(State &s, const KArgs &a, int64_t i, int reason) {
-        const int64_t n = a.ld;
+    __device__ static void finish(State &s, const KArgs &a, const KArgs &g, int64_t i, int reason) {
+        const int64_t n = g.ld;
         renorm(s, a);
         cplx z = to_std(s.z) + a.t.Zn[s.w];
-        a.Z[2 * i] = z.re; a.Z[2 * i + 1] = z.im;
+        g.Z[2 * i] = z.re; g.Z[2 * i + 1] = z.im;
         int f = 1;
         // perturbation.py:1377-1380 writes zn and dzndc back only; the
         // standard dzndz field keeps the 0 written by numba_initialize
-        if (DZ_ON(a)) { a.Z[2 * (n + i)] = 0.; a.Z[2 * (n + i) + 1] = 0.; f = 2; }
+        if (DZ_ON(a)) { g.Z[2 * (n + i)] = 0.; g.Z[2 * (n + i) + 1] = 0.; f = 2; }
         if (DC_ON(a)) {
             cplx d = to_std(add_n(as_z(s.d), DCz(a.t, s.w)));
-            a.Z[2 * (f * n + i)] = d.re; a.Z[2 * (f * n + i) + 1] = d.im;
+            g.Z[2 * (f * n + i)] = d.re; g.Z[2 * (f * n + i) + 1] = d.im;
         }
-        if constexpr (ORB) orbit_finish_holo<KIND, DEG>(s.orb, a, s.n, to_std(s.c), i);
-        a.U[i] = s.w; a.stop_iter[i] = s.n; a.stop_reason[i] = (int8_t)reason;
+        if constexpr (ORB) orbit_finish_holo<KIND, DEG>(s.orb, a, g, s.n, to_std(s.c), i);
+        g.U[i] = s.w; g.stop_iter[i] = s.n; g.stop_reason[i] = (int8_t)reason;
     }
 };
 
@@ -637,14 +637,14 @@ struct BsStd {
         return -1;
     }
 
-    __device__ static void finish(const State &s, const KArgs &a, int64_t i, int reason) {
-        const int64_t n = a.ld;
+    __device__ static void finish(const State &s, const KArgs &a, const KArgs &g, int64_t i, int reason) {
+        const int64_t n = g.ld;
         const cplx R = a.t.Zn[s.w];
-        a.Z[i] = s.x + R.re; a.Z[n + i] = s.y + R.im;
+        g.Z[i] = s.x + R.re; g.Z[n + i] = s.y + R.im;
         if (a.calc_dc)
-            for (int q = 0; q < 4; q++) a.Z[(2 + q) * n + i] = s.P[q] + a.t.bs[q][s.w];
-        if constexpr (ORB) orbit_finish_bs<FL>(s.orb, a, s.n, s.a, s.b, i);
-        a.U[i] = s.w; a.stop_iter[i] = s.n; a.stop_reason[i] = (int8_t)reason;
+            for (int q = 0; q < 4; q++) g.Z[(2 + q) * n + i] = s.P[q] + a.t.bs[q][s.w];
+        if constexpr (ORB) orbit_finish_bs<FL>(s.orb, a, g, s.n, s.a, s.b, i);
+        g.U[i] = s.w; g.stop_iter[i] = s.n; g.stop_reason[i] = (int8_t)reason;
     }
 };
 
@@ -764,14 +764,14 @@ struct BsXr {
         return -1;
     }
 
-    __device__ static void finish(const State &s, const KArgs &a, int64_t i, int reason) {
-        const int64_t n = a.ld;
+    __device__ static void finish(const State &s, const KArgs &a, const KArgs &g, int64_t i, int reason) {
+        const int64_t n = g.ld;
         const cplx R = a.t.Zn[s.w];
-        a.Z[i] = to_std(s.x + R.re); a.Z[n + i] = to_std(s.y + R.im);
+        g.Z[i] = to_std(s.x + R.re); g.Z[n + i] = to_std(s.y + R.im);
         if (a.calc_dc)
-            for (int q = 0; q < 4; q++) a.Z[(2 + q) * n + i] = to_std(s.P[q] + PATH(a.t, q, s.w));
-        if constexpr (ORB) orbit_finish_bs<FL>(s.orb, a, s.n, to_std(s.a), to_std(s.b), i);
-        a.U[i] = s.w; a.stop_iter[i] = s.n; a.stop_reason[i] = (int8_t)reason;
+            for (int q = 0; q < 4; q++) g.Z[(2 + q) * n + i] = to_std(s.P[q] + PATH(a.t, q, s.w));
+        if constexpr (ORB) orbit_finish_bs<FL>(s.orb, a, g, s.n, to_std(s.a), to_std(s.b), i);
+        g.U[i] = s.w; g.stop_iter[i] = s.n; g.stop_reason[i] = (int8_t)reason;
     }
 };
 
