@@ -57,7 +57,10 @@ tile_fn select_tile_lds(const LaunchCfg &c, bool full, int der) {
     }
     if (c.kind == KIND_BS) {
         switch (c.flavor) {
-#define FSG_BS(F) case F: return c.xr ? fn_lds<BsXr<F>>(full) : fn_lds<BsStd<F>>(full);
+#define FSG_BS(F) \
+    case F: \
+        if (c.xr) return der & 1 ? fn_lds<BsXr<F, false, 1>>(full) : fn_lds<BsXr<F, false, 0>>(full); \
+        return fn_lds<BsStd<F>>(full);
             FSG_BS(1) FSG_BS(2) FSG_BS(3) FSG_BS(4) FSG_BS(5)
 #undef FSG_BS
             default: return nullptr;

@@ -648,11 +648,50 @@ struct BsStd {
     }
 };
 
-// Burning-ship family, Xrange deltas (xl.hpp reals)
-template <int FL, bool ORB = false>
+// Burning-ship family, Xrange deltas, on drifting mantissas as HoloXr: x and y
+// share one exponent (e), the four Jacobian deltas another (eP), a and b a
+// third; a shared exponent changes no rounding, since the mantissas stay far
+// inside the binary64 range.  An orbit point's Jacobian values are brought to
+// the scale of the deltas' mantissas divided by z's, R' = R 2^(eR + e - eP),
+// so that a product of z's mantissa with one is a delta's mantissa; X, Y and
+// their sums with x and y are binary64 values.  The folds' derivative terms
+// of the orbit (a pixel on the other side of a fold than the orbit) are formed
+// in a branch.  An orbit point whose larger coordinate is below 2^LOW_Z (zero,
+// the Xrange register) takes the general step on separate exponents.
+// Bound by vector instruction issue; with every real on its own exponent, each
+// sum aligned, tested for zero and each result renormalised, a trip took 515
+// instructions (1920x1080 at 1e-800: 1831 us, now 840).
+template <int FL, bool ORB = false, int DER = -1>
 struct BsXr {
-    struct State { xlf x, y, P[4], a, b; double xs, ys; int32_t w, n; bool dyn; OrbitRec<ORB> orb; };
+    __device__ static bool DC_ON(const KArgs &a) { if constexpr (DER >= 0) return DER != 0; else return a.calc_dc != 0; }
+    struct State { double x, y, P[4], a, b, xs, ys; int32_t e, eP, ec, w, n; bool dyn; OrbitRec<ORB> orb; };
+    static constexpr bool LAZY = true;
+    static constexpr int32_t LOW_Z = -20, FAR = 256;
 
+    // two (four) values on one exponent, the larger normalised
+    __device__ static void norm2(double &x, double &y, int32_t &e) {
+        const xl v = xl_n(x, y, e);
+        x = v.re; y = v.im; e = v.e;
+    }
+    __device__ static void norm4(double *P, int32_t &e) {
+        const double mx = fmax(fmax(fabs(P[0]), fabs(P[1])), fmax(fabs(P[2]), fabs(P[3])));
+        const int32_t k = dexp(mx) - 1;
+        for (int q = 0; q < 4; q++) P[q] = ldexp(P[q], -k);
+        e = (mx == 0.) ? XL_ZERO_E : e + k;
+    }
+    __device__ static void renorm(State &s, const KArgs &a) {
+        norm2(s.x, s.y, s.e);
+        if (DC_ON(a)) norm4(s.P, s.eP);
+    }
+    // separate exponents, and back
+    __device__ static void join2(xlf u, xlf v, double &x, double &y, int32_t &e) {
+        e = max(u.e, v.e);
+        x = ldexp(u.m, shift_of(u.e, e)); y = ldexp(v.m, shift_of(v.e, e));
+    }
+    __device__ static void join4(const xlf *u, double *P, int32_t &e) {
+        e = max(max(u[0].e, u[1].e), max(u[2].e, u[3].e));
+        for (int q = 0; q < 4; q++) P[q] = ldexp(u[q].m, shift_of(u[q].e, e));
+    }
     __device__ static xlf PATH(const Tables &t, int q, int32_t i) { return xlf_of(t.bs[q][i], t.bs_e[q][i]); }
     // orbit point i, normalised per coordinate: the register's Xrange
     // values where the binary64 orbit underflows, the binary64 values
@@ -669,13 +708,108 @@ struct BsXr {
     }
 
     __device__ static void init(State &s, const KArgs &a, double px, double py) {
-        s.a = xlf_of(a.dx_m * (a.lin[0] * px + a.lin[1] * py), a.dx_e) + xlf_of(a.drift_m[0], a.drift_e[0]);
-        s.b = xlf_of(a.dx_m * (a.lin[2] * px + a.lin[3] * py), a.dx_e) + xlf_of(a.drift_m[1], a.drift_e[1]);
-        const xlf z0 = xlf_zero();
-        s.x = z0; s.y = z0; s.P[0] = s.P[1] = s.P[2] = s.P[3] = z0;
+        join2(xlf_of(a.dx_m * (a.lin[0] * px + a.lin[1] * py), a.dx_e) + xlf_of(a.drift_m[0], a.drift_e[0]),
+              xlf_of(a.dx_m * (a.lin[2] * px + a.lin[3] * py), a.dx_e) + xlf_of(a.drift_m[1], a.drift_e[1]), s.a, s.b, s.ec);
+        s.x = s.y = 0.; s.P[0] = s.P[1] = s.P[2] = s.P[3] = 0.;
+        s.e = s.eP = XL_ZERO_E;
         s.xs = 0.; s.ys = 0.;
         s.w = 0; s.n = 0; s.dyn = true;
         s.orb.reset(a.backshift);
+    }
+
+    // The fold |F + f| - |F| of burning_ship.py:19-60 (diffabs, ddX, ddx), F in
+    // the scale of f's mantissa: sg is F's sign, cross whether F + f lies on
+    // the other side of zero.
+    struct Fold {
+        double F, f;              // sg F, sg f
+        uint32_t sg;
+        bool cross;
+        __device__ Fold(double Fv, double fv) {
+            sg = Fv < 0. ? 0x80000000u : 0u;
+            F = flip(Fv, sg); f = flip(fv, sg);
+            cross = !(F + f >= 0.);
+        }
+        // sign bit of the value F + f (a z that underflows binary64 included)
+        __device__ uint32_t sum_sign() const { return flip(F + f, sg) < 0. ? 0x80000000u : 0u; }
+        __device__ double diff() const { return cross ? -__builtin_fma(2., F, f) : f; }
+    };
+    __device__ static double flip(double v, uint32_t sg) { return from_bits(bits(v) ^ ((uint64_t)sg << 32)); }
+
+    // one step on shared exponents (bs_hess and bs_zn of models.hpp, the same
+    // operations in the same order); a, b: c's parts in z's scale; R: the
+    // orbit's Jacobian as above
+    __device__ static void fast_step(State &s, const KArgs &ka, double X, double Y, double a, double b, const double *R) {
+        const int32_t e = s.e;
+        const double x = s.x, y = s.y, xs = s.xs, ys = s.ys;
+        const double Ux = __builtin_fma(2., X, xs), Uy = __builtin_fma(2., Y, ys);     // x + 2 X, y + 2 Y
+        const double Xs = X + xs, Ys = Y + ys;
+        const double q0 = x * Ux - y * Uy;                                  // Re (z (z + 2 Z))
+        constexpr bool FX = FL == 4 || FL == 5, FXY = FL == 1 || FL == 5, FY = FL == 2 || FL == 3;
+        const double t0 = FXY ? x * ys + x * Y + y * X : X * y + Y * x + x * ys;
+        // the fold of the x part (X^2 - Y^2), of the y part (X Y), of Y
+        const double Fx = FX ? X * X - Y * Y : 0., Fy = FXY ? X * Y : FY ? Y : 0.;
+        const Fold gx(FX ? ldexp(Fx, -e) : 0., q0), gy(FXY || FY ? ldexp(Fy, -e) : 0., FY ? y : t0);
+        const double da = gy.diff(), ab = fabs(Ys);
+        const uint32_t sy = FY ? gy.sum_sign() : 0u;
+        if (DC_ON(ka)) {
+            double P[4];
+#pragma unroll
+            for (int c = 0; c < 2; c++) {                                   // d/da, d/db
+                const double xp = s.P[c], yp = s.P[2 + c], Xp = R[c], Yp = R[2 + c];
+                const double xe = ldexp(xp, e), ye = ldexp(yp, e);          // the deltas in R's scale
+                if constexpr (FX) {
+                    const double o = xp * Ux + x * (xe + 2. * Xp) - yp * Uy - y * (ye + 2. * Yp);
+                    P[c] = flip(o, gx.sg);
+                    if (gx.cross) P[c] = -flip(2. * ldexp(2. * (X * Xp - Y * Yp), -e) + o, gx.sg);
+                } else if constexpr (FL == 3) {
+                    const double h = gy.cross ? -flip(2. * ldexp(Yp, -e) + yp, gy.sg) : flip(yp, gy.sg);
+                    P[c] = xp * Ux + x * (xe + 2. * Xp) - Yp * da - Y * h - yp * ab - flip(y, sy) * (Yp + ye);
+                } else {
+                    P[c] = 2. * ((Xs * xp + Xp * x) - (Ys * yp + Yp * y));
+                }
+                if constexpr (FXY) {
+                    const double o = xp * ys + xs * yp + xp * Y + x * Yp + yp * X + y * Xp;
+                    P[2 + c] = 2. * flip(o, gy.sg);
+                    if (gy.cross) P[2 + c] = -2. * flip(2. * ldexp(Xp * Y + X * Yp, -e) + o, gy.sg);
+                } else if constexpr (FL == 2) {
+                    const double h = gy.cross ? -flip(2. * ldexp(Yp, -e) + yp, gy.sg) : flip(yp, gy.sg);
+                    P[2 + c] = 2. * (Xp * da + X * h + xp * ab + flip(x, sy) * (Yp + ye));
+                } else {
+                    P[2 + c] = 2. * (Xp * y + X * yp + Yp * x + Y * xp + xp * ys + xs * yp);
+                }
+            }
+            for (int q = 0; q < 4; q++) s.P[q] = P[q];
+        }
+        if constexpr (FX) s.x = gx.diff() + a;
+        else if constexpr (FL == 3) s.x = x * Ux - Y * da - y * ab + a;
+        else s.x = q0 + a;
+        if constexpr (FXY) s.y = __builtin_fma(2., da, -b);
+        else if constexpr (FL == 2) s.y = __builtin_fma(2., X * da + x * ab, -b);
+        else s.y = __builtin_fma(2., t0, -b);
+    }
+
+    // the same on separate exponents
+    __device__ static void general_step(State &s, const KArgs &a, int32_t kx, int32_t ky, cplx R0) {
+        const Tables &t = a.t;
+        xlf X, Y;
+        ZRv(t, kx, ky, R0, X, Y);
+        const xzf x = as_zf(xlf_of(s.x, s.e)), y = as_zf(xlf_of(s.y, s.e)), Xz = as_zf(X), Yz = as_zf(Y);
+        if (DC_ON(a)) {
+            const xzf z0 = as_zf(xlf_zero());
+            xzf Rd[4] = {z0, z0, z0, z0};
+            // the host's Xrange path records keep |mantissa| within 2^+-100 (a
+            // zero entry with the zero exponent code): used as loaded
+            if (!s.dyn) for (int q = 0; q < 4; q++) { Rd[q].m = t.bs[q][s.w]; Rd[q].e = t.bs_e[q][s.w]; }
+            xzf P[4];
+            for (int q = 0; q < 4; q++) P[q] = as_zf(xlf_of(s.P[q], s.eP));
+            bs_hess<FL>(x, y, P, Xz, Yz, Rd);
+            xlf Pn[4];
+            for (int q = 0; q < 4; q++) Pn[q] = xlf_of(P[q]);
+            join4(Pn, s.P, s.eP);
+        }
+        xzf nx = x, ny = y;
+        bs_zn<FL>(nx, ny, Xz, Yz, as_zf(xlf_of(s.a, s.ec)), as_zf(xlf_of(s.b, s.ec)));
+        join2(xlf_of(nx), xlf_of(ny), s.x, s.y, s.e);
     }
 
     __device__ static int step(State &s, const KArgs &a, Counters &k) {
@@ -686,20 +820,30 @@ struct BsXr {
             k.tries++;
             if (st == 0) break;
             {
-                const double *M = t.M + 8 * idx;
+                // A z + B c and A J on shared exponents; the coefficients are
+                // split into mantissas on one exponent each (they reach the
+                // ends of the binary64 range)
+                double M[8];
+                for (int q = 0; q < 8; q++) M[q] = t.M[8 * idx + q];
                 s.n += st; s.w += st;
-                const xzf x = as_zf(s.x), y = as_zf(s.y);
-                const xzf ca = as_zf(s.a), cb = as_zf(s.b);
-                const xzf nx = mul_w(M[0], x) + mul_w(M[1], y) + mul_w(M[4], ca) + mul_w(M[5], cb);
-                const xzf ny = mul_w(M[2], x) + mul_w(M[3], y) + mul_w(M[6], ca) + mul_w(M[7], cb);
-                s.x = xlf_of(nx); s.y = xlf_of(ny);
-                s.xs = to_std(s.x); s.ys = to_std(s.y);
-                if (a.calc_dc) {
-                    const xzf P0 = as_zf(s.P[0]), P1 = as_zf(s.P[1]), P2 = as_zf(s.P[2]), P3 = as_zf(s.P[3]);
-                    s.P[0] = xlf_of(mul_w(M[0], P0) + mul_w(M[1], P2));
-                    s.P[1] = xlf_of(mul_w(M[0], P1) + mul_w(M[1], P3));
-                    s.P[2] = xlf_of(mul_w(M[2], P0) + mul_w(M[3], P2));
-                    s.P[3] = xlf_of(mul_w(M[2], P1) + mul_w(M[3], P3));
+                renorm(s, a);
+                int32_t eA = 0, eB = 0;
+                norm4(M, eA);
+                norm4(M + 4, eB);
+                double x = s.x, y = s.y;
+                int32_t e = s.e + eA, sc = s.ec + eB - e;
+                if (sc > FAR) { x = ldexp(x, -sc); y = ldexp(y, -sc); e += sc; sc = 0; }
+                s.x = M[0] * x + M[1] * y + ldexp(M[4] * s.a, sc) + ldexp(M[5] * s.b, sc);
+                s.y = M[2] * x + M[3] * y + ldexp(M[6] * s.a, sc) + ldexp(M[7] * s.b, sc);
+                s.e = e;
+                s.xs = ldexp(s.x, e); s.ys = ldexp(s.y, e);
+                if (DC_ON(a)) {
+                    const double P0 = s.P[0], P1 = s.P[1], P2 = s.P[2], P3 = s.P[3];
+                    s.P[0] = M[0] * P0 + M[1] * P2;
+                    s.P[1] = M[0] * P1 + M[1] * P3;
+                    s.P[2] = M[2] * P0 + M[3] * P2;
+                    s.P[3] = M[2] * P1 + M[3] * P3;
+                    s.eP += eA;
                 }
                 k.bla++; k.bla_it += st;
             }
@@ -708,27 +852,31 @@ struct BsXr {
         // the step's table reads first, its tests together (as in HoloStd)
         const int32_t w1 = (s.w + 1 >= t.order) ? 0 : s.w + 1;
         const int32_t kx0 = t.zn_k[2 * s.w], ky0 = t.zn_k[2 * s.w + 1];
-        const int32_t kx1 = t.zn_k[2 * w1], ky1 = t.zn_k[2 * w1 + 1];
         const cplx R0 = t.Zn[s.w], R1 = t.Zn[w1];
-        xlf X, Y;
-        ZRv(t, kx0, ky0, R0, X, Y);
-        // one iteration on lazily normalised values, renormalised once
-        const xzf x = as_zf(s.x), y = as_zf(s.y), Xz = as_zf(X), Yz = as_zf(Y);
-        if (a.calc_dc) {
-            const xzf z0 = as_zf(xlf_zero());
-            xzf Rd[4] = {z0, z0, z0, z0};
-            // the host's Xrange path records keep |mantissa| within 2^+-100 (a
-            // zero entry with the zero exponent code): used as loaded, as
-            // HoloXr's DCz
-            if (!s.dyn) for (int q = 0; q < 4; q++) { Rd[q].m = t.bs[q][s.w]; Rd[q].e = t.bs_e[q][s.w]; }
-            xzf P[4] = {as_zf(s.P[0]), as_zf(s.P[1]), as_zf(s.P[2]), as_zf(s.P[3])};
-            bs_hess<FL>(x, y, P, Xz, Yz, Rd);
-            for (int q = 0; q < 4; q++) s.P[q] = xlf_of(P[q]);
+        double R[4] = {0., 0., 0., 0.};
+        int32_t Re[4] = {XL_ZERO_E, XL_ZERO_E, XL_ZERO_E, XL_ZERO_E};
+        if (DC_ON(a)) for (int q = 0; q < 4; q++) { R[q] = t.bs[q][s.w]; Re[q] = t.bs_e[q][s.w]; }
+        if (max(kx0, ky0) < LOW_Z) {
+            general_step(s, a, kx0, ky0, R0);
+        } else {
+            if (s.dyn) for (int q = 0; q < 4; q++) { R[q] = 0.; Re[q] = XL_ZERO_E; }
+            int32_t sc = s.ec - s.e, sR[4];
+            for (int q = 0; q < 4; q++) sR[q] = Re[q] + s.e - s.eP;
+            const int32_t mR = DC_ON(a) ? max(max(sR[0], sR[1]), max(sR[2], sR[3])) : 0;
+            if (max(sc, mR) > FAR) {
+                int32_t up = 0;
+                if (sc > FAR) { s.x = ldexp(s.x, -sc); s.y = ldexp(s.y, -sc); s.e += sc; up = sc; sc = 0; }
+                if (DC_ON(a)) {
+                    const int32_t m = mR + up;
+                    const int32_t dn = m > FAR ? m : 0;
+                    for (int q = 0; q < 4; q++) { s.P[q] = ldexp(s.P[q], -dn); sR[q] += up - dn; }
+                    s.eP += dn;
+                }
+            }
+            for (int q = 0; q < 4; q++) R[q] = ldexp(R[q], sR[q]);
+            fast_step(s, a, R0.re, R0.im, ldexp(s.a, sc), ldexp(s.b, sc), R);
         }
-        xzf nx = x, ny = y;
-        bs_zn<FL>(nx, ny, Xz, Yz, as_zf(s.a), as_zf(s.b));
-        s.x = xlf_of(nx); s.y = xlf_of(ny);
-        s.xs = to_std(s.x); s.ys = to_std(s.y);
+        s.xs = ldexp(s.x, s.e); s.ys = ldexp(s.y, s.e);
         const double XX = s.xs + R1.re, YY = s.ys + R1.im;
         const bool t_esc = XX * XX + YY * YY > a.M2;
         const bool reb_div = w1 >= t.div_iter - 1;
@@ -740,26 +888,30 @@ struct BsXr {
         s.w = w1;
         s.orb.record(s.n, a.backshift, XX, YY);
         if (t_esc) return 1;
+        bool reb = reb_div;
+        xlf x = xlf_of(s.x, s.e), y = xlf_of(s.y, s.e);
         if (reb_div) {
-            s.xs = XX; s.ys = YY;
-            s.x = xlf_of(XX, 0); s.y = xlf_of(YY, 0);
-            if (a.calc_dc) for (int q = 0; q < 4; q++) s.P[q] = s.P[q] + PATH(t, q, s.w);
+            x = xlf_of(XX, 0); y = xlf_of(YY, 0);
+        } else {
+            s.dyn = dyn;
+            if (s.dyn) {
+                xlf X1, Y1;
+                ZRv(t, t.zn_k[2 * w1], t.zn_k[2 * w1 + 1], R1, X1, Y1);
+                const xlf XXx = x + X1, YYx = y + Y1;
+                reb = le(XXx * XXx + YYx * YYx, x * x + y * y);
+                if (reb) { x = XXx; y = YYx; }
+            }
+        }
+        if (reb) {
+            s.xs = to_std(x); s.ys = to_std(y);
+            join2(x, y, s.x, s.y, s.e);
+            if (DC_ON(a)) {
+                xlf Pn[4];
+                for (int q = 0; q < 4; q++) Pn[q] = xlf_of(s.P[q], s.eP) + PATH(t, q, s.w);
+                join4(Pn, s.P, s.eP);
+            }
             s.w = 0;
             k.reb++;
-            return -1;
-        }
-        s.dyn = dyn;
-        if (s.dyn) {
-            xlf X1, Y1;
-            ZRv(t, kx1, ky1, R1, X1, Y1);
-            const xlf XXx = s.x + X1, YYx = s.y + Y1;
-            if (le(XXx * XXx + YYx * YYx, s.x * s.x + s.y * s.y)) {
-                s.x = XXx; s.y = YYx;
-                s.xs = to_std(XXx); s.ys = to_std(YYx);
-                if (a.calc_dc) for (int q = 0; q < 4; q++) s.P[q] = s.P[q] + PATH(t, q, s.w);
-                s.w = 0;
-                k.reb++;
-            }
         }
         return -1;
     }
@@ -767,10 +919,10 @@ struct BsXr {
     __device__ static void finish(const State &s, const KArgs &a, const KArgs &g, int64_t i, int reason) {
         const int64_t n = g.ld;
         const cplx R = a.t.Zn[s.w];
-        g.Z[i] = to_std(s.x + R.re); g.Z[n + i] = to_std(s.y + R.im);
-        if (a.calc_dc)
-            for (int q = 0; q < 4; q++) g.Z[(2 + q) * n + i] = to_std(s.P[q] + PATH(a.t, q, s.w));
-        if constexpr (ORB) orbit_finish_bs<FL>(s.orb, a, g, s.n, to_std(s.a), to_std(s.b), i);
+        g.Z[i] = to_std(xlf_of(s.x, s.e) + R.re); g.Z[n + i] = to_std(xlf_of(s.y, s.e) + R.im);
+        if (DC_ON(a))
+            for (int q = 0; q < 4; q++) g.Z[(2 + q) * n + i] = to_std(xlf_of(s.P[q], s.eP) + PATH(a.t, q, s.w));
+        if constexpr (ORB) orbit_finish_bs<FL>(s.orb, a, g, s.n, to_std(xlf_of(s.a, s.ec)), to_std(xlf_of(s.b, s.ec)), i);
         g.U[i] = s.w; g.stop_iter[i] = s.n; g.stop_reason[i] = (int8_t)reason;
     }
 };
