@@ -8,48 +8,35 @@ namespace fsg {
 template <class Model> static tile_fn fn_lds(bool full) {
     return full ? k_tile_lds<Model, true> : k_tile_lds<Model, false>;
 }
-// z^d + c of degree 6..8 with extended-range deltas needs more than the 128
-// VGPRs a 1024-lane block allows (it spilled): 512-lane blocks
-template <class Model> static tile_fn fn_lds512(bool full) {
-    return full ? k_tile_lds<Model, true, 512> : k_tile_lds<Model, false, 512>;
-}
-
-int tile_lds_block(const LaunchCfg &c) { return 1024; }
-
-// z^2 + c in extended range, the headline case: one instantiation per
-// combination of derivatives (der: bit 0 dz/dc, bit 1 dz/dz)
-static tile_fn fn_lds_m2xr(bool full, int der) {
+// One instantiation per combination of derivatives (der: bit 0 dz/dc, bit 1
+// dz/dz), so that the step is straight-line code: z^2 + c for all four; z^d + c
+// for the two that frames use (dz/dc, both), the others reading them from the
+// launch arguments (z^3 + c at 1e-800 with dz/dc, with the BLA jump's change:
+// 694 -> 587 us; z^6 + c 654 -> 551 us).
+template <template <int> class Model> static tile_fn fn_lds_der(bool full, int der) {
     switch (der) {
-        case 0: return fn_lds<HoloXr<KIND_M2, 2, false, 0>>(full);
-        case 1: return fn_lds<HoloXr<KIND_M2, 2, false, 1>>(full);
-        case 2: return fn_lds<HoloXr<KIND_M2, 2, false, 2>>(full);
-        default: return fn_lds<HoloXr<KIND_M2, 2, false, 3>>(full);
+        case 0: return fn_lds<Model<0>>(full);
+        case 1: return fn_lds<Model<1>>(full);
+        case 2: return fn_lds<Model<2>>(full);
+        default: return fn_lds<Model<3>>(full);
     }
 }
-
-// the same with binary64 deltas
-static tile_fn fn_lds_m2std(bool full, int der) {
-    switch (der) {
-        case 0: return fn_lds<HoloStd<KIND_M2, 2, false, 0>>(full);
-        case 1: return fn_lds<HoloStd<KIND_M2, 2, false, 1>>(full);
-        case 2: return fn_lds<HoloStd<KIND_M2, 2, false, 2>>(full);
-        default: return fn_lds<HoloStd<KIND_M2, 2, false, 3>>(full);
-    }
+template <template <int> class Model> static tile_fn fn_lds_der2(bool full, int der) {
+    return der == 1 ? fn_lds<Model<1>>(full) : der == 3 ? fn_lds<Model<3>>(full) : fn_lds<Model<-1>>(full);
 }
+template <int DER> using M2Xr = HoloXr<KIND_M2, 2, false, DER>;
+template <int DER> using M2Std = HoloStd<KIND_M2, 2, false, DER>;
+template <int D> struct MnModels {
+    template <int DER> using Xr = HoloXr<KIND_MN, D, false, DER>;
+    template <int DER> using Std = HoloStd<KIND_MN, D, false, DER>;
+};
 
 tile_fn select_tile_lds(const LaunchCfg &c, bool full, int der) {
-    if (tile_lds_block(c) == 512) {
-        switch (c.degree) {
-            case 6: return fn_lds512<HoloXr<KIND_MN, 6>>(full);
-            case 7: return fn_lds512<HoloXr<KIND_MN, 7>>(full);
-            case 8: return fn_lds512<HoloXr<KIND_MN, 8>>(full);
-            default: return nullptr;
-        }
-    }
-    if (c.kind == KIND_M2) return c.xr ? fn_lds_m2xr(full, der) : fn_lds_m2std(full, der);
+    if (c.kind == KIND_M2) return c.xr ? fn_lds_der<M2Xr>(full, der) : fn_lds_der<M2Std>(full, der);
     if (c.kind == KIND_MN) {
         switch (c.degree) {
-#define FSG_MN(D) case D: return c.xr ? fn_lds<HoloXr<KIND_MN, D>>(full) : fn_lds<HoloStd<KIND_MN, D>>(full);
+#define FSG_MN(D) \
+    case D: return c.xr ? fn_lds_der2<MnModels<D>::Xr>(full, der) : fn_lds_der2<MnModels<D>::Std>(full, der);
             FSG_MN(2) FSG_MN(3) FSG_MN(4) FSG_MN(5) FSG_MN(6) FSG_MN(7) FSG_MN(8)
 #undef FSG_MN
             default: return nullptr;

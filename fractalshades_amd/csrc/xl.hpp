@@ -34,9 +34,17 @@ constexpr int32_t XL_ZERO_E = -(1 << 26);
 
 FSG_DEV int32_t dexp(double v) { return __builtin_amdgcn_frexp_exp(v); }
 
+// max(|x|, |y|) in one instruction: fmax first quiets each operand that may be
+// a signalling NaN with an instruction of its own
+FSG_DEV double amax(double x, double y) {
+    double r;
+    asm("v_max_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(x), "v"(y));
+    return r;
+}
+
 // normalised: larger component in [1, 2), or (0, 0, XL_ZERO_E)
 FSG_DEV xl xl_n(double re, double im, int32_t e) {
-    const double mx = fmax(fabs(re), fabs(im));
+    const double mx = amax(re, im);
     const int32_t k = dexp(mx) - 1;
     xl r;
     r.re = ldexp(re, -k);
@@ -158,7 +166,7 @@ struct xz { double re, im; int32_t e; };
 FSG_DEV xz xz_mk(double re, double im, int32_t e) {
     xz r;
     r.re = re; r.im = im;
-    r.e = (fmax(fabs(re), fabs(im)) == 0.) ? XL_ZERO_E : e;
+    r.e = (amax(re, im) == 0.) ? XL_ZERO_E : e;
     return r;
 }
 FSG_DEV xz as_z(xl a) { xz r; r.re = a.re; r.im = a.im; r.e = a.e; return r; }
