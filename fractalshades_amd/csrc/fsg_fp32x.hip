@@ -925,7 +925,8 @@ hipError_t launch_tile_f32(const LaunchCfg &cfg, const KArgs &a, hipStream_t str
                      : bs ? select_bsx_lds(cfg) : select_f32_lds(cfg, al.ldsx.full != 0);
         const int fill = fl ? fill_blocks(reinterpret_cast<const void *>(fl), 1024, al.ldsx.bytes) : -1;
         if (fill > 0) {
-            hipLaunchKernelGGL(fl, dim3(launch_blocks(fill, al, 1024)), dim3(1024),
+            const int block = tile_block(fill, al);
+            hipLaunchKernelGGL(fl, dim3(launch_blocks(fill, al, block)), dim3(block),
                                (size_t)al.ldsx.bytes, stream, al);
             return hipGetLastError();
         }

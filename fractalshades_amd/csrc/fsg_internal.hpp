@@ -119,7 +119,7 @@ struct LaunchCfg { int kind, degree, flavor, xr, precision, orbit; };
 
 hipError_t launch_tile(const LaunchCfg &cfg, const KArgs &a, hipStream_t stream);
 // the calc_orbit instantiations (fsg_orbit.hip) and the LDS-staged ones
-// (fsg_lds.hip, 1024-lane blocks)
+// (fsg_lds.hip, blocks of up to 1024 lanes)
 typedef void (*tile_fn)(const KArgs);
 tile_fn select_tile_orbit(const LaunchCfg &cfg);
 // der: the derivatives the launch computes (bit 0 dz/dc, bit 1 dz/dz)
@@ -137,6 +137,7 @@ int grid_fill_blocks(const void *kernel);          // blocks filling the GPU at 
 int fill_blocks(const void *kernel, int block, int lds_bytes);   // the same for any block / LDS size
 // plan the LDS staging of a launch's tables (bytes = 0 when they do not fit)
 LdsPlan plan_lds(const Tables &t, int bla_dim, int max_bytes);
+int tile_block(int fill, const KArgs &a);          // lanes of an LDS-staged launch's blocks
 int launch_blocks(int fill, const KArgs &a, int block = 256);   // capped by max_blocks and the pixel count
 int max_lds_bytes();                // LDS bytes a block may use (FSG_LDS_BYTES caps it)
 

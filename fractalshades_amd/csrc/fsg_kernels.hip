@@ -219,10 +219,32 @@ int tile_kernel_blocks(const LaunchCfg &cfg) {
     return grid_fill_blocks(reinterpret_cast<const void *>(f));
 }
 
+// blocks that a launch may have, of the fill that the GPU holds
+static int block_cap(int fill, const KArgs &a) {
+    if (a.max_blocks > 0 && a.max_blocks < fill) return a.max_blocks;
+    if (a.max_blocks < 0) return (fill + (-a.max_blocks) - 1) / (-a.max_blocks);   // a share of the GPU
+    return fill;
+}
+
+// Lanes of an LDS-staged launch's blocks, of which a compute unit holds one
+// (160 KB of tables, 1024 lanes of 128 registers): the fewest that give each
+// pixel a lane, in steps of one wave per SIMD.  A launch of fewer pixels than
+// the chip has lanes then runs on every compute unit it may use, with one to
+// three waves per SIMD instead of four on some and none on the others; each
+// wave's trips are shorter where fewer share its issue.  Measured, 1024 ->
+// 256 lanes at 64x64, 200x200 and 256x256 pixels: z^2 + c at 1e-300 74 -> 57,
+// 78 -> 60, 86 -> 60 us, z^3 + c at 1e-800 204 -> 133, 190 -> 136, 196 -> 142;
+// 512 lanes at 362x362: 84 -> 65, 203 -> 154; burning ship at 1e-800 157 ->
+// 116.  128 lanes lose to 256 (the tables' copy).  With more pixels than
+// lanes the smaller blocks only halve the chip (m3, 512x512: 224 us, 256
+// lanes 279).
+int tile_block(int fill, const KArgs &a) {
+    const int64_t lanes = 256 * (int64_t)block_cap(fill, a);
+    return 256 * (int)std::min<int64_t>(4, std::max<int64_t>(1, (a.npts + lanes - 1) / lanes));
+}
+
 int launch_blocks(int fill, const KArgs &a, int block) {
-    int blocks = fill;
-    if (a.max_blocks > 0 && a.max_blocks < blocks) blocks = a.max_blocks;
-    if (a.max_blocks < 0) blocks = (fill + (-a.max_blocks) - 1) / (-a.max_blocks);   // a share of the GPU
+    int blocks = block_cap(fill, a);
     const int64_t need = (a.npts + block - 1) / block;
     if (need < blocks) blocks = (int)(need > 0 ? need : 1);
     return blocks;
@@ -320,9 +342,9 @@ hipError_t launch_tile(const LaunchCfg &cfg, const KArgs &a, hipStream_t stream)
         al.lds = plan_lds(a.t, cfg.kind == KIND_BS ? 8 : 4, max_lds_bytes());
         const int der = (a.calc_dc ? 1 : 0) | (a.calc_dz ? 2 : 0);
         tile_fn f = al.lds.bytes > 0 ? select_tile_lds(cfg, lds_plan_full(a.t, al.lds), der) : nullptr;
-        const int block = 1024;
-        const int fill = f ? fill_blocks(reinterpret_cast<const void *>(f), block, al.lds.bytes) : -1;
+        const int fill = f ? fill_blocks(reinterpret_cast<const void *>(f), 1024, al.lds.bytes) : -1;
         if (fill > 0) {
+            const int block = tile_block(fill, al);
             hipLaunchKernelGGL(f, dim3(launch_blocks(fill, al, block)), dim3(block), (size_t)al.lds.bytes,
                                stream, al);
             return hipGetLastError();

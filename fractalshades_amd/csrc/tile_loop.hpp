@@ -333,8 +333,8 @@ __global__ void __launch_bounds__(256) k_tile(const KArgs a) {
 // The same loop with the reference tables staged in LDS: the loop is bound
 // by the latency of its table reads (orbit point, derivative paths, BLA
 // radius and coefficients at the lane's own iteration index), and an LDS
-// read answers in a fraction of an L2 hit's time.  One 1024-lane block per
-// CU (or more when they fit) copies the tables once, then runs the loop.
+// read answers in a fraction of an L2 hit's time.  One block of up to 1024
+// lanes (tile_block) per CU, or more when they fit, copies the tables once, then runs the loop.
 // FULL: the plan stages every table the launch has, so each table pointer
 // is either null or an LDS address, and the compiler reads the tables with
 // LDS instructions instead of generic (flat) ones
