@@ -381,6 +381,8 @@ int fill_args(fsg_ctx *c, KArgs &a) {
     a.calc_dz = (c->d.kind != FSG_KIND_BS && c->d.interior_detect) ? 1 : 0;
     a.M2 = c->d.M_divergence * c->d.M_divergence;
     a.eps2 = c->d.epsilon_stationnary * c->d.epsilon_stationnary;
+    a.esc_lo = std::sqrt(0.5 * a.M2) * (1. - 1e-12);
+    a.eps_hi = std::sqrt(a.eps2) * (1. + 1e-12);
     a.calc_orbit = c->d.calc_orbit ? 1 : 0;
     a.backshift = c->d.calc_orbit ? c->d.backshift : 1;
     if (c->d.kind == FSG_KIND_BS) a.nz = 2 + (a.calc_dc ? 4 : 0) + 2 * a.calc_orbit;

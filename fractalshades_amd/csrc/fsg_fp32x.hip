@@ -224,7 +224,7 @@ __device__ __forceinline__ float l2(float x, float y) { return __builtin_sqrtf(x
 
 template <int KIND, int DEG>
 struct HoloS32 {
-    struct State { xs z, c, d, h; float cx, cy, e2; int32_t w, n, steps; bool dyn, nul; };
+    struct State { xs z, c, d, h; float cx, cy, e2; int32_t w, n, jl, steps; bool dyn, nul; };
 
     // c in z's scale, after z's exponent moved
     __device__ static void sync_c(State &s) {
@@ -275,7 +275,7 @@ struct HoloS32 {
         s.d = xs_zero(); s.h = xs_zero();
         s.e2 = 0.f;
         sync_c(s);
-        s.w = 0; s.n = 0; s.steps = 0; s.dyn = true; s.nul = false;
+        s.w = 0; s.n = 0; s.jl = 0; s.steps = 0; s.dyn = true; s.nul = false;
     }
 
     // one plain step on mantissas: the orbit point Zf (absolute, binary32),
@@ -372,19 +372,24 @@ struct HoloS32 {
         return xs{ex, ey, T};
     }
 
-    __device__ static int step(State &s, const KArgs &a, Counters &k) {
+    __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason) {
+        reason = step_reason(s, a, k);
+        return reason >= 0;
+    }
+    // the stop reason, -1: not stopped
+    __device__ static int step_reason(State &s, const KArgs &a, Counters &k) {
         const Tables &t = a.t;
         const xs *Zx = (const xs *)a.tx.Zx, *DC = (const xs *)a.tx.DCx, *DZ = (const xs *)a.tx.DZx;
         if (++s.steps > FP32X_STEP_CAP) return REASON_UNSURE;
         if ((s.w & 7) == 0) {
             renorm(s);
-            while (t.bla_on && (s.w & 7) == 0) {
+            k.looks += t.bla_on != 0;
+            while (t.bla_on) {
                 const double az = ldexp((double)hypotf(s.z.x, s.z.y), max(s.z.e, -2000));
                 const double eb = err_abs(s) + 0x1p-21 * az;
                 int32_t idx;
                 bool unsure = false;
                 const int32_t st = bla_find_m(t, az, eb, s.w, idx, unsure);
-                k.tries++;
                 if (unsure) return REASON_UNSURE;
                 if (st == 0) break;
                 // z <- A z + B c, d <- A d, h <- A h (A, B normalised records)
@@ -402,10 +407,10 @@ struct HoloS32 {
                 s.n += st;
                 s.w += st;                      // w + st < first_invalid <= order
                 renorm(s);
-                k.bla++; k.bla_it += st;
+                s.jl += st; k.bla++;
             }
         }
-        s.n += 1; k.plain++;
+        s.n += 1;
         const xs Zr = Zx[s.w];
         const xs Zd = (a.calc_dc && !s.dyn) ? DC[s.w] : xs_zero();
         const xs Zh = a.calc_dz ? (s.nul ? DZ[0] : DZ[s.w]) : xs_zero();
@@ -663,7 +668,7 @@ hipError_t build_xsr_tables(const Tables &t, TablesX &x, hipStream_t stream) {
 
 template <int FL>
 struct BsF32 {
-    struct State { xsr x, y, P[4], a, b; double xs, ys; int32_t w, n; bool dyn; };
+    struct State { xsr x, y, P[4], a, b; double xs, ys; int32_t w, n, jl; bool dyn; };
 
     // the tables hold xsr_from of the binary64 values (build_xsr_tables)
     __device__ static xsr PATH(const KArgs &a, int q, int32_t i) { return static_cast<const xsr *>(a.tx.BSx[q])[i]; }
@@ -678,17 +683,20 @@ struct BsF32 {
         const xsr z0 = xsr{0.f, XS_ZERO_E};
         s.x = z0; s.y = z0; s.P[0] = s.P[1] = s.P[2] = s.P[3] = z0;
         s.xs = 0.; s.ys = 0.;
-        s.w = 0; s.n = 0; s.dyn = true;
+        s.w = 0; s.n = 0; s.jl = 0; s.dyn = true;
     }
 
-    __device__ static int step(State &s, const KArgs &a, Counters &k) {
+    __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason) {
+        reason = step_reason(s, a, k);
+        return reason >= 0;
+    }
+    // the stop reason, -1: not stopped
+    __device__ static int step_reason(State &s, const KArgs &a, Counters &k) {
         const Tables &t = a.t;
-        while (t.bla_on && (s.w & 7) == 0) {
-            int32_t idx;
-            const int32_t st = bla_find(t, hypot_key(s.xs, s.ys), s.w, idx);
-            k.tries++;
-            if (st == 0) break;
-            {
+        if (t.bla_on && (s.w & 7) == 0) {
+            k.looks++;
+            int32_t idx, st;
+            while ((st = bla_find(t, hypot_key(s.xs, s.ys), s.w, idx)) != 0) {
                 const double *M = t.M + 8 * idx;
                 s.n += st; s.w += st;
                 const xzs x = as_zs(s.x), y = as_zs(s.y), ca = as_zs(s.a), cb = as_zs(s.b);
@@ -702,10 +710,10 @@ struct BsF32 {
                     s.P[2] = xsr_of(mul_w(M[2], P0) + mul_w(M[3], P2));
                     s.P[3] = xsr_of(mul_w(M[2], P1) + mul_w(M[3], P3));
                 }
-                k.bla++; k.bla_it += st;
+                s.jl += st; k.bla++;
             }
         }
-        s.n += 1; k.plain++;
+        s.n += 1;
         xsr X, Y;
         ZR(a, s.w, X, Y);
         // one iteration on lazily normalised values, renormalised once

@@ -87,6 +87,9 @@ struct KArgs {
     double drift_m[2]; int32_t drift_e[2];
     int32_t max_iter; int32_t calc_dc; int32_t calc_dz; int32_t pad2;
     double M2, eps2;
+    // filters of the escape and interior tests: |Z + z|^2 > M2 only if a component
+    // exceeds esc_lo, |dz/dz|^2 < eps2 only if each component is below eps_hi
+    double esc_lo, eps_hi;
     // pixels: complex128 screen offsets in units of dx ("c_pix")
     const double *pix;
     int64_t npts;

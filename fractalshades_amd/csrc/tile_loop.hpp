@@ -8,8 +8,11 @@
 
 namespace fsg {
 
-// a lane's counts (a lane's plain steps stay far below 2^32: 2000 s of them)
-struct Counters { unsigned plain, bla, reb, tries; unsigned long long bla_it; };
+// a lane's counts (a lane's plain steps stay far below 2^32: 2000 s of them).
+// looks: runs of BLA lookups, each of which ends with one that does not jump.
+// A pixel's plain steps and the iterations its jumps cover are added when it
+// stops, from its n and its sum of jump lengths (State::jl).
+struct Counters { unsigned plain, bla, reb, looks; unsigned long long bla_it; };
 
 // Stop reason of a pixel whose binary32 result may differ from the binary64
 // loop's (a decision taken within the pixel's error bound): set by the
@@ -295,8 +298,9 @@ __device__ __forceinline__ void tile_loop(const KArgs &a) {
                 if constexpr (is_lazy<Model>::value) {
                     if ((++trips & renorm_mask) == 0u) Model::renorm(s, a);
                 }
-                reason = Model::step(s, a, k);
-            } while (reason < 0);
+            } while (!Model::step(s, a, k, reason));
+            k.plain += (unsigned)(s.n - s.jl);
+            k.bla_it += (unsigned)s.jl;
             Model::finish(s, a, cold_args(), idx, reason);
             unsure += (reason == REASON_UNSURE);
         }
@@ -310,7 +314,7 @@ __device__ __forceinline__ void tile_loop(const KArgs &a) {
     __shared__ unsigned long long part[16][6];
     static_assert(sizeof(part) <= TILE_STATIC_LDS, "static LDS of the tile loop");
     const unsigned long long c[6] = {wave_sum(k.plain), wave_sum(k.bla), wave_sum(k.bla_it),
-                                     wave_sum(k.reb), wave_sum(k.tries), wave_sum(unsure)};
+                                     wave_sum(k.reb), wave_sum((unsigned long long)k.looks + k.bla), wave_sum(unsure)};
     const int wv = (int)(threadIdx.x >> 6);
     if (__lane_id() == 0) {
 #pragma unroll
