@@ -2,6 +2,7 @@
 filter taken by one component decides first: the oracle's results bit for bit
 for escape radii from 2 to 1e100 and stationarity bounds from loose to one
 whose square underflows, binary64 and extended-range deltas."""
+import numpy as np
 import pytest
 
 import frames
@@ -39,4 +40,7 @@ def test_stop_tests_bitexact(model, dx, radius, eps):
     ref = orc.OracleCtx(args.fields, args.arrays).cycles(c_pix)
     assert 2 * ref[1].max() < len(args.arrays["Zn_path"])  # no pixel past the reference orbit's end
     got, _ = run_gpu(args, c_pix)
+    for Z in (got[0], ref[0]):                  # an overflown pixel's NaNs have no sign
+        v = Z.view(np.float64)
+        v[np.isnan(v)] = np.nan
     assert_same(got, ref)
