@@ -292,13 +292,17 @@ __device__ __forceinline__ void tile_loop(const KArgs &a) {
         if (filled == 0u) break;
         if (__lane_id() < filled) {
             Model::init(s, g, g.pix[2 * idx], g.pix[2 * idx + 1]);
-            unsigned trips = 0;
             int reason;
-            do {
-                if constexpr (is_lazy<Model>::value) {
-                    if ((++trips & renorm_mask) == 0u) Model::renorm(s, a);
+            if constexpr (is_lazy<Model>::value) {
+                // trips: uniform over the lanes still iterating, in a scalar register
+                unsigned trips = 0;
+                for (;; trips++) {
+                    if ((trips & renorm_mask) == renorm_mask) Model::renorm(s, a, (int32_t)trips);
+                    if (Model::step(s, a, k, reason, (int32_t)trips)) break;
                 }
-            } while (!Model::step(s, a, k, reason));
+            } else {
+                while (!Model::step(s, a, k, reason)) {}
+            }
             k.plain += (unsigned)(s.n - s.jl);
             k.bla_it += (unsigned)s.jl;
             Model::finish(s, a, cold_args(), idx, reason);

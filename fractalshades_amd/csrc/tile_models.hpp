@@ -286,12 +286,14 @@ struct HoloStd {
 // 2^+-700: a step multiplies it by at least 2^(LOW_Z (d - 1)) but for
 // cancellation and at most d |Z + z|^(d - 1), and adds no more than 2^FAR
 // times the operand's mantissa.
-// The loop is bound by vector instruction issue: a z^2 + c step takes 104
-// instructions (dz/dc and dz/dz on; 58 are the algorithmic flops) where
-// normalising every result and aligning every sum took 174.  2048x2048 frames
-// with it: 1e-300 999 -> 792 us, 1e-2000 1212 -> 1027 us, interior-dominated
-// 24.7 -> 22.3 ms; 1920x1080 at 1e-800: z^3 + c 850 -> 729 us, z^6 + c 868 ->
-// 666 us.
+// The loop is bound by vector instruction issue (97 % of the cycles on the
+// 2048x2048 frames): a z^2 + c step takes about 80 instructions (dz/dc and
+// dz/dz on; 58 are the algorithmic flops) where normalising every result and
+// aligning every sum took 174.  2048x2048 frames, with drifting mantissas and
+// then with what a step shares with the last one carried and the exponents of
+// dz/dc and dz/dz relative to the trips: 1e-300 999 -> 792, 636 -> 596 us,
+// 1e-2000 1212 -> 1027, 850 -> 774 us, interior-dominated 24.7 -> 22.3, 17.3 ->
+// 16.5 ms; 1920x1080 at 1e-800: z^3 + c 850 -> 729 us, z^6 + c 868 -> 666 us.
 // DER >= 0 fixes the derivatives at compile time (bit 0: dz/dc, bit 1:
 // dz/dz): the step is then one block of straight-line code, which the
 // compiler schedules across the z, dz/dc and dz/dz recurrences; DER = -1
@@ -300,8 +302,17 @@ template <int KIND, int DEG, bool ORB = false, int DER = -1>
 struct HoloXr {
     __device__ static bool DC_ON(const KArgs &a) { if constexpr (DER >= 0) return (DER & 1) != 0; else return a.calc_dc != 0; }
     __device__ static bool DZ_ON(const KArgs &a) { if constexpr (DER >= 0) return (DER & 2) != 0; else return a.calc_dz != 0; }
-    struct State { xl z, d, h, c; cplx zs; int32_t w, n, jl; bool dyn, nul; OrbitRec<ORB> orb; };
+    // z^2 + c carries what a step shares with the one before it: the orbit
+    // point Z at w and its code kz, A = Z + z (the value of the escape test) and
+    // the dZndz value Zh; they are loaded where w becomes a multiple of 8 (the
+    // first step, a jump, a rebase, the end of a period).
+    struct State { xl z, d, h, c; cplx zs, Z, A; xz Zh; int32_t kz, w, n, jl; bool dyn, nul; OrbitRec<ORB> orb; };
     static constexpr bool LAZY = true;
+    // z^2 + c: each step multiplies dz/dc and dz/dz by 2, so their exponents
+    // grow by one a trip.  d.e and h.e then hold t - (exponent), t the trips of
+    // the pixel, and a step leaves them as they are.  rel converts both ways.
+    static constexpr bool REL = KIND == KIND_M2;
+    __device__ static int32_t rel(int32_t e, int32_t t) { return REL ? t - e : e; }
     static constexpr int32_t LOW_Z = (KIND == KIND_M2) ? -20 : -60 / (DEG - 1), HIGH_Z = 60, FAR = 256;
 
     // The z^d + c derivative recurrence of one quantity: its delta v 2^e, the
@@ -330,11 +341,21 @@ struct HoloXr {
         }
     };
 
-    __device__ static void renorm(State &s, const KArgs &a) {
+    // after t trips
+    __device__ static void renorm(State &s, const KArgs &a, int32_t t) {
         s.z = xl_of(as_z(s.z));
-        if (DC_ON(a)) s.d = xl_of(as_z(s.d));
-        if (DZ_ON(a)) s.h = xl_of(as_z(s.h));
+        const int32_t zero = rel(XL_ZERO_E, t);
+        if (DC_ON(a)) renorm_deriv(s.d, zero);
+        if (DZ_ON(a)) renorm_deriv(s.h, zero);
     }
+    __device__ static void renorm_deriv(xl &v, int32_t zero) {
+        const double mx = amax(v.re, v.im);
+        const int32_t k = dexp(mx) - 1;
+        v.re = ldexp(v.re, -k); v.im = ldexp(v.im, -k);
+        v.e = mx == 0. ? zero : REL ? v.e - k : v.e + k;
+    }
+    // a derivative with its exponent, after t trips
+    __device__ static xl deriv(const xl &v, int32_t t) { xl r = v; r.e = rel(v.e, t); return xl_of(as_z(r)); }
 
     // derivative path values, unnormalised: the host's Xrange records keep
     // |mantissa| within 2^+-100, and a zero entry carries the zero exponent
@@ -358,18 +379,22 @@ struct HoloXr {
     __device__ static void init(State &s, const KArgs &a, double px, double py) {
         s.c = c_from_pix_xl(a, px, py);
         s.z = xl_zero(); s.d = xl_zero(); s.h = xl_zero();
+        s.d.e = s.h.e = rel(XL_ZERO_E, 0);
         s.zs = zc();
         s.w = 0; s.n = 0; s.jl = 0; s.dyn = true; s.nul = false;
         s.orb.reset(a.backshift);
     }
 
-    __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason) {
+    __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason, int32_t trip) {
         const Tables &t = a.t;
-        if (t.bla_on && (s.w & 7) == 0) {
-            s.z = xl_of(as_z(s.z));                              // as the key takes it
-            k.looks++;
+        if ((KIND == KIND_M2 || t.bla_on) && (s.w & 7) == 0) {
             int32_t idx, st;
-            while ((st = bla_lookup(t, s.z, s.w, idx)) != 0) {
+            const int32_t w0 = s.w;
+            if (t.bla_on) {
+                s.z = xl_of(as_z(s.z));                          // as the key takes it
+                k.looks++;
+            }
+            while (t.bla_on && (st = bla_lookup(t, s.z, s.w, idx)) != 0) {
                 const double *Mb = t.M + 4 * idx;
                 cplx A = mk(Mb[0], Mb[1]), B = mk(Mb[2], Mb[3]);
                 s.n += st;
@@ -385,10 +410,16 @@ struct HoloXr {
                 if (sc > FAR) { s.z.re = ldexp(s.z.re, -sc); s.z.im = ldexp(s.z.im, -sc); ez += sc; sc = 0; }
                 const cplx u = mk(s.z.re, s.z.im) * A, v = mk(s.c.re, s.c.im) * B;
                 s.z = xl_n(u.re + ldexp(v.re, sc), u.im + ldexp(v.im, sc), ez);
-                s.zs = mk(ldexp(s.z.re, s.z.e), ldexp(s.z.im, s.z.e));
-                if (DC_ON(a)) { const cplx p = mk(s.d.re, s.d.im) * A; s.d.re = p.re; s.d.im = p.im; s.d.e += kA; }
-                if (DZ_ON(a)) { const cplx p = mk(s.h.re, s.h.im) * A; s.h.re = p.re; s.h.im = p.im; s.h.e += kA; }
+                if (DC_ON(a)) { const cplx p = mk(s.d.re, s.d.im) * A; s.d.re = p.re; s.d.im = p.im; s.d.e += REL ? -kA : kA; }
+                if (DZ_ON(a)) { const cplx p = mk(s.h.re, s.h.im) * A; s.h.re = p.re; s.h.im = p.im; s.h.e += REL ? -kA : kA; }
                 s.jl += st; k.bla++;
+            }
+            if (s.w != w0) s.zs = mk(ldexp(s.z.re, s.z.e), ldexp(s.z.im, s.z.e));
+            if constexpr (KIND == KIND_M2) {
+                s.Z = t.Zn[s.w];
+                s.kz = t.zn_k[s.w];
+                if (DZ_ON(a)) s.Zh = DZz(t, s.nul ? 0 : s.w);
+                s.A = s.zs + s.Z;
             }
         }
         s.n += 1;
@@ -396,56 +427,74 @@ struct HoloXr {
         // orbit point, its code and the path values at w, the next orbit
         // point and its code (escape and rebase tests) and the dZndz value of
         // the interior test (z^d + c: after the step, whose partial products
-        // need the registers; loaded first, it spilled at d = 3)
-        const int32_t w1 = (s.w + 1 >= t.order) ? 0 : s.w + 1;
-        const int32_t k0 = t.zn_k[s.w];
-        const cplx Z0 = t.Zn[s.w], Z1 = t.Zn[w1];
+        // need the registers; loaded first, it spilled at d = 3).  A step at
+        // the end of the period or next to the orbit's last point (edge) takes
+        // the general tests.
+        int32_t w1 = s.w + 1, wh = w1;                   // wh: index of the interior test's dZndz value
+        const bool edge = w1 >= min(t.order, t.div_iter - 1);
+        if (edge) {
+            pin(w1);
+            if (w1 >= t.order) { w1 = 0; wh = s.n == t.order ? t.L : 0; }
+        }
+        if (DZ_ON(a) && s.nul) wh = 0;
+        cplx Z0, Z1;
+        int32_t k0, k1 = 0;
         xz Zd = xz_zero(), Zh = xz_zero(), H1 = xz_zero();
         if (DC_ON(a)) Zd = DCz(t, s.w);
-        if (DZ_ON(a)) {
-            Zh = DZz(t, s.nul ? 0 : s.w);
-            if constexpr (KIND == KIND_M2) H1 = DZz(t, s.nul ? 0 : (s.n == t.order ? t.L : w1));
+        if constexpr (KIND == KIND_M2) {
+            Z0 = s.Z; k0 = s.kz;
+            if (DZ_ON(a)) Zh = s.Zh;
+        } else {
+            Z0 = t.Zn[s.w]; k0 = t.zn_k[s.w]; Z1 = t.Zn[w1];
+            if (DZ_ON(a)) Zh = DZz(t, s.nul ? 0 : s.w);
         }
         if constexpr (KIND == KIND_M2) {
             // mandelbrot_M2.py:607-622: z (z + 2 Z) + c, 2 ((Z + z) d + Zd z)
-            cplx A = s.zs + Z0;                                      // Z + z
+            cplx A = s.A;                                            // Z + z
             cplx W = mk(__builtin_fma(2., Z0.re, s.zs.re), __builtin_fma(2., Z0.im, s.zs.im));   // z + 2 Z
-            int32_t eK = 0;                                          // their exponent
+            int32_t zt = s.z.e - trip;
+            pin(zt);
             if (k0 < LOW_Z || s.dyn) {
                 if (s.dyn) Zd = xz_zero();
                 if (k0 < LOW_Z) {
                     const xl Zr = ZRv(t, k0, Z0);
                     s.z = xl_of(as_z(s.z));
-                    eK = max(Zr.e, s.z.e);
+                    zt = s.z.e - trip;
+                    int32_t eK = max(Zr.e, s.z.e);               // exponent of A and W
                     if (eK < XL_ZERO_E / 2) eK = 0;              // Z = z = 0
                     const int32_t sZ = shift_of(Zr.e, eK), sz = shift_of(s.z.e, eK);
                     const cplx Zk = mk(ldexp(Zr.re, sZ), ldexp(Zr.im, sZ)), zk = mk(ldexp(s.z.re, sz), ldexp(s.z.im, sz));
                     A = Zk + zk;
                     W = mk(__builtin_fma(2., Zk.re, zk.re), __builtin_fma(2., Zk.im, zk.im));
+                    s.z.e += eK; s.d.e -= eK; s.h.e -= eK;
                 }
             }
             // the shifts of c and of the paths' terms to the exponents of
             // z W, A d and A h
-            int32_t ez = s.z.e + eK, ed = s.d.e + eK, eh = s.h.e + eK;
-            int32_t sz = s.c.e - ez;
-            int32_t sd = DC_ON(a) ? Zd.e + s.z.e - ed : -1, sh = DZ_ON(a) ? Zh.e + s.z.e - eh : -1;
+            int32_t sz = s.c.e - s.z.e;
+            int32_t sd = DC_ON(a) ? Zd.e + zt + s.d.e : -1, sh = DZ_ON(a) ? Zh.e + zt + s.h.e : -1;
+            pin(sd); pin(sh);
+            pin_after(w1, W.re, W.im);
+            Z1 = t.Zn[w1]; k1 = t.zn_k[w1];
             if (max(sz, max(sd, sh)) > FAR) {
-                if (sz > FAR) { W = mk(ldexp(W.re, -sz), ldexp(W.im, -sz)); ez += sz; sz = 0; }
-                if (sd > FAR) { s.d.re = ldexp(s.d.re, -sd); s.d.im = ldexp(s.d.im, -sd); ed += sd; sd = 0; }
-                if (sh > FAR) { s.h.re = ldexp(s.h.re, -sh); s.h.im = ldexp(s.h.im, -sh); eh += sh; sh = 0; }
+                if (sz > FAR) { W = mk(ldexp(W.re, -sz), ldexp(W.im, -sz)); s.z.e += sz; sz = 0; }
+                if (sd > FAR) { s.d.re = ldexp(s.d.re, -sd); s.d.im = ldexp(s.d.im, -sd); s.d.e -= sd; sd = 0; }
+                if (sh > FAR) { s.h.re = ldexp(s.h.re, -sh); s.h.im = ldexp(s.h.im, -sh); s.h.e -= sh; sh = 0; }
             }
             const cplx z = mk(s.z.re, s.z.im);
             if (DC_ON(a)) {
                 const cplx u = A * mk(s.d.re, s.d.im), v = mk(Zd.re, Zd.im) * z;
-                s.d.re = u.re + ldexp(v.re, sd); s.d.im = u.im + ldexp(v.im, sd); s.d.e = ed + 1;
+                s.d.re = u.re + ldexp(v.re, sd); s.d.im = u.im + ldexp(v.im, sd);
             }
             if (DZ_ON(a)) {
                 const cplx u = A * mk(s.h.re, s.h.im), v = mk(Zh.re, Zh.im) * z;
-                s.h.re = u.re + ldexp(v.re, sh); s.h.im = u.im + ldexp(v.im, sh); s.h.e = eh + 1;
+                pin_after(wh, v.re, v.im);
+                H1 = DZz(t, wh);
+                s.h.re = u.re + ldexp(v.re, sh); s.h.im = u.im + ldexp(v.im, sh);
             }
             const cplx u = z * W;
-            s.z.re = u.re + ldexp(s.c.re, sz); s.z.im = u.im + ldexp(s.c.im, sz); s.z.e = ez;
-            s.zs = mk(ldexp(s.z.re, ez), ldexp(s.z.im, ez));
+            s.z.re = u.re + ldexp(s.c.re, sz); s.z.im = u.im + ldexp(s.c.im, sz);
+            s.zs = mk(ldexp(s.z.re, s.z.e), ldexp(s.z.im, s.z.e));
         } else {
             // mandelbrot_Mn.py:646-729 (p_zn_derivs of models.hpp).  zk, Zk: z
             // and Z in units of 2^eK; the running factor mul of term q is then
@@ -500,7 +549,7 @@ struct HoloXr {
             if (DZ_ON(a)) { s.h.re = D[1].t.re; s.h.im = D[1].t.im; s.h.e = D[1].e + (DEG - 1) * eK; }
             s.z.re = tmp.re + ldexp(s.c.re, sz); s.z.im = tmp.im + ldexp(s.c.im, sz); s.z.e = ez;
             s.zs = mk(ldexp(s.z.re, ez), ldexp(s.z.im, ez));
-            if (DZ_ON(a)) H1 = DZz(t, s.nul ? 0 : (s.n == t.order ? t.L : w1));
+            if (DZ_ON(a)) H1 = DZz(t, wh);
         }
         s.w = w1;
         // the stop and rebase tests evaluated together, as in HoloStd
@@ -509,25 +558,27 @@ struct HoloXr {
         bool t_int = false;
         double qre = 0.;
         if (DZ_ON(a)) {
-            qre = ldexp(s.h.re, s.h.e) + ldexp(H1.re, H1.e);
+            qre = ldexp(s.h.re, rel(s.h.e, trip + 1)) + ldexp(H1.re, H1.e);
             t_int = fabs(qre) < a.eps_hi;
         }
         const cplx ZZ = s.zs + Z1;
         const bool t_esc = ORB ? ZZ.re * ZZ.re + ZZ.im * ZZ.im > a.M2 : amax(ZZ.re, ZZ.im) > a.esc_lo;
-        const bool reb_div = s.w >= t.div_iter - 1;
         const bool dyn = (fabs(ZZ.re) <= fabs(s.zs.re)) && (fabs(ZZ.im) <= fabs(s.zs.im));
+        if constexpr (KIND == KIND_M2) { s.Z = Z1; s.kz = k1; s.A = ZZ; s.Zh = H1; }
         if constexpr (!ORB) {
-            if (!(s.n >= a.max_iter || t_int || t_esc || reb_div || dyn)) { s.dyn = false; return false; }
+            if (!(s.n >= a.max_iter || t_int || t_esc || edge || dyn)) { s.dyn = false; return false; }
         }
-        if (s.n >= a.max_iter) { reason = 0; return true; }
+        const auto stop = [&](int r) { s.d.e = rel(s.d.e, trip + 1); reason = r; return true; };
+        if (s.n >= a.max_iter) return stop(0);
         if (t_int) {
-            const double qim = ldexp(s.h.im, s.h.e) + ldexp(H1.im, H1.e);
-            if (qre * qre + qim * qim < a.eps2) { reason = 2; return true; }
+            const double qim = ldexp(s.h.im, rel(s.h.e, trip + 1)) + ldexp(H1.im, H1.e);
+            if (qre * qre + qim * qim < a.eps2) return stop(2);
         }
         s.orb.record(s.n, a.backshift, ZZ.re, ZZ.im);
-        if (t_esc && (ORB || ZZ.re * ZZ.re + ZZ.im * ZZ.im > a.M2)) { reason = 1; return true; }
+        if (t_esc && (ORB || ZZ.re * ZZ.re + ZZ.im * ZZ.im > a.M2)) return stop(1);
         // both rebases (perturbation.py:1283-1372) share the derivative
         // updates: one block, whichever of them a lane takes
+        const bool reb_div = s.w >= t.div_iter - 1;
         bool reb = reb_div;
         xl ZZx;
         if (!reb_div) {
@@ -542,10 +593,11 @@ struct HoloXr {
             if (reb_div) { s.zs = ZZ; s.z = xl_of(ZZ); }
             else { s.z = ZZx; s.zs = to_std(ZZx); }
             // the path values unnormalised: the sum's normalisation covers them
-            if (DC_ON(a)) s.d = add_n(as_z(xl_of(as_z(s.d))), DCz(t, s.w));
+            if (DC_ON(a)) { s.d = add_n(as_z(deriv(s.d, trip + 1)), DCz(t, s.w)); s.d.e = rel(s.d.e, trip + 1); }
             if (DZ_ON(a)) {
-                s.h = xl_of(as_z(s.h));
+                s.h = deriv(s.h, trip + 1);
                 if (!s.nul) s.h = add_n(as_z(s.h), H1);   // dZndz at w (at L after a full period)
+                s.h.e = rel(s.h.e, trip + 1);
                 s.nul = true;
             }
             s.w = 0;
@@ -556,7 +608,7 @@ struct HoloXr {
 
     __device__ static void finish(State &s, const KArgs &a, const KArgs &g, int64_t i, int reason) {
         const int64_t n = g.ld;
-        renorm(s, a);
+        s.z = xl_of(as_z(s.z));
         cplx z = to_std(s.z) + a.t.Zn[s.w];
         g.Z[2 * i] = z.re; g.Z[2 * i + 1] = z.im;
         int f = 1;
@@ -564,7 +616,7 @@ struct HoloXr {
         // standard dzndz field keeps the 0 written by numba_initialize
         if (DZ_ON(a)) { g.Z[2 * (n + i)] = 0.; g.Z[2 * (n + i) + 1] = 0.; f = 2; }
         if (DC_ON(a)) {
-            cplx d = to_std(add_n(as_z(s.d), DCz(a.t, s.w)));
+            cplx d = to_std(add_n(as_z(xl_of(as_z(s.d))), DCz(a.t, s.w)));
             g.Z[2 * (f * n + i)] = d.re; g.Z[2 * (f * n + i) + 1] = d.im;
         }
         if constexpr (ORB) orbit_finish_holo<KIND, DEG>(s.orb, a, g, s.n, to_std(s.c), i);
@@ -688,7 +740,7 @@ struct BsXr {
         for (int q = 0; q < 4; q++) P[q] = ldexp(P[q], -k);
         e = (mx == 0.) ? XL_ZERO_E : e + k;
     }
-    __device__ static void renorm(State &s, const KArgs &a) {
+    __device__ static void renorm(State &s, const KArgs &a, int32_t = 0) {
         norm2(s.x, s.y, s.e);
         if (DC_ON(a)) norm4(s.P, s.eP);
     }
@@ -821,7 +873,7 @@ struct BsXr {
         join2(xlf_of(nx), xlf_of(ny), s.x, s.y, s.e);
     }
 
-    __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason) {
+    __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason, int32_t) {
         const Tables &t = a.t;
         if (t.bla_on && (s.w & 7) == 0) {
             k.looks++;
