@@ -695,23 +695,28 @@ struct BsF32 {
         const Tables &t = a.t;
         if (t.bla_on && (s.w & 7) == 0) {
             k.looks++;
-            int32_t idx, st;
-            while ((st = bla_find(t, hypot_key(s.xs, s.ys), s.w, idx)) != 0) {
-                const double *M = t.M + 8 * idx;
-                s.n += st; s.w += st;
-                const xzs x = as_zs(s.x), y = as_zs(s.y), ca = as_zs(s.a), cb = as_zs(s.b);
-                s.x = xsr_of(mul_w(M[0], x) + mul_w(M[1], y) + mul_w(M[4], ca) + mul_w(M[5], cb));
-                s.y = xsr_of(mul_w(M[2], x) + mul_w(M[3], y) + mul_w(M[6], ca) + mul_w(M[7], cb));
-                s.xs = xsr_to_d(s.x); s.ys = xsr_to_d(s.y);
-                if (a.calc_dc) {
-                    const xzs P0 = as_zs(s.P[0]), P1 = as_zs(s.P[1]), P2 = as_zs(s.P[2]), P3 = as_zs(s.P[3]);
-                    s.P[0] = xsr_of(mul_w(M[0], P0) + mul_w(M[1], P2));
-                    s.P[1] = xsr_of(mul_w(M[0], P1) + mul_w(M[1], P3));
-                    s.P[2] = xsr_of(mul_w(M[2], P0) + mul_w(M[3], P2));
-                    s.P[3] = xsr_of(mul_w(M[2], P1) + mul_w(M[3], P3));
+            int32_t stage, idx;
+            do {
+                stage = bla_find(t, hypot_key(s.xs, s.ys), s.w, idx);
+                if (stage >= 0) {
+                    const int32_t st = 8 << stage;
+                    const double *M = t.M + 8 * idx;
+                    s.n += st; s.w += st;
+                    const xzs x = as_zs(s.x), y = as_zs(s.y), ca = as_zs(s.a), cb = as_zs(s.b);
+                    s.x = xsr_of(mul_w(M[0], x) + mul_w(M[1], y) + mul_w(M[4], ca) + mul_w(M[5], cb));
+                    s.y = xsr_of(mul_w(M[2], x) + mul_w(M[3], y) + mul_w(M[6], ca) + mul_w(M[7], cb));
+                    s.xs = xsr_to_d(s.x); s.ys = xsr_to_d(s.y);
+                    if (a.calc_dc) {
+                        const xzs P0 = as_zs(s.P[0]), P1 = as_zs(s.P[1]), P2 = as_zs(s.P[2]), P3 = as_zs(s.P[3]);
+                        s.P[0] = xsr_of(mul_w(M[0], P0) + mul_w(M[1], P2));
+                        s.P[1] = xsr_of(mul_w(M[0], P1) + mul_w(M[1], P3));
+                        s.P[2] = xsr_of(mul_w(M[2], P0) + mul_w(M[3], P2));
+                        s.P[3] = xsr_of(mul_w(M[2], P1) + mul_w(M[3], P3));
+                    }
+                    s.jl += st; k.bla++;
                 }
-                s.jl += st; k.bla++;
-            }
+                pin(stage);
+            } while (stage >= 0);
         }
         s.n += 1;
         xsr X, Y;

@@ -54,6 +54,13 @@ __device__ __forceinline__ int64_t grid_slot(int64_t s, int64_t n, int64_t w) {
     return (int64_t)grid_slot_t<uint64_t>((uint64_t)s, (uint64_t)n, (uint64_t)w);
 }
 
+// v as it is, for the compiler a new value: it neither rewrites what follows
+// in terms of what v was made from nor turns a branch around it into selects
+__device__ __forceinline__ void pin(int32_t &v) { asm("" : "+v"(v)); }
+// the same, not before x and y are known: a load at index v then takes the
+// registers that x and y were made from instead of copying into them later
+__device__ __forceinline__ void pin_after(int32_t &v, double x, double y) { asm("" : "+v"(v) : "v"(x), "v"(y)); }
+
 // --------------------------------------------------------------------------
 // BLA stage selection (ref_BLA_get, perturbation.py:2116-2170).  The tree
 // keeps the stage s >= 3 jump starting at iteration w (a multiple of 2^s) at
@@ -65,31 +72,41 @@ __device__ __forceinline__ int64_t grid_slot(int64_t s, int64_t n, int64_t w) {
 // perturbation.py:2020-2023), so r never grows with the stage for a fixed
 // start.  The highest valid stage is therefore found by bisection, with
 // about log2(stages) dependent loads instead of one per stage.
-// Returns the jump length (0 if no stage is valid) and the entry index.
+// Returns the stage less 3 and the entry's index, -1 if no stage is valid; the
+// jump covers 8 << stage iterations.
 // zk: the key of |z| (bla_key.hpp), compared with the radii's keys.
+// A run of lookups is written do { if (stage >= 0) jump; pin(stage); } while
+// (stage >= 0): the jump then updates the pixel's state in place, where a loop
+// left from its middle copies it at every lookup (14 instructions).
+// A lookup takes 13 vector instructions besides the key where the lowest stage
+// fails, 6 more and 8 per bisection step where it does not; with the bounds
+// computed before the first test and closed intervals it took 18 and 13 a step.
 __device__ __forceinline__ int32_t bla_find(const Tables &t, int64_t zk, int32_t w, int32_t &idx) {
-    const int32_t it = w >> 3;
     const int32_t invalid_step = t.first_invalid - w;
-    if (invalid_step <= 8) return 0;
-    const int32_t tz = (it == 0) ? 31 : __builtin_ctz((uint32_t)it);
-    const int32_t s_inv = 31 - __builtin_clz((uint32_t)(invalid_step - 1));   // 2^s < invalid_step
-    int32_t hi = min(min(3 + tz, t.stages_bla - 1), s_inv);
-    int32_t lo = 3, best = 0;
-    if (hi >= 3) {
+    int32_t stage = -1;
+    if (invalid_step > 8 && t.stages_bla > 3) {
+        const int64_t *rk = t.rk + (w >> 2);        // rk[2^s - 1]: stage s + 3
         // the lowest stage first: invalid there, invalid at every stage (the
         // prefix property), which settles 40 % of the lookups of the 1e-300
         // frame in one read instead of about four (C2 -2.8 %)
-        if (!(zk < t.rk[2 * it])) return 0;
-        best = 3; lo = 4;
+        if (zk < rk[0]) {
+            // stages that start at w (w a multiple of 2^stage; every one at
+            // w = 0), that the table has, and whose jump stays valid
+            // (2^stage < invalid_step)
+            const int32_t starts = __builtin_ctz((uint32_t)w | 0x80000000u);
+            const int32_t fits = 31 - __builtin_clz((uint32_t)(invalid_step - 1));
+            int32_t hi = min(min(starts, t.stages_bla - 1), fits) - 2;         // stage valid, hi not
+            stage = 0;
+            while (hi - stage > 1) {
+                const int32_t mid = (stage + hi) >> 1;
+                if (zk < rk[(1 << mid) - 1]) stage = mid;
+                else hi = mid;
+            }
+        }
     }
-    while (lo <= hi) {
-        const int32_t mid = (lo + hi) >> 1;
-        if (zk < t.rk[2 * it + (1 << (mid - 3)) - 1]) { best = mid; lo = mid + 1; }
-        else hi = mid - 1;
-    }
-    if (best == 0) return 0;
-    idx = 2 * it + (1 << (best - 3)) - 1;
-    return 1 << best;
+    pin(stage);            // one value for the caller's test, not an exit for each test above
+    idx = (w >> 2) + (1 << stage) - 1;
+    return stage;
 }
 
 // --------------------------------------------------------------------------

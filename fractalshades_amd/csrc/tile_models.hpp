@@ -168,17 +168,22 @@ struct HoloStd {
         const Tables &t = a.t;
         if (t.bla_on && (s.w & 7) == 0) {
             k.looks++;
-            int32_t idx, st;
-            while ((st = bla_lookup(t, s.z.re, s.z.im, s.w, idx)) != 0) {
-                const double *Mb = t.M + 4 * idx;
-                cplx A = mk(Mb[0], Mb[1]), B = mk(Mb[2], Mb[3]);
-                s.n += st;
-                s.w += st;                      // w + st < first_invalid <= order
-                s.z = A * s.z + B * s.c;
-                if (DC_ON(a)) s.d = A * s.d;
-                if (DZ_ON(a)) s.h = A * s.h;
-                s.jl += st; k.bla++;
-            }
+            int32_t stage, idx;
+            do {
+                stage = bla_lookup(t, s.z.re, s.z.im, s.w, idx);
+                if (stage >= 0) {
+                    const int32_t st = 8 << stage;
+                    const double *Mb = t.M + 4 * idx;
+                    cplx A = mk(Mb[0], Mb[1]), B = mk(Mb[2], Mb[3]);
+                    s.n += st;
+                    s.w += st;                      // w + st < first_invalid <= order
+                    s.z = A * s.z + B * s.c;
+                    if (DC_ON(a)) s.d = A * s.d;
+                    if (DZ_ON(a)) s.h = A * s.h;
+                    s.jl += st; k.bla++;
+                }
+                pin(stage);
+            } while (stage >= 0);
         }
         s.n += 1;
         // Every table value the step reads is loaded here, before any of it
@@ -388,33 +393,46 @@ struct HoloXr {
     __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason, int32_t trip) {
         const Tables &t = a.t;
         if ((KIND == KIND_M2 || t.bla_on) && (s.w & 7) == 0) {
-            int32_t idx, st;
+            int32_t stage, idx;
             const int32_t w0 = s.w;
             if (t.bla_on) {
                 s.z = xl_of(as_z(s.z));                          // as the key takes it
                 k.looks++;
+                do {
+                    stage = bla_lookup(t, s.z, s.w, idx);
+                    if (stage >= 0) {
+                        const int32_t st = 8 << stage;
+                        const double *Mb = t.M + 4 * idx;
+                        cplx A = mk(Mb[0], Mb[1]), B = mk(Mb[2], Mb[3]);
+                        s.n += st;
+                        s.w += st;
+                        // A's exponent apart: A can be near the end of the binary64
+                        // range, and dz/dc and dz/dz keep drifting mantissas (z alone
+                        // is normalised, for the next lookup): 56 vector instructions
+                        // instead of 86, with amax the 2048x2048 frames 720 -> 675 us
+                        // (1e-300), 946 -> 887 us (1e-2000), 20.4 -> 18.3 ms (interior)
+                        const int32_t kA = dexp(amax(A.re, A.im)) - 1;
+                        A = mk(ldexp(A.re, -kA), ldexp(A.im, -kA));
+                        int32_t ez = s.z.e + kA, sc = s.c.e - ez;
+                        pin(sc);
+                        if (sc > FAR) {
+                            pin(sc);
+                            s.z.re = ldexp(s.z.re, -sc); s.z.im = ldexp(s.z.im, -sc); ez += sc; sc = 0;
+                        }
+                        const cplx u = mk(s.z.re, s.z.im) * A, v = mk(s.c.re, s.c.im) * B;
+                        s.z = xl_n(u.re + ldexp(v.re, sc), u.im + ldexp(v.im, sc), ez);
+                        if (DC_ON(a)) { const cplx p = mk(s.d.re, s.d.im) * A; s.d.re = p.re; s.d.im = p.im; s.d.e += REL ? -kA : kA; }
+                        if (DZ_ON(a)) { const cplx p = mk(s.h.re, s.h.im) * A; s.h.re = p.re; s.h.im = p.im; s.h.e += REL ? -kA : kA; }
+                        s.jl += st; k.bla++;
+                    }
+                    pin(stage);
+                } while (stage >= 0);
             }
-            while (t.bla_on && (st = bla_lookup(t, s.z, s.w, idx)) != 0) {
-                const double *Mb = t.M + 4 * idx;
-                cplx A = mk(Mb[0], Mb[1]), B = mk(Mb[2], Mb[3]);
-                s.n += st;
-                s.w += st;
-                // A's exponent apart: A can be near the end of the binary64
-                // range, and dz/dc and dz/dz keep drifting mantissas (z alone
-                // is normalised, for the next lookup): 56 vector instructions
-                // instead of 86, with amax the 2048x2048 frames 720 -> 675 us
-                // (1e-300), 946 -> 887 us (1e-2000), 20.4 -> 18.3 ms (interior)
-                const int32_t kA = dexp(amax(A.re, A.im)) - 1;
-                A = mk(ldexp(A.re, -kA), ldexp(A.im, -kA));
-                int32_t ez = s.z.e + kA, sc = s.c.e - ez;
-                if (sc > FAR) { s.z.re = ldexp(s.z.re, -sc); s.z.im = ldexp(s.z.im, -sc); ez += sc; sc = 0; }
-                const cplx u = mk(s.z.re, s.z.im) * A, v = mk(s.c.re, s.c.im) * B;
-                s.z = xl_n(u.re + ldexp(v.re, sc), u.im + ldexp(v.im, sc), ez);
-                if (DC_ON(a)) { const cplx p = mk(s.d.re, s.d.im) * A; s.d.re = p.re; s.d.im = p.im; s.d.e += REL ? -kA : kA; }
-                if (DZ_ON(a)) { const cplx p = mk(s.h.re, s.h.im) * A; s.h.re = p.re; s.h.im = p.im; s.h.e += REL ? -kA : kA; }
-                s.jl += st; k.bla++;
+            if (s.w != w0) {
+                int32_t e = s.z.e;
+                pin(e);
+                s.zs = mk(ldexp(s.z.re, e), ldexp(s.z.im, e));
             }
-            if (s.w != w0) s.zs = mk(ldexp(s.z.re, s.z.e), ldexp(s.z.im, s.z.e));
             if constexpr (KIND == KIND_M2) {
                 s.Z = t.Zn[s.w];
                 s.kz = t.zn_k[s.w];
@@ -644,22 +662,27 @@ struct BsStd {
         const Tables &t = a.t;
         if (t.bla_on && (s.w & 7) == 0) {
             k.looks++;
-            int32_t idx, st;
-            while ((st = bla_lookup(t, s.x, s.y, s.w, idx)) != 0) {
-                const double *M = t.M + 8 * idx;
-                s.n += st; s.w += st;
-                double nx = M[0] * s.x + M[1] * s.y + M[4] * s.a + M[5] * s.b;
-                double ny = M[2] * s.x + M[3] * s.y + M[6] * s.a + M[7] * s.b;
-                s.x = nx; s.y = ny;
-                if (a.calc_dc) {
-                    double p0 = M[0] * s.P[0] + M[1] * s.P[2];
-                    double p1 = M[0] * s.P[1] + M[1] * s.P[3];
-                    double p2 = M[2] * s.P[0] + M[3] * s.P[2];
-                    double p3 = M[2] * s.P[1] + M[3] * s.P[3];
-                    s.P[0] = p0; s.P[1] = p1; s.P[2] = p2; s.P[3] = p3;
+            int32_t stage, idx;
+            do {
+                stage = bla_lookup(t, s.x, s.y, s.w, idx);
+                if (stage >= 0) {
+                    const int32_t st = 8 << stage;
+                    const double *M = t.M + 8 * idx;
+                    s.n += st; s.w += st;
+                    double nx = M[0] * s.x + M[1] * s.y + M[4] * s.a + M[5] * s.b;
+                    double ny = M[2] * s.x + M[3] * s.y + M[6] * s.a + M[7] * s.b;
+                    s.x = nx; s.y = ny;
+                    if (a.calc_dc) {
+                        double p0 = M[0] * s.P[0] + M[1] * s.P[2];
+                        double p1 = M[0] * s.P[1] + M[1] * s.P[3];
+                        double p2 = M[2] * s.P[0] + M[3] * s.P[2];
+                        double p3 = M[2] * s.P[1] + M[3] * s.P[3];
+                        s.P[0] = p0; s.P[1] = p1; s.P[2] = p2; s.P[3] = p3;
+                    }
+                    s.jl += st; k.bla++;
                 }
-                s.jl += st; k.bla++;
-            }
+                pin(stage);
+            } while (stage >= 0);
         }
         s.n += 1;
         // the step's table reads first, its tests together (as in HoloStd)
@@ -877,35 +900,40 @@ struct BsXr {
         const Tables &t = a.t;
         if (t.bla_on && (s.w & 7) == 0) {
             k.looks++;
-            int32_t idx, st;
-            while ((st = bla_lookup(t, s.xs, s.ys, s.w, idx)) != 0) {
-                // A z + B c and A J on shared exponents; the coefficients are
-                // split into mantissas on one exponent each (they reach the
-                // ends of the binary64 range)
-                double M[8];
-                for (int q = 0; q < 8; q++) M[q] = t.M[8 * idx + q];
-                s.n += st; s.w += st;
-                renorm(s, a);
-                int32_t eA = 0, eB = 0;
-                norm4(M, eA);
-                norm4(M + 4, eB);
-                double x = s.x, y = s.y;
-                int32_t e = s.e + eA, sc = s.ec + eB - e;
-                if (sc > FAR) { x = ldexp(x, -sc); y = ldexp(y, -sc); e += sc; sc = 0; }
-                s.x = M[0] * x + M[1] * y + ldexp(M[4] * s.a, sc) + ldexp(M[5] * s.b, sc);
-                s.y = M[2] * x + M[3] * y + ldexp(M[6] * s.a, sc) + ldexp(M[7] * s.b, sc);
-                s.e = e;
-                s.xs = ldexp(s.x, e); s.ys = ldexp(s.y, e);
-                if (DC_ON(a)) {
-                    const double P0 = s.P[0], P1 = s.P[1], P2 = s.P[2], P3 = s.P[3];
-                    s.P[0] = M[0] * P0 + M[1] * P2;
-                    s.P[1] = M[0] * P1 + M[1] * P3;
-                    s.P[2] = M[2] * P0 + M[3] * P2;
-                    s.P[3] = M[2] * P1 + M[3] * P3;
-                    s.eP += eA;
+            int32_t stage, idx;
+            do {
+                stage = bla_lookup(t, s.xs, s.ys, s.w, idx);
+                if (stage >= 0) {
+                    const int32_t st = 8 << stage;
+                    // A z + B c and A J on shared exponents; the coefficients are
+                    // split into mantissas on one exponent each (they reach the
+                    // ends of the binary64 range)
+                    double M[8];
+                    for (int q = 0; q < 8; q++) M[q] = t.M[8 * idx + q];
+                    s.n += st; s.w += st;
+                    renorm(s, a);
+                    int32_t eA = 0, eB = 0;
+                    norm4(M, eA);
+                    norm4(M + 4, eB);
+                    double x = s.x, y = s.y;
+                    int32_t e = s.e + eA, sc = s.ec + eB - e;
+                    if (sc > FAR) { x = ldexp(x, -sc); y = ldexp(y, -sc); e += sc; sc = 0; }
+                    s.x = M[0] * x + M[1] * y + ldexp(M[4] * s.a, sc) + ldexp(M[5] * s.b, sc);
+                    s.y = M[2] * x + M[3] * y + ldexp(M[6] * s.a, sc) + ldexp(M[7] * s.b, sc);
+                    s.e = e;
+                    s.xs = ldexp(s.x, e); s.ys = ldexp(s.y, e);
+                    if (DC_ON(a)) {
+                        const double P0 = s.P[0], P1 = s.P[1], P2 = s.P[2], P3 = s.P[3];
+                        s.P[0] = M[0] * P0 + M[1] * P2;
+                        s.P[1] = M[0] * P1 + M[1] * P3;
+                        s.P[2] = M[2] * P0 + M[3] * P2;
+                        s.P[3] = M[2] * P1 + M[3] * P3;
+                        s.eP += eA;
+                    }
+                    s.jl += st; k.bla++;
                 }
-                s.jl += st; k.bla++;
-            }
+                pin(stage);
+            } while (stage >= 0);
         }
         s.n += 1;
         // the step's table reads first, its tests together (as in HoloStd)

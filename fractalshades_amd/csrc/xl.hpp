@@ -42,13 +42,6 @@ FSG_DEV double amax(double x, double y) {
     return r;
 }
 
-// v as it is, for the compiler a new value: it neither rewrites what follows
-// in terms of what v was made from nor turns a branch around it into selects
-FSG_DEV void pin(int32_t &v) { asm("" : "+v"(v)); }
-// the same, not before x and y are known: a load at index v then takes the
-// registers that x and y were made from instead of copying into them later
-FSG_DEV void pin_after(int32_t &v, double x, double y) { asm("" : "+v"(v) : "v"(x), "v"(y)); }
-
 // normalised: larger component in [1, 2), or (0, 0, XL_ZERO_E)
 FSG_DEV xl xl_n(double re, double im, int32_t e) {
     const double mx = amax(re, im);
