@@ -125,6 +125,7 @@ hipError_t launch_tile(const LaunchCfg &cfg, const KArgs &a, hipStream_t stream)
 // (fsg_lds.hip, blocks of up to 1024 lanes)
 typedef void (*tile_fn)(const KArgs);
 tile_fn select_tile_orbit(const LaunchCfg &cfg);
+tile_fn select_tile_orbit_lds(const LaunchCfg &cfg, bool full, int der);
 // der: the derivatives the launch computes (bit 0 dz/dc, bit 1 dz/dz)
 tile_fn select_tile_lds(const LaunchCfg &cfg, bool full, int der);
 // true when the plan stages every table the launch reads

@@ -337,7 +337,7 @@ hipError_t launch_tile(const LaunchCfg &cfg, const KArgs &a, hipStream_t stream)
     // FSG_TABLES=global keeps the tables in global memory (for comparisons)
     const char *tables = std::getenv("FSG_TABLES");
     const bool no_lds = tables && !std::strcmp(tables, "global");
-    if (!cfg.orbit && !no_lds) {
+    if (!no_lds) {
         KArgs al = a;
         al.lds = plan_lds(a.t, cfg.kind == KIND_BS ? 8 : 4, max_lds_bytes());
         const int der = (a.calc_dc ? 1 : 0) | (a.calc_dz ? 2 : 0);

@@ -32,6 +32,7 @@ template <int D> struct MnModels {
 };
 
 tile_fn select_tile_lds(const LaunchCfg &c, bool full, int der) {
+    if (c.orbit) return select_tile_orbit_lds(c, full, der);
     if (c.kind == KIND_M2) return c.xr ? fn_lds_der<M2Xr>(full, der) : fn_lds_der<M2Std>(full, der);
     if (c.kind == KIND_MN) {
         switch (c.degree) {

@@ -18,18 +18,25 @@ namespace fsg {
 
 // calc_orbit recorder: the last two full orbit points (Z + z), taken at the
 // escape test of plain steps when n reaches the next multiple of backshift
-// (perturbation.py:1266-1273; n // backshift > div_shift is n >= next).
+// (perturbation.py:1266-1273; n // backshift > div_shift is n >= next).  A
+// step at which nothing is due passes the recorder by with the stop tests; the
+// division is for a jump over several multiples.
 template <bool ORB> struct OrbitRec {
     __device__ void reset(int32_t) {}
+    __device__ bool due(int32_t) const { return false; }
     __device__ void record(int32_t, int32_t, double, double) {}
 };
 template <> struct OrbitRec<true> {
     int32_t next, i1, i2;
     double x1, y1, x2, y2;
     __device__ void reset(int32_t b) { next = b; i1 = 0; i2 = 0; x1 = y1 = x2 = y2 = 0.; }
+    __device__ bool due(int32_t n) const { return n >= next; }
     __device__ void record(int32_t n, int32_t b, double x, double y) {
         if (n >= next) {
-            next = (n / b + 1) * b;
+            int32_t over = n - next;
+            pin(over);
+            next += b;
+            if (over >= b) { pin(over); next = (n / b + 1) * b; }
             i2 = i1; x2 = x1; y2 = y1;
             i1 = n; x1 = x; y1 = y;
         }
@@ -214,8 +221,8 @@ struct HoloStd {
         // The stop and rebase tests are evaluated together: a step that meets
         // none of them (nearly every step) leaves by one branch, and the
         // tests' own order (max_iter, interior, escape, rebase) is kept on
-        // the other path.  (The orbit recorder runs between the tests: its
-        // kernels take that path on every step.)  The first branch takes the
+        // the other path.  (The orbit recorder runs between the tests: a
+        // step with a point to record takes that path.)  The first branch takes the
         // interior and escape tests by filters that let every step pass that
         // meets them, one component against a bound, and the other path the
         // tests themselves: nine vector instructions less a step
@@ -224,19 +231,17 @@ struct HoloStd {
         bool t_int = false;
         if (DZ_ON(a)) t_int = fabs(s.h.re + H1.re) < a.eps_hi;
         const cplx ZZ = s.z + Z1;
-        const bool t_esc = ORB ? ZZ.re * ZZ.re + ZZ.im * ZZ.im > a.M2 : amax(ZZ.re, ZZ.im) > a.esc_lo;
+        const bool t_esc = amax(ZZ.re, ZZ.im) > a.esc_lo;
         const bool reb_div = s.w >= t.div_iter - 1;
         const bool dyn = (fabs(ZZ.re) <= fabs(s.z.re)) && (fabs(ZZ.im) <= fabs(s.z.im));
-        if constexpr (!ORB) {
-            if (!(s.n >= a.max_iter || t_int || t_esc || reb_div || dyn)) { s.dyn = false; return false; }
-        }
+        if (!(s.n >= a.max_iter || t_int || t_esc || reb_div || dyn || s.orb.due(s.n))) { s.dyn = false; return false; }
         if (s.n >= a.max_iter) { reason = 0; return true; }
         if (t_int) {
             const cplx q = s.h + H1;
             if (q.re * q.re + q.im * q.im < a.eps2) { reason = 2; return true; }
         }
         s.orb.record(s.n, a.backshift, ZZ.re, ZZ.im);
-        if (t_esc && (ORB || ZZ.re * ZZ.re + ZZ.im * ZZ.im > a.M2)) { reason = 1; return true; }
+        if (t_esc && ZZ.re * ZZ.re + ZZ.im * ZZ.im > a.M2) { reason = 1; return true; }
         bool reb = reb_div;
         if (!reb) {
             s.dyn = dyn;
@@ -580,12 +585,10 @@ struct HoloXr {
             t_int = fabs(qre) < a.eps_hi;
         }
         const cplx ZZ = s.zs + Z1;
-        const bool t_esc = ORB ? ZZ.re * ZZ.re + ZZ.im * ZZ.im > a.M2 : amax(ZZ.re, ZZ.im) > a.esc_lo;
+        const bool t_esc = amax(ZZ.re, ZZ.im) > a.esc_lo;
         const bool dyn = (fabs(ZZ.re) <= fabs(s.zs.re)) && (fabs(ZZ.im) <= fabs(s.zs.im));
         if constexpr (KIND == KIND_M2) { s.Z = Z1; s.kz = k1; s.A = ZZ; s.Zh = H1; }
-        if constexpr (!ORB) {
-            if (!(s.n >= a.max_iter || t_int || t_esc || edge || dyn)) { s.dyn = false; return false; }
-        }
+        if (!(s.n >= a.max_iter || t_int || t_esc || edge || dyn || s.orb.due(s.n))) { s.dyn = false; return false; }
         const auto stop = [&](int r) { s.d.e = rel(s.d.e, trip + 1); reason = r; return true; };
         if (s.n >= a.max_iter) return stop(0);
         if (t_int) {
@@ -593,7 +596,7 @@ struct HoloXr {
             if (qre * qre + qim * qim < a.eps2) return stop(2);
         }
         s.orb.record(s.n, a.backshift, ZZ.re, ZZ.im);
-        if (t_esc && (ORB || ZZ.re * ZZ.re + ZZ.im * ZZ.im > a.M2)) return stop(1);
+        if (t_esc && ZZ.re * ZZ.re + ZZ.im * ZZ.im > a.M2) return stop(1);
         // both rebases (perturbation.py:1283-1372) share the derivative
         // updates: one block, whichever of them a lane takes
         const bool reb_div = s.w >= t.div_iter - 1;
@@ -696,16 +699,14 @@ struct BsStd {
         }
         bs_zn<FL>(s.x, s.y, R.re, R.im, s.a, s.b);
         const double XX = s.x + R1.re, YY = s.y + R1.im;
-        const bool t_esc = ORB ? XX * XX + YY * YY > a.M2 : amax(XX, YY) > a.esc_lo;
+        const bool t_esc = amax(XX, YY) > a.esc_lo;
         const bool reb_div = w1 >= t.div_iter - 1;
         const bool dyn = (fabs(XX) <= fabs(s.x)) && (fabs(YY) <= fabs(s.y));
-        if constexpr (!ORB) {
-            if (!(s.n >= a.max_iter || t_esc || reb_div || dyn)) { s.w = w1; s.dyn = false; return false; }
-        }
+        if (!(s.n >= a.max_iter || t_esc || reb_div || dyn || s.orb.due(s.n))) { s.w = w1; s.dyn = false; return false; }
         if (s.n >= a.max_iter) { reason = 0; return true; }
         s.w = w1;
         s.orb.record(s.n, a.backshift, XX, YY);
-        if (t_esc && (ORB || XX * XX + YY * YY > a.M2)) { reason = 1; return true; }
+        if (t_esc && XX * XX + YY * YY > a.M2) { reason = 1; return true; }
         bool reb = reb_div;
         if (!reb) {
             s.dyn = dyn;
@@ -965,16 +966,14 @@ struct BsXr {
         }
         s.xs = ldexp(s.x, s.e); s.ys = ldexp(s.y, s.e);
         const double XX = s.xs + R1.re, YY = s.ys + R1.im;
-        const bool t_esc = ORB ? XX * XX + YY * YY > a.M2 : amax(XX, YY) > a.esc_lo;
+        const bool t_esc = amax(XX, YY) > a.esc_lo;
         const bool reb_div = w1 >= t.div_iter - 1;
         const bool dyn = (fabs(XX) <= fabs(s.xs)) && (fabs(YY) <= fabs(s.ys));
-        if constexpr (!ORB) {
-            if (!(s.n >= a.max_iter || t_esc || reb_div || dyn)) { s.w = w1; s.dyn = false; return false; }
-        }
+        if (!(s.n >= a.max_iter || t_esc || reb_div || dyn || s.orb.due(s.n))) { s.w = w1; s.dyn = false; return false; }
         if (s.n >= a.max_iter) { reason = 0; return true; }
         s.w = w1;
         s.orb.record(s.n, a.backshift, XX, YY);
-        if (t_esc && (ORB || XX * XX + YY * YY > a.M2)) { reason = 1; return true; }
+        if (t_esc && XX * XX + YY * YY > a.M2) { reason = 1; return true; }
         bool reb = reb_div;
         xlf x = xlf_of(s.x, s.e), y = xlf_of(s.y, s.e);
         if (reb_div) {
