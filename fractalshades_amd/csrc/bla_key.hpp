@@ -51,6 +51,10 @@ FSG_HD int64_t modulus_key(double q, int32_t e) {
 // key of |x + iy| for binary64 x, y, deciding as hypot2(x, y) < r does
 FSG_HD int64_t hypot_key(double x, double y) {
     const double mx = fmax(fabs(x), fabs(y));
+    // The prescale by a power of two is exact and leaves the key as it is: not
+    // needed while the larger square's last place lies above the subnormal
+    // range (a smaller square that is subnormal is then below half of it).
+    if (mx >= 0x1p-480 && mx <= 0x1p500) return (int64_t)bits(x * x + y * y);
     if (!(mx >= 0x1p-900 && mx <= 0x1p500)) {            // zero, tiny, huge or NaN
         const double h = hypot2(x, y);
         return h == h ? radius_key(h) : INT64_MAX;

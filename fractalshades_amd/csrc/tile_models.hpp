@@ -162,7 +162,8 @@ template <int KIND, int DEG, bool ORB = false, int DER = -1>
 struct HoloStd {
     __device__ static bool DC_ON(const KArgs &a) { if constexpr (DER >= 0) return (DER & 1) != 0; else return a.calc_dc != 0; }
     __device__ static bool DZ_ON(const KArgs &a) { if constexpr (DER >= 0) return (DER & 2) != 0; else return a.calc_dz != 0; }
-    struct State { cplx z, d, h, c; int32_t w, n, jl; bool dyn, nul; OrbitRec<ORB> orb; };
+    // Z, A, Zh: as in HoloXr, for z^2 + c
+    struct State { cplx z, d, h, c, Z, A, Zh; int32_t w, n, jl; bool dyn, nul; OrbitRec<ORB> orb; };
 
     __device__ static void init(State &s, const KArgs &a, double px, double py) {
         s.c = to_std(c_from_pix(a, px, py));
@@ -173,10 +174,10 @@ struct HoloStd {
 
     __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason) {
         const Tables &t = a.t;
-        if (t.bla_on && (s.w & 7) == 0) {
-            k.looks++;
-            int32_t stage, idx;
-            do {
+        if ((KIND == KIND_M2 || t.bla_on) && (s.w & 7) == 0) {
+            int32_t stage = -1, idx;
+            if (t.bla_on) k.looks++;
+            if (t.bla_on) do {
                 stage = bla_lookup(t, s.z.re, s.z.im, s.w, idx);
                 if (stage >= 0) {
                     const int32_t st = 8 << stage;
@@ -191,31 +192,55 @@ struct HoloStd {
                 }
                 pin(stage);
             } while (stage >= 0);
+            if constexpr (KIND == KIND_M2) {
+                s.Z = t.Zn[s.w];
+                if (DZ_ON(a)) s.Zh = t.dz[s.nul ? 0 : s.w];
+                s.A = s.Z + s.z;
+            }
         }
         s.n += 1;
-        // Every table value the step reads is loaded here, before any of it
-        // is used: the orbit point and path values at w, the next orbit point
+        // z^d + c: every table value the step reads is loaded here, before any of
+        // it is used: the orbit point and path values at w, the next orbit point
         // (escape and rebase tests) and the dZndz value of the interior test,
         // whose indexes are known at the start of the step.  A pixel whose
         // wave has no other work left (the last, longest pixels of a launch)
         // then waits for one table round trip per step instead of one per
-        // test.
-        const int32_t w1 = (s.w + 1 >= t.order) ? 0 : s.w + 1;
-        const cplx Zr = t.Zn[s.w];
-        const cplx Z1 = t.Zn[w1];
-        cplx Zd = zc(), Zh = zc(), H1 = zc();
-        if (DC_ON(a)) { const cplx v = t.dc[s.w]; Zd = s.dyn ? zc() : v; }
-        if (DZ_ON(a)) {
-            Zh = t.dz[s.nul ? 0 : s.w];
-            H1 = t.dz[s.nul ? 0 : (s.n == t.order ? t.L : w1)];
+        // test.  z^2 + c carries half of them and loads the others where the
+        // registers of the old ones are free (HoloXr).  512x512 at 1e-40: 43.9
+        // -> 41.4 us.
+        int32_t w1 = s.w + 1, wh = w1;                   // wh: index of the interior test's dZndz value
+        const bool edge = w1 >= min(t.order, t.div_iter - 1);
+        if (edge) {
+            pin(w1);
+            if (w1 >= t.order) { w1 = 0; wh = s.n == t.order ? t.L : 0; }
+        }
+        if (DZ_ON(a) && s.nul) wh = 0;
+        cplx Z1, Zd = zc(), H1 = zc();
+        if (DC_ON(a)) Zd = t.dc[s.w];
+        if (s.dyn) {
+            pin(w1);
+            Zd = zc();
         }
         if constexpr (KIND == KIND_MN) {
+            const cplx Zr = t.Zn[s.w];
+            Z1 = t.Zn[w1];
+            cplx Zh = zc();
+            if (DZ_ON(a)) { Zh = t.dz[s.nul ? 0 : s.w]; H1 = t.dz[wh]; }
             s.z = mn_step<DEG>(s.z, Zr, s.c, DC_ON(a), DZ_ON(a), s.d, s.h, s.d, s.h, Zd, Zh,
                                [](cplx u, cplx v) { return u + v; });
         } else {
-            if (DC_ON(a)) s.d = p_deriv<KIND, DEG>(s.z, s.d, Zr, Zd);
-            if (DZ_ON(a)) s.h = p_deriv<KIND, DEG>(s.z, s.h, Zr, Zh);
-            s.z = p_zn<KIND, DEG>(s.z, Zr, s.c);
+            // mandelbrot_M2.py:607-622: z (z + 2 Z) + c, 2 ((Z + z) d + Zd z)
+            const cplx W = mk(__builtin_fma(2., s.Z.re, s.z.re), __builtin_fma(2., s.Z.im, s.z.im));
+            pin_after(w1, W.re, W.im);
+            Z1 = t.Zn[w1];
+            if (DC_ON(a)) s.d = muls(2., s.A * s.d + Zd * s.z);
+            if (DZ_ON(a)) {
+                const cplx v = s.Zh * s.z;
+                pin_after(wh, v.re, v.im);
+                H1 = t.dz[wh];
+                s.h = muls(2., s.A * s.h + v);
+            }
+            s.z = s.z * W + s.c;
         }
         s.w = w1;
         // The stop and rebase tests are evaluated together: a step that meets
@@ -232,9 +257,9 @@ struct HoloStd {
         if (DZ_ON(a)) t_int = fabs(s.h.re + H1.re) < a.eps_hi;
         const cplx ZZ = s.z + Z1;
         const bool t_esc = amax(ZZ.re, ZZ.im) > a.esc_lo;
-        const bool reb_div = s.w >= t.div_iter - 1;
         const bool dyn = (fabs(ZZ.re) <= fabs(s.z.re)) && (fabs(ZZ.im) <= fabs(s.z.im));
-        if (!(s.n >= a.max_iter || t_int || t_esc || reb_div || dyn || s.orb.due(s.n))) { s.dyn = false; return false; }
+        if constexpr (KIND == KIND_M2) { s.Z = Z1; s.A = ZZ; s.Zh = H1; }
+        if (!(s.n >= a.max_iter || t_int || t_esc || edge || dyn || s.orb.due(s.n))) { s.dyn = false; return false; }
         if (s.n >= a.max_iter) { reason = 0; return true; }
         if (t_int) {
             const cplx q = s.h + H1;
@@ -242,7 +267,7 @@ struct HoloStd {
         }
         s.orb.record(s.n, a.backshift, ZZ.re, ZZ.im);
         if (t_esc && ZZ.re * ZZ.re + ZZ.im * ZZ.im > a.M2) { reason = 1; return true; }
-        bool reb = reb_div;
+        bool reb = s.w >= t.div_iter - 1;
         if (!reb) {
             s.dyn = dyn;
             reb = dyn;
