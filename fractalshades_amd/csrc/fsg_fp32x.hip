@@ -29,10 +29,9 @@ constexpr int32_t XS_ZERO_E = -(1 << 28);   // exponent of 0: aligns to nothing
 __device__ __forceinline__ int32_t fexp(float v) { return __builtin_amdgcn_frexp_expf(v); }
 
 __device__ __forceinline__ xs xs_norm(float x, float y, int32_t e) {
-    float mx = fmaxf(fabsf(x), fabsf(y));
-    if (mx == 0.f) return xs{0.f, 0.f, XS_ZERO_E};
-    int32_t k = fexp(mx) - 1;                  // mx in [2^k, 2^(k+1))
-    return xs{ldexpf(x, -k), ldexpf(y, -k), e + k};
+    const float mx = fmaxf(fabsf(x), fabsf(y));
+    const int32_t k = fexp(mx) - 1;            // mx in [2^k, 2^(k+1))
+    return xs{ldexpf(x, -k), ldexpf(y, -k), mx == 0.f ? XS_ZERO_E : e + k};
 }
 
 __device__ __forceinline__ xs operator+(xs a, xs b) {
@@ -195,36 +194,53 @@ constexpr int32_t FP32X_STEP_CAP = 1 << 16;
 // within eb, so the binary64 loop takes the same stage unless a radius lies
 // within eb of |z|; only the accepted stage's radius and the next stage's
 // can (the radii do not grow with the stage for one start).
+// Returns the stage less 3, -1 if no stage is valid; idx as bla_find.  The
+// lowest stage first, then on a half-open interval, as there.
 __device__ __forceinline__ int32_t bla_find_m(const Tables &t, double az, double eb, int32_t w,
                                               int32_t &idx, bool &unsure) {
-    const int32_t it = w >> 3;
     const int32_t invalid_step = t.first_invalid - w;
-    if (invalid_step <= 8) return 0;
-    const int32_t tz = (it == 0) ? 31 : __builtin_ctz((uint32_t)it);
-    const int32_t s_inv = 31 - __builtin_clz((uint32_t)(invalid_step - 1));
-    const int32_t cap = min(min(3 + tz, t.stages_bla - 1), s_inv);
-    int32_t hi = cap, lo = 3, best = 0;
-    double rb = 0.;
-    while (lo <= hi) {
-        const int32_t mid = (lo + hi) >> 1;
-        const double r = t.r[2 * it + (1 << (mid - 3)) - 1];
-        if (az < r) { best = mid; rb = r; lo = mid + 1; }
-        else hi = mid - 1;
+    int32_t stage = -1;
+    if (invalid_step > 8 && t.stages_bla > 3) {
+        const double *r = t.r + (w >> 2);            // r[2^s - 1]: stage s + 3
+        const double r0 = r[0];
+        if (!(az < r0)) {
+            unsure = az - r0 < eb;
+        } else {
+            const int32_t starts = __builtin_ctz((uint32_t)w | 0x80000000u);
+            const int32_t fits = 31 - __builtin_clz((uint32_t)(invalid_step - 1));
+            const int32_t end = min(min(starts, t.stages_bla - 1), fits) - 2;
+            int32_t hi = end;                        // stage valid, hi not
+            stage = 0;
+            while (hi - stage > 1) {
+                const int32_t mid = (stage + hi) >> 1;
+                if (az < r[(1 << mid) - 1]) stage = mid;
+                else hi = mid;
+            }
+            unsure = r[(1 << stage) - 1] - az <= eb;
+            if (hi < end && az - r[(1 << hi) - 1] < eb) unsure = true;
+        }
     }
-    if (best > 0 && rb - az <= eb) unsure = true;
-    const int32_t nxt = best > 0 ? best + 1 : 3;
-    if (nxt <= cap && az - t.r[2 * it + (1 << (nxt - 3)) - 1] < eb) unsure = true;
-    if (best == 0) return 0;
-    idx = 2 * it + (1 << (best - 3)) - 1;
-    return 1 << best;
+    pin(stage);
+    idx = (w >> 2) + (1 << stage) - 1;
+    return stage;
+}
+
+// Record i of a table, by 12 i = (3 i) 4: two shifts and adds, where the
+// compiler's multiplication by 12 issues over four instructions' time.
+__device__ __forceinline__ int32_t times3(int32_t i) { int32_t k = i + 2 * i; pin(k); return k; }
+__device__ __forceinline__ xs at3(const xs *p, int32_t i3) {
+    return *reinterpret_cast<const xs *>(reinterpret_cast<const float *>(p) + i3);
 }
 
 __device__ __forceinline__ float l1(float x, float y) { return fabsf(x) + fabsf(y); }
 __device__ __forceinline__ float l2(float x, float y) { return __builtin_sqrtf(x * x + y * y); }
 
-template <int KIND, int DEG>
+// DER as in HoloXr.
+template <int KIND, int DEG, int DER = -1>
 struct HoloS32 {
-    struct State { xs z, c, d, h; float cx, cy, e2; int32_t w, n, jl, steps; bool dyn, nul; };
+    __device__ static bool DC_ON(const KArgs &a) { if constexpr (DER >= 0) return (DER & 1) != 0; else return a.calc_dc != 0; }
+    __device__ static bool DZ_ON(const KArgs &a) { if constexpr (DER >= 0) return (DER & 2) != 0; else return a.calc_dz != 0; }
+    struct State { xs z, c, d, h; float cx, cy, e2; int32_t w, n, jl; bool dyn, nul; };
 
     // c in z's scale, after z's exponent moved
     __device__ static void sync_c(State &s) {
@@ -238,10 +254,10 @@ struct HoloS32 {
         s.e2 = ldexpf(s.e2, -2 * k);
         sync_c(s);
     }
-    __device__ static void renorm(State &s) {
+    __device__ static void renorm(State &s, const KArgs &a) {
         renorm_z(s);
-        s.d = xs_norm(s.d.x, s.d.y, s.d.e);
-        s.h = xs_norm(s.h.x, s.h.y, s.h.e);
+        if (DC_ON(a)) s.d = xs_norm(s.d.x, s.d.y, s.d.e);
+        if (DZ_ON(a)) s.h = xs_norm(s.h.x, s.h.y, s.h.e);
     }
     // a scaled value as a lazily normalised record (a zero mantissa takes
     // the zero exponent, so that it never sets the exponent of a sum)
@@ -275,7 +291,7 @@ struct HoloS32 {
         s.d = xs_zero(); s.h = xs_zero();
         s.e2 = 0.f;
         sync_c(s);
-        s.w = 0; s.n = 0; s.jl = 0; s.steps = 0; s.dyn = true; s.nul = false;
+        s.w = 0; s.n = 0; s.jl = 0; s.dyn = true; s.nul = false;
     }
 
     // one plain step on mantissas: the orbit point Zf (absolute, binary32),
@@ -287,7 +303,7 @@ struct HoloS32 {
         if constexpr (KIND == KIND_M2) {
             fp1 = 4.f * (sx * sx + sy * sy);                                  // |f'|^2
             // 2 ((Z + z) d + Zd z): both terms on the larger exponent
-            if (a.calc_dc) {
+            if (DC_ON(a)) {
                 const int32_t E = max(s.d.e, Zd.e + s.z.e);
                 const float k1 = ldexpf(1.f, max(s.d.e - E, -200)), k2 = ldexpf(1.f, max(Zd.e + s.z.e - E, -200));
                 const float ax = k1 * s.d.x, ay = k1 * s.d.y, bx = k2 * Zd.x, by = k2 * Zd.y;
@@ -295,7 +311,7 @@ struct HoloS32 {
                 s.d.y = ax * sy + ay * sx + (bx * s.z.y + by * s.z.x);
                 s.d.e = E + 1;
             }
-            if (a.calc_dz) {
+            if (DZ_ON(a)) {
                 const int32_t E = max(s.h.e, Zh.e + s.z.e);
                 const float k1 = ldexpf(1.f, max(s.h.e - E, -200)), k2 = ldexpf(1.f, max(Zh.e + s.z.e - E, -200));
                 const float ax = k1 * s.h.x, ay = k1 * s.h.y, bx = k2 * Zh.x, by = k2 * Zh.y;
@@ -332,8 +348,8 @@ struct HoloS32 {
             for (int q = 1; q < DEG; q++) { g *= ls; gt *= lt; }
             fp1 = (float)DEG * g;
             fp1 *= fp1;
-            if (a.calc_dc) s.d = dstep(s, Zd, s.d, ux, uy, Zfx, Zfy);
-            if (a.calc_dz) s.h = dstep(s, Zh, s.h, ux, uy, Zfx, Zfy);
+            if (DC_ON(a)) s.d = dstep(s, Zd, s.d, ux, uy, Zfx, Zfy);
+            if (DZ_ON(a)) s.h = dstep(s, Zh, s.h, ux, uy, Zfx, Zfy);
             const float fr = KE * ((float)(DEG * DEG) * gt * l1(s.z.x, s.z.y) + l1(s.cx, s.cy));
             s.e2 = fp1 * s.e2 + fr * fr;
             s.z.x = tx + s.cx; s.z.y = ty + s.cy;
@@ -372,61 +388,76 @@ struct HoloS32 {
         return xs{ex, ey, T};
     }
 
-    __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason) {
-        reason = step_reason(s, a, k);
-        return reason >= 0;
-    }
-    // the stop reason, -1: not stopped
-    __device__ static int step_reason(State &s, const KArgs &a, Counters &k) {
+    __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason, int32_t trip) {
         const Tables &t = a.t;
         const xs *Zx = (const xs *)a.tx.Zx, *DC = (const xs *)a.tx.DCx, *DZ = (const xs *)a.tx.DZx;
-        if (++s.steps > FP32X_STEP_CAP) return REASON_UNSURE;
+        if (trip >= FP32X_STEP_CAP) { reason = REASON_UNSURE; return true; }
         if ((s.w & 7) == 0) {
-            renorm(s);
+            renorm(s, a);
+            int32_t go = t.bla_on ? 0 : -1;
             k.looks += t.bla_on != 0;
-            while (t.bla_on) {
+            while (go >= 0) {
                 const double az = ldexp((double)hypotf(s.z.x, s.z.y), max(s.z.e, -2000));
                 const double eb = err_abs(s) + 0x1p-21 * az;
                 int32_t idx;
                 bool unsure = false;
-                const int32_t st = bla_find_m(t, az, eb, s.w, idx, unsure);
-                if (unsure) return REASON_UNSURE;
-                if (st == 0) break;
-                // z <- A z + B c, d <- A d, h <- A h (A, B normalised records)
-                const xs A = ((const xs *)a.tx.Ax)[idx], B = ((const xs *)a.tx.Bx)[idx];
-                const int32_t E = max(A.e, B.e);
-                const float ka = ldexpf(1.f, max(A.e - E, -200)), kb = ldexpf(1.f, max(B.e - E, -200));
-                const float Ax = ka * A.x, Ay = ka * A.y, Bx = kb * B.x, By = kb * B.y;
-                const float nx = Ax * s.z.x - Ay * s.z.y + (Bx * s.cx - By * s.cy);
-                const float ny = Ax * s.z.y + Ay * s.z.x + (Bx * s.cy + By * s.cx);
-                const float fr = KE * (l1(Ax, Ay) * l1(s.z.x, s.z.y) + l1(Bx, By) * l1(s.cx, s.cy));
-                s.e2 = (Ax * Ax + Ay * Ay) * s.e2 + fr * fr;
-                s.z.x = nx; s.z.y = ny; s.z.e += E;
-                if (a.calc_dc) { float x, y; cmul(A.x, A.y, s.d.x, s.d.y, x, y); s.d = xs{x, y, s.d.e + A.e}; }
-                if (a.calc_dz) { float x, y; cmul(A.x, A.y, s.h.x, s.h.y, x, y); s.h = xs{x, y, s.h.e + A.e}; }
-                s.n += st;
-                s.w += st;                      // w + st < first_invalid <= order
-                renorm(s);
-                s.jl += st; k.bla++;
+                const int32_t stage = bla_find_m(t, az, eb, s.w, idx, unsure);
+                go = unsure ? -2 : stage;
+                if (go >= 0) {
+                    const int32_t st = 8 << stage;
+                    // z <- A z + B c, d <- A d, h <- A h (A, B normalised records)
+                    const int32_t i3 = times3(idx);
+                    const xs A = at3((const xs *)a.tx.Ax, i3), B = at3((const xs *)a.tx.Bx, i3);
+                    const int32_t E = max(A.e, B.e);
+                    const float ka = ldexpf(1.f, max(A.e - E, -200)), kb = ldexpf(1.f, max(B.e - E, -200));
+                    const float Ax = ka * A.x, Ay = ka * A.y, Bx = kb * B.x, By = kb * B.y;
+                    const float nx = Ax * s.z.x - Ay * s.z.y + (Bx * s.cx - By * s.cy);
+                    const float ny = Ax * s.z.y + Ay * s.z.x + (Bx * s.cy + By * s.cx);
+                    const float fr = KE * (l1(Ax, Ay) * l1(s.z.x, s.z.y) + l1(Bx, By) * l1(s.cx, s.cy));
+                    s.e2 = (Ax * Ax + Ay * Ay) * s.e2 + fr * fr;
+                    s.z.x = nx; s.z.y = ny; s.z.e += E;
+                    if (DC_ON(a)) { float x, y; cmul(A.x, A.y, s.d.x, s.d.y, x, y); s.d = xs{x, y, s.d.e + A.e}; }
+                    if (DZ_ON(a)) { float x, y; cmul(A.x, A.y, s.h.x, s.h.y, x, y); s.h = xs{x, y, s.h.e + A.e}; }
+                    s.n += st;
+                    s.w += st;                      // w + st < first_invalid <= order
+                    renorm(s, a);
+                    s.jl += st; k.bla++;
+                }
+                pin(go);
             }
+            if (go == -2) { reason = REASON_UNSURE; return true; }
         }
         s.n += 1;
-        const xs Zr = Zx[s.w];
-        const xs Zd = (a.calc_dc && !s.dyn) ? DC[s.w] : xs_zero();
-        const xs Zh = a.calc_dz ? (s.nul ? DZ[0] : DZ[s.w]) : xs_zero();
+        int32_t w1 = s.w + 1, wh = w1;                   // wh: index of the interior test's dZndz value
+        const bool edge = w1 >= min(t.order, t.div_iter - 1);
+        if (edge) {
+            pin(w1);
+            if (w1 >= t.order) { w1 = 0; wh = s.n == t.order ? t.L : 0; }
+        }
+        if (DZ_ON(a) && s.nul) wh = 0;
+        const int32_t w3 = times3(s.w);
+        const xs Zr = at3(Zx, w3);
+        const cplx Zn1 = t.Zn[w1];
+        xs Zd = xs_zero(), Zh = xs_zero(), H1 = xs_zero();
+        if (DC_ON(a)) Zd = at3(DC, w3);
+        if (DZ_ON(a)) { Zh = at3(DZ, s.nul ? 0 : w3); H1 = at3(DZ, times3(wh)); }
+        if (s.dyn) {
+            pin(w1);
+            Zd = xs_zero();
+        }
         constexpr int32_t LOW = (KIND == KIND_M2) ? -60 : -100 / (DEG - 1);
         if (Zr.e >= LOW) {
             fast_step(s, a, ldexpf(Zr.x, Zr.e), ldexpf(Zr.y, Zr.e), Zd, Zh);
             if (l1(s.z.x, s.z.y) > RENORM_AT) renorm_z(s);
-            if (l1(s.d.x, s.d.y) > RENORM_AT) s.d = xs_norm(s.d.x, s.d.y, s.d.e);
-            if (l1(s.h.x, s.h.y) > RENORM_AT) s.h = xs_norm(s.h.x, s.h.y, s.h.e);
+            if (DC_ON(a) && l1(s.d.x, s.d.y) > RENORM_AT) s.d = xs_norm(s.d.x, s.d.y, s.d.e);
+            if (DZ_ON(a) && l1(s.h.x, s.h.y) > RENORM_AT) s.h = xs_norm(s.h.x, s.h.y, s.h.e);
         } else {
             // the orbit point is below binary32's comfortable range: one step
             // on lazily normalised records (products add exponents, sums align)
             const xt z0 = tz(s.z), Zt = as_t(Zr);
             const int32_t e0 = s.z.e;
-            if (a.calc_dc) s.d = of_t(p_deriv<KIND, DEG>(z0, tz(s.d), Zt, as_t(Zd)));
-            if (a.calc_dz) s.h = of_t(p_deriv<KIND, DEG>(z0, tz(s.h), Zt, as_t(Zh)));
+            if (DC_ON(a)) s.d = of_t(p_deriv<KIND, DEG>(z0, tz(s.d), Zt, as_t(Zd)));
+            if (DZ_ON(a)) s.h = of_t(p_deriv<KIND, DEG>(z0, tz(s.h), Zt, as_t(Zh)));
             const xs nz = of_t(p_zn<KIND, DEG>(z0, Zt, as_t(s.c)));
             // |f'(Z + z)| <= d (|Z| + |z|)^(d-1), the step's terms <= |z| (|z| + d |Z|)^(d-1):
             // magnitudes in units of 2^E, E the larger of |z|'s and |Z|'s exponents
@@ -446,19 +477,43 @@ struct HoloS32 {
             const float fr = KE * (l1(s.z.x, s.z.y) + l1(s.cx, s.cy));
             s.e2 = (float)(prop + fresh * fresh) + fr * fr;
         }
-        s.w += 1;
-        if (s.w >= t.order) s.w = 0;
+        s.w = w1;
+        // The tests, behind filters: a step whose error estimate is below
+        // |z| / 256 and that comes near no test's threshold leaves here (nearly
+        // every step), without the error bound's square root, the extended sum
+        // of the interior test and the comparisons' margins.  Escape: |Z + z|
+        // may reach M / 2 only if a component reaches esc_lo / 2.  Rebase: twice
+        // the error bound, 16 sqrt(e2) <= |z| / 16, is below a tenth of z's
+        // larger component.  Interior: |dz/dz| within the margin of eps has its
+        // real part there.
+        // 1279x719 at 1e-300 with interior detection, with the branch-free
+        // normalisation, the lookup of bla_find and the addresses above: the
+        // binary32 pass 317 -> 229 us, the frame 439 -> 354 us.
+        const cplx z64 = zd(s);
+        const cplx ZZ = z64 + Zn1;
+        const double mz = fmax(fabs(z64.re), fabs(z64.im));
+        const bool rough = !(s.e2 <= 0x1p-16f * (s.z.x * s.z.x + s.z.y * s.z.y));
+        const bool t_esc = !(fmax(fabs(ZZ.re), fabs(ZZ.im)) <= 0.5 * a.esc_lo && mz <= a.esc_lo);
+        const double mg = __builtin_fma(0.1, mz, 1e-290);       // (a subnormal z: decided by the tests)
+        const bool near = fabs(ZZ.re) <= fabs(z64.re) + mg && fabs(ZZ.im) <= fabs(z64.im) + mg;
+        bool t_int = false;
+        if (DZ_ON(a)) t_int = !(fabsf(ldexpf(s.h.x, s.h.e) + ldexpf(H1.x, H1.e)) >= fmaxf(1.01f * (float)a.eps_hi, 0x1p-100f));
+        if (!(s.n >= a.max_iter || edge || rough || t_esc || near || t_int)) { s.dyn = false; return false; }
+        reason = decide(s, a, k, Zx, DC, z64, ZZ, Zn1, H1);
+        return reason >= 0;
+    }
+    // the tests of a step themselves: the stop reason, -1 if it does not stop
+    __device__ static int decide(State &s, const KArgs &a, Counters &k, const xs *Zx, const xs *DC, cplx z64, cplx ZZ,
+                                 cplx Zn1, const xs &H1) {
+        const Tables &t = a.t;
         if (s.n >= a.max_iter) return 0;
-        if (a.calc_dz) {
-            const xs q = s.h + (s.nul ? DZ[0] : (s.n == t.order ? DZ[t.L] : DZ[s.w]));
+        if (DZ_ON(a)) {
+            const xs q = s.h + H1;
             const double q2 = ldexp(xs_abs2_m(q), 2 * max(q.e, -2000));
             if (fabs(q2 - a.eps2) <= INTERIOR_MARGIN * a.eps2) return REASON_UNSURE;
             if (q2 < a.eps2) return 2;
         }
         // escape and rebase tests in binary64, on the binary64 orbit
-        const cplx z64 = zd(s);
-        const cplx Zn1 = t.Zn[s.w];
-        const cplx ZZ = z64 + Zn1;
         const double eabs = err_abs(s);
         const double r2 = ZZ.re * ZZ.re + ZZ.im * ZZ.im;
         // an error as large as a quarter of the escape radius leaves no decision certain
@@ -469,42 +524,35 @@ struct HoloS32 {
             if (fabs(sqrt(r2) - m) <= eabs + 0x1p-50 * m) return REASON_UNSURE;
             if (r2 > a.M2) return 1;
         }
-        if (s.w >= t.div_iter - 1) {
+        bool reb = s.w >= t.div_iter - 1;
+        if (!reb) {
+            // dynamic rebase: |ZZ| <= |z| component-wise; uncertain when a
+            // component lies within twice the error bound of its threshold
+            // (a zero orbit point leaves ZZ = z in both loops: certain)
+            const double dre = fabs(ZZ.re) - fabs(z64.re), dim = fabs(ZZ.im) - fabs(z64.im);
+            const double mg = 2. * eabs;
+            const bool zero_ref = (Zn1.re == 0. && Zn1.im == 0.);
+            if (!zero_ref && dre <= mg && dim <= mg && !(dre < -mg && dim < -mg)) return REASON_UNSURE;
+            s.dyn = (dre <= 0.) && (dim <= 0.);
+            if (s.dyn) {
+                // the binary64 loop confirms with the extended-range |ZZ|^2 <= |z|^2,
+                // which can decide otherwise only where z or the orbit point
+                // underflows binary64: left to that loop
+                if (fabs(z64.re) + fabs(z64.im) < 1e-290 || (zero_ref && Zx[s.w].e != XS_ZERO_E))
+                    return REASON_UNSURE;
+                const xs ZZx = s.z + Zx[s.w];
+                reb = xs_abs2_le(ZZx, s.z);
+            }
+        }
+        if (reb) {
             set_z(s, ZZ.re, ZZ.im);
-            if (a.calc_dc) s.d = s.d + DC[s.w];
-            if (a.calc_dz) {
-                if (!s.nul) s.h = s.h + (s.n == t.order ? DZ[t.L] : DZ[s.w]);
+            if (DC_ON(a)) s.d = s.d + DC[s.w];
+            if (DZ_ON(a)) {
+                if (!s.nul) s.h = s.h + H1;       // dZndz at w (at L after a full period)
                 s.nul = true;
             }
             s.w = 0;
             k.reb++;
-            return -1;
-        }
-        // dynamic rebase: |ZZ| <= |z| component-wise; uncertain when a
-        // component lies within twice the error bound of its threshold
-        // (a zero orbit point leaves ZZ = z in both loops: certain)
-        const double dre = fabs(ZZ.re) - fabs(z64.re), dim = fabs(ZZ.im) - fabs(z64.im);
-        const double mg = 2. * eabs;
-        const bool zero_ref = (Zn1.re == 0. && Zn1.im == 0.);
-        if (!zero_ref && dre <= mg && dim <= mg && !(dre < -mg && dim < -mg)) return REASON_UNSURE;
-        s.dyn = (dre <= 0.) && (dim <= 0.);
-        if (s.dyn) {
-            // the binary64 loop confirms with the extended-range |ZZ|^2 <= |z|^2,
-            // which can decide otherwise only where z or the orbit point
-            // underflows binary64: left to that loop
-            if (fabs(z64.re) + fabs(z64.im) < 1e-290 || (zero_ref && Zx[s.w].e != XS_ZERO_E))
-                return REASON_UNSURE;
-            const xs ZZx = s.z + Zx[s.w];
-            if (xs_abs2_le(ZZx, s.z)) {
-                set_z(s, ZZ.re, ZZ.im);
-                if (a.calc_dc) s.d = s.d + DC[s.w];
-                if (a.calc_dz) {
-                    if (!s.nul) s.h = s.h + (s.n == t.order ? DZ[t.L] : DZ[s.w]);
-                    s.nul = true;
-                }
-                s.w = 0;
-                k.reb++;
-            }
         }
         return -1;
     }
@@ -516,12 +564,12 @@ struct HoloS32 {
         const cplx z = zd(s) + a.t.Zn[s.w];
         g.Z[2 * i] = z.re; g.Z[2 * i + 1] = z.im;
         int f = 1;
-        if (a.calc_dz) {
+        if (DZ_ON(a)) {
             const cplx h = xs_to_d(xs_norm(s.h.x, s.h.y, s.h.e));
             g.Z[2 * (n + i)] = h.re; g.Z[2 * (n + i) + 1] = h.im;
             f = 2;
         }
-        if (a.calc_dc) {
+        if (DC_ON(a)) {
             const cplx d = xs_to_d(xs_norm(s.d.x, s.d.y, s.d.e) + ((const xs *)a.tx.DCx)[s.w]);
             g.Z[2 * (f * n + i)] = d.re; g.Z[2 * (f * n + i) + 1] = d.im;
         }
@@ -686,7 +734,7 @@ struct BsF32 {
         s.w = 0; s.n = 0; s.jl = 0; s.dyn = true;
     }
 
-    __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason) {
+    __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason, int32_t) {
         reason = step_reason(s, a, k);
         return reason >= 0;
     }
@@ -913,8 +961,10 @@ template <class Model> static tile_fn fn_lds_x(bool full) {
     return full ? k_tile_lds_x<Model, true> : k_tile_lds_x<Model, false>;
 }
 
-static tile_fn select_f32_lds(const LaunchCfg &c, bool full) {
-    if (c.kind == KIND_M2) return fn_lds_x<HoloS32<KIND_M2, 2>>(full);
+// z^2 + c is compiled for the derivatives that frames use (dz/dc, both)
+static tile_fn select_f32_lds(const LaunchCfg &c, bool full, int der) {
+    if (c.kind == KIND_M2) return der == 1 ? fn_lds_x<HoloS32<KIND_M2, 2, 1>>(full)
+                                  : der == 3 ? fn_lds_x<HoloS32<KIND_M2, 2, 3>>(full) : fn_lds_x<HoloS32<KIND_M2, 2>>(full);
     if (c.kind == KIND_MN) {
         switch (c.degree) {
 #define FSG_MN(D) case D: return fn_lds_x<HoloS32<KIND_MN, D>>(full);
@@ -935,7 +985,7 @@ hipError_t launch_tile_f32(const LaunchCfg &cfg, const KArgs &a, hipStream_t str
         const bool bs = cfg.kind == KIND_BS;
         al.ldsx = bs ? plan_lds_bsx(a.t, max_lds_bytes()) : plan_lds_x(a.t, a.tx, max_lds_bytes());
         tile_fn fl = al.ldsx.bytes <= 0 ? nullptr
-                     : bs ? select_bsx_lds(cfg) : select_f32_lds(cfg, al.ldsx.full != 0);
+                     : bs ? select_bsx_lds(cfg) : select_f32_lds(cfg, al.ldsx.full != 0, (a.calc_dc ? 1 : 0) | (a.calc_dz ? 2 : 0));
         const int fill = fl ? fill_blocks(reinterpret_cast<const void *>(fl), 1024, al.ldsx.bytes) : -1;
         if (fill > 0) {
             const int block = tile_block(fill, al);

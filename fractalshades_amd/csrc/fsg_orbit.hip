@@ -30,10 +30,9 @@ tile_fn select_tile_orbit(const LaunchCfg &c) {
 
 // The same with the tables in LDS: z^2 + c compiled for the derivatives that
 // frames use (dz/dc, both), the others reading them from the launch arguments.
-// 1001x667 at 1e-150 with dz/dc: 126 us from global memory, every step through
-// the recorder, now 112 (1e-150) and 170 -> 135 at
-// 1e-300; the burning ship with extended range spills here and is faster all
-// the same (1e-800: 421 -> 379).
+// 1001x667 with dz/dc, from global memory with every step through the recorder
+// and now: 133 -> 119 us at 1e-150, 171 -> 135 at 1e-300; the burning ship with
+// extended range spills here and is faster all the same (1e-800: 421 -> 379).
 template <class Model> static tile_fn fn_lds(bool full) {
     return full ? k_tile_lds<Model, true> : k_tile_lds<Model, false>;
 }

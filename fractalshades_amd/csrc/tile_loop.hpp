@@ -310,15 +310,12 @@ __device__ __forceinline__ void tile_loop(const KArgs &a) {
         if (__lane_id() < filled) {
             Model::init(s, g, g.pix[2 * idx], g.pix[2 * idx + 1]);
             int reason;
-            if constexpr (is_lazy<Model>::value) {
-                // trips: uniform over the lanes still iterating, in a scalar register
-                unsigned trips = 0;
-                for (;; trips++) {
+            // trips: uniform over the lanes still iterating, in a scalar register
+            for (unsigned trips = 0;; trips++) {
+                if constexpr (is_lazy<Model>::value) {
                     if ((trips & renorm_mask) == renorm_mask) Model::renorm(s, a, (int32_t)trips);
-                    if (Model::step(s, a, k, reason, (int32_t)trips)) break;
                 }
-            } else {
-                while (!Model::step(s, a, k, reason)) {}
+                if (Model::step(s, a, k, reason, (int32_t)trips)) break;
             }
             k.plain += (unsigned)(s.n - s.jl);
             k.bla_it += (unsigned)s.jl;

@@ -172,7 +172,7 @@ struct HoloStd {
         s.orb.reset(a.backshift);
     }
 
-    __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason) {
+    __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason, int32_t) {
         const Tables &t = a.t;
         if ((KIND == KIND_M2 || t.bla_on) && (s.w & 7) == 0) {
             int32_t stage = -1, idx;
@@ -686,7 +686,7 @@ struct BsStd {
         s.orb.reset(a.backshift);
     }
 
-    __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason) {
+    __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason, int32_t) {
         const Tables &t = a.t;
         if (t.bla_on && (s.w & 7) == 0) {
             k.looks++;
