@@ -243,7 +243,76 @@ int stages_of(int64_t L) {
 
 }  // namespace
 
+// Pinned host buffers through which the results of host-buffer tiles come
+// back: one copy of everything instead of five copies to pageable memory, each
+// of which stages through the runtime's own pinned buffers and is waited for.
+// A call takes a buffer and gives it back (a user's contexts come and go with
+// the frames, pinning memory costs more than a tile), so concurrent calls never
+// share one.  At most KEEP buffers of at most MAX_BYTES are kept, none once the
+// last context is gone.
+namespace {
+class PinnedPool {
+public:
+    static constexpr size_t MAX_BYTES = 16u << 20, ROUND = 1u << 20;
+    struct Buf { char *p = nullptr; size_t bytes = 0; };
+    // a null buffer when the bytes are too many or no memory can be pinned
+    Buf take(size_t bytes) {
+        Buf b;
+        if (bytes == 0 || bytes > MAX_BYTES) return b;
+        {
+            std::lock_guard<std::mutex> g(mu_);
+            size_t best = free_.size();
+            for (size_t i = 0; i < free_.size(); i++)
+                if (free_[i].bytes >= bytes && (best == free_.size() || free_[i].bytes < free_[best].bytes)) best = i;
+            if (best < free_.size()) {
+                b = free_[best];
+                free_.erase(free_.begin() + (std::ptrdiff_t)best);
+                return b;
+            }
+        }
+        void *p = nullptr;
+        const size_t rounded = (bytes + ROUND - 1) / ROUND * ROUND;
+        if (hipHostMalloc(&p, rounded, hipHostMallocPortable) != hipSuccess) { (void)hipGetLastError(); return b; }
+        b.p = static_cast<char *>(p);
+        b.bytes = rounded;
+        return b;
+    }
+    void give(Buf b) {
+        if (!b.p) return;
+        {
+            std::lock_guard<std::mutex> g(mu_);
+            if (users_ > 0 && free_.size() < KEEP) { free_.push_back(b); return; }
+        }
+        (void)hipHostFree(b.p);
+    }
+    void join() { std::lock_guard<std::mutex> g(mu_); users_++; }
+    void leave() {
+        std::vector<Buf> last;
+        {
+            std::lock_guard<std::mutex> g(mu_);
+            if (--users_ == 0) last.swap(free_);
+        }
+        for (const Buf &b : last) (void)hipHostFree(b.p);
+    }
+
+private:
+    static constexpr size_t KEEP = 4;
+    std::mutex mu_;
+    std::vector<Buf> free_;
+    int users_ = 0;
+};
+// never destroyed: a context may outlive this file's statics
+PinnedPool &pinned_pool() { static PinnedPool *p = new PinnedPool; return *p; }
+struct PoolUser {
+    PoolUser() { pinned_pool().join(); }
+    ~PoolUser() { pinned_pool().leave(); }
+    PoolUser(const PoolUser &) = delete;
+    PoolUser &operator=(const PoolUser &) = delete;
+};
+}  // namespace
+
 struct fsg_ctx {
+    PoolUser pool_user;
     fsg_ref_desc d;
     int32_t L, div_iter, order, first_invalid;
     int device;
@@ -270,7 +339,6 @@ struct fsg_ctx {
     const uint32_t *stop_d = nullptr;
     char *buf = nullptr;
     size_t buf_bytes = 0;
-    unsigned long long *work = nullptr;
     std::vector<void *> owned;
     // orbit, Xrange register and BLA coefficients: owned jointly by every
     // context created on the same reference (fsg_ctx_create_shared)
@@ -465,11 +533,13 @@ size_t staging_bytes(const fsg_ctx *c, int64_t n) {
     return align256(pb) + align256(zb) + 2 * align256(ub) + align256(rb);
 }
 
-// one tile through device staging at b (staging_bytes(c, n) bytes) with the
-// cursor and counters at work; the caller holds c->mu
+// One tile through device staging at b (staging_bytes(c, n) bytes) with the
+// cursor and counters at work; the caller holds c->mu.  pooled: work follows
+// the staging, and the results come back in one copy to a pinned buffer (when
+// there is one).  200x200 at 1e-12, the whole call: 495 -> 370 us.
 int tile_staged(fsg_ctx *c, const double *c_pix, int64_t n, int64_t grid_w, double *Z, int32_t *U,
                 int8_t *stop_reason, int32_t *stop_iter, const volatile uint8_t *interrupted,
-                fsg_stats *stats, char *b, unsigned long long *work) {
+                fsg_stats *stats, char *b, unsigned long long *work, bool pooled) {
     const size_t pb = (size_t)n * 16, zb = z_bytes(c, n), ub = (size_t)n * 4, rb = (size_t)n;
     const size_t off_z = align256(pb), off_u = off_z + align256(zb), off_i = off_u + align256(ub);
     const size_t off_r = off_i + align256(ub);
@@ -487,10 +557,23 @@ int tile_staged(fsg_ctx *c, const double *c_pix, int64_t n, int64_t grid_w, doub
                     reinterpret_cast<int32_t *>(b + off_u), reinterpret_cast<int8_t *>(b + off_r),
                     reinterpret_cast<int32_t *>(b + off_i), work, c->stream, true, -1, 0, grid_w, stop);
     if (rc) return rc;
+    constexpr size_t STAT_BYTES = 64;                 // the counters, first words of the work area
+    struct Lease {
+        PinnedPool::Buf b;
+        hipStream_t stream;
+        // a call that fails leaves with its copy under way
+        ~Lease() {
+            if (b.p && stream) (void)hipStreamSynchronize(stream);
+            pinned_pool().give(b);
+        }
+    } host{{}, c->stream};
+    const size_t back = staging_bytes(c, n) - off_z + STAT_BYTES;
+    if (pooled && n > 0) host.b = pinned_pool().take(back);
+    if (host.b.p) FSG_HIP(hipMemcpyAsync(host.b.p, b + off_z, back, hipMemcpyDeviceToHost, c->stream));
     if (stop) {
         // wait for the kernel (its end event), passing the caller's interrupt
         // flag on to it (the reference polls it after every pixel,
-        // perturbation.py:1042-1043); the copies to pageable host memory are
+        // perturbation.py:1042-1043); copies to pageable host memory are
         // enqueued after, since enqueueing them can block this thread
         int spins = 0;
         hipError_t q;
@@ -501,17 +584,26 @@ int tile_staged(fsg_ctx *c, const double *c_pix, int64_t n, int64_t grid_w, doub
         }
         if (q != hipSuccess) return fail(FSG_E_HIP, std::string("tile: ") + hipGetErrorString(q));
     }
-    if (n > 0) {
+    if (n > 0 && !host.b.p) {
         FSG_HIP(hipMemcpyAsync(Z, b + off_z, zb, hipMemcpyDeviceToHost, c->stream));
         FSG_HIP(hipMemcpyAsync(U, b + off_u, ub, hipMemcpyDeviceToHost, c->stream));
         FSG_HIP(hipMemcpyAsync(stop_iter, b + off_i, ub, hipMemcpyDeviceToHost, c->stream));
         FSG_HIP(hipMemcpyAsync(stop_reason, b + off_r, rb, hipMemcpyDeviceToHost, c->stream));
     }
     FSG_HIP(hipStreamSynchronize(c->stream));
+    host.stream = nullptr;
+    const char *const h = host.b.p;
+    if (h) {
+        std::memcpy(Z, h, zb);
+        std::memcpy(U, h + (off_u - off_z), ub);
+        std::memcpy(stop_iter, h + (off_i - off_z), ub);
+        std::memcpy(stop_reason, h + (off_r - off_z), rb);
+    }
     if (stats) {
         std::memset(stats, 0, sizeof(*stats));
-        unsigned long long w[WORK_WORDS];
-        FSG_HIP(hipMemcpy(w, work, sizeof(w), hipMemcpyDeviceToHost));
+        unsigned long long w[STAT_BYTES / 8];
+        if (h) std::memcpy(w, h + (back - STAT_BYTES), sizeof(w));
+        else FSG_HIP(hipMemcpy(w, work, sizeof(w), hipMemcpyDeviceToHost));
         stats->plain_steps = w[1]; stats->bla_steps = w[2]; stats->bla_iters = w[3]; stats->rebases = w[4];
         stats->bla_lookups = w[5]; stats->redo_pixels = w[6];
         float ms = 0.f;
@@ -736,10 +828,6 @@ int ctx_create(const fsg_ref_desc *desc, fsg_ctx *base, fsg_ctx **out) {
         if (be != hipSuccess || hipStreamSynchronize(c->stream) != hipSuccess)
             return cleanup(fail(FSG_E_HIP, "FP32X table build failed"));
     }
-    hipError_t err;
-    c->work = dalloc<unsigned long long>(WORK_WORDS, err);
-    if (err != hipSuccess) return cleanup(fail(FSG_E_NOMEM, "hipMalloc work"));
-    c->owned.push_back(c->work);
     *out = c;
     return 0;
 }
@@ -807,13 +895,14 @@ int fsg_tile_grid(fsg_ctx *c, const double *c_pix, int64_t n, int64_t grid_w, do
     if (grid_w < 0) return fail(FSG_E_INVALID, "negative grid width");
     if (interrupted && *interrupted) return FSG_INTERRUPTED;
     std::lock_guard<std::mutex> lk(c->mu);
-    const size_t total = staging_bytes(c, n);
+    const size_t staged = staging_bytes(c, n), total = staged + WORK_WORDS * sizeof(unsigned long long);
     if (total > c->buf_bytes) {
         if (c->buf) { (void)hipFree(c->buf); c->buf = nullptr; c->buf_bytes = 0; }
         if (hipMalloc(&c->buf, total) != hipSuccess) { c->buf = nullptr; return fail(FSG_E_NOMEM, "hipMalloc tile buffers"); }
         c->buf_bytes = total;
     }
-    return tile_staged(c, c_pix, n, grid_w, Z, U, stop_reason, stop_iter, interrupted, stats, c->buf, c->work);
+    return tile_staged(c, c_pix, n, grid_w, Z, U, stop_reason, stop_iter, interrupted, stats, c->buf,
+                       reinterpret_cast<unsigned long long *>(static_cast<char *>(c->buf) + staged), true);
 }
 
 int fsg_tile_grid_noalloc(fsg_ctx *c, const double *c_pix, int64_t n, int64_t grid_w, double *Z,
@@ -838,7 +927,7 @@ int fsg_tile_grid_noalloc(fsg_ctx *c, const double *c_pix, int64_t n, int64_t gr
     std::lock_guard<std::mutex> lk_dev(g_scratch[c->device].mu);
     std::lock_guard<std::mutex> lk(c->mu);
     return tile_staged(c, c_pix, n, grid_w, Z, U, stop_reason, stop_iter, interrupted, stats,
-                       base, reinterpret_cast<unsigned long long *>(base + FSG_NOALLOC_SCRATCH_BYTES));
+                       base, reinterpret_cast<unsigned long long *>(base + FSG_NOALLOC_SCRATCH_BYTES), false);
 }
 
 int fsg_tile_device(fsg_ctx *c, const double *d_c_pix, int64_t n, double *d_Z, int32_t *d_U,
