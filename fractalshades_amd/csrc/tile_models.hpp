@@ -359,7 +359,7 @@ struct HoloXr {
         int32_t e, eG, s1, s2;
         __device__ void set(const xl &d, const xz &Zp, int32_t et) {
             v = mk(d.re, d.im); e = d.e; Z = mk(Zp.re, Zp.im);
-            eG = Zp.e < XL_ZERO_E / 2 ? e : Zp.e;          // a zero value has no scale of its own
+            eG = Zp.e;                                     // (a zero value, far below: near() takes v's scale)
             s1 = e - eG; s2 = et - s1;
         }
         // the exponents moved together where a shift is out of range
@@ -389,8 +389,6 @@ struct HoloXr {
         v.re = ldexp(v.re, -k); v.im = ldexp(v.im, -k);
         v.e = mx == 0. ? zero : REL ? v.e - k : v.e + k;
     }
-    // a derivative with its exponent, after t trips
-    __device__ static xl deriv(const xl &v, int32_t t) { xl r = v; r.e = rel(v.e, t); return xl_of(as_z(r)); }
 
     // derivative path values, unnormalised: the host's Xrange records keep
     // |mantissa| within 2^+-100, and a zero entry carries the zero exponent
@@ -625,27 +623,42 @@ struct HoloXr {
         // both rebases (perturbation.py:1283-1372) share the derivative
         // updates: one block, whichever of them a lane takes
         const bool reb_div = s.w >= t.div_iter - 1;
-        bool reb = reb_div;
+        bool reb = reb_div, plain = true;                // plain: the new z is ZZ
         xl ZZx;
         if (!reb_div) {
             s.dyn = dyn;
             if (s.dyn) {
-                s.z = xl_of(as_z(s.z));
-                ZZx = s.z + ZRv(t, t.zn_k[w1], Z1);
-                reb = le_abs2(ZZx, s.z);
+                // Decided by |z + Z|^2 <= |z|^2 on extended-range values.  Where
+                // no component of ZZ is zero or small (the components of z are
+                // then no smaller), ZZ is their sum to the bit, the squares
+                // round alike, and components that are no larger have a sum of
+                // squares that is no larger: 5 instructions instead of 60
+                // (1920x1080 at 1e-800: z^3 + c 541 -> 513 us, z^6 + c 555 -> 520).
+                const int32_t kr = KIND == KIND_M2 ? k1 : t.zn_k[w1];
+                plain = amax(ZZ.re, ZZ.im) >= 0x1p-480 && amin(ZZ.re, ZZ.im) >= 0x1p-1000 && kr >= ZK_REGISTER;
+                reb = true;
+                if (!plain) {
+                    s.z = xl_of(as_z(s.z));
+                    ZZx = s.z + ZRv(t, kr, Z1);
+                    reb = le_abs2(ZZx, s.z);
+                }
             }
         }
         if (reb) {
-            if (reb_div) { s.zs = ZZ; s.z = xl_of(ZZ); }
+            if (plain) { s.zs = ZZ; s.z = xl_of(ZZ); }
             else { s.z = ZZx; s.zs = to_std(ZZx); }
-            // the path values unnormalised: the sum's normalisation covers them
-            if (DC_ON(a)) { s.d = add_n(as_z(deriv(s.d, trip + 1)), DCz(t, s.w)); s.d.e = rel(s.d.e, trip + 1); }
-            if (DZ_ON(a)) {
-                s.h = deriv(s.h, trip + 1);
-                if (!s.nul) s.h = add_n(as_z(s.h), H1);   // dZndz at w (at L after a full period)
-                s.h.e = rel(s.h.e, trip + 1);
-                s.nul = true;
+            // Neither term normalised: the sum aligns them by their exponents,
+            // and what a drifting mantissa loses there lies far below the other
+            // term's last place; the sum's normalisation covers the result.
+            if (DC_ON(a)) {
+                s.d = add_n(xz{s.d.re, s.d.im, rel(s.d.e, trip + 1)}, DCz(t, s.w));
+                s.d.e = rel(s.d.e, trip + 1);
             }
+            if (DZ_ON(a) && !s.nul) {
+                s.h = add_n(xz{s.h.re, s.h.im, rel(s.h.e, trip + 1)}, H1);   // dZndz at w (at L after a full period)
+                s.h.e = rel(s.h.e, trip + 1);
+            }
+            s.nul = DZ_ON(a);
             s.w = 0;
             k.reb++;
         }

@@ -42,6 +42,12 @@ FSG_DEV double amax(double x, double y) {
     return r;
 }
 
+FSG_DEV double amin(double x, double y) {
+    double r;
+    asm("v_min_f64 %0, |%1|, |%2|" : "=v"(r) : "v"(x), "v"(y));
+    return r;
+}
+
 // normalised: larger component in [1, 2), or (0, 0, XL_ZERO_E)
 FSG_DEV xl xl_n(double re, double im, int32_t e) {
     const double mx = amax(re, im);
