@@ -72,6 +72,11 @@ struct LdsPlan {
     int32_t zn, dc, dc_e, dz, dz_e, bs[4], bs_e[4], zn_k, r, M;
 };
 
+// What a plan stages of the tables that the launch reads: all of them; the orbit,
+// its codes and the BLA radii but none of the derivative paths; or another
+// part.  The kernels of the first two know each table's address space.
+enum LdsShape { LDS_PART = 0, LDS_FULL = 1, LDS_ORBIT = 2 };
+
 // The binary32 form's tables staged in LDS (byte offsets, -1 = read from
 // global memory): orbit (binary64, for the escape tests), BLA radii, and the
 // xs orbit, derivative paths and BLA coefficients.  full: all of them; else
@@ -125,11 +130,10 @@ hipError_t launch_tile(const LaunchCfg &cfg, const KArgs &a, hipStream_t stream)
 // (fsg_lds.hip, blocks of up to 1024 lanes)
 typedef void (*tile_fn)(const KArgs);
 tile_fn select_tile_orbit(const LaunchCfg &cfg);
-tile_fn select_tile_orbit_lds(const LaunchCfg &cfg, bool full, int der);
+tile_fn select_tile_orbit_lds(const LaunchCfg &cfg, LdsShape shape, int der);
 // der: the derivatives the launch computes (bit 0 dz/dc, bit 1 dz/dz)
-tile_fn select_tile_lds(const LaunchCfg &cfg, bool full, int der);
-// true when the plan stages every table the launch reads
-bool lds_plan_full(const Tables &t, const LdsPlan &p);
+tile_fn select_tile_lds(const LaunchCfg &cfg, LdsShape shape, int der);
+LdsShape lds_shape(const Tables &t, const LdsPlan &p);
 // radii_only: M already holds the coefficients (shared with another
 // context of the same orbit); write the radii r only
 // rk: the radii's keys, written with r

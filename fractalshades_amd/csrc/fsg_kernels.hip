@@ -325,12 +325,15 @@ LdsPlan plan_lds(const Tables &t, int bla_dim, int max_bytes) {
     return p;
 }
 
-bool lds_plan_full(const Tables &t, const LdsPlan &p) {
-    bool ok = p.zn >= 0 && (!t.zn_k || p.zn_k >= 0) && (!t.dz || p.dz >= 0) &&
-              (!t.dz_e || p.dz_e >= 0) && (!t.dc || p.dc >= 0) && (!t.dc_e || p.dc_e >= 0) &&
-              (!t.bla_on || (p.r >= 0 && p.M >= 0));
-    for (int q = 0; q < 4; q++) ok = ok && (!t.bs[q] || p.bs[q] >= 0) && (!t.bs_e[q] || p.bs_e[q] >= 0);
-    return ok;
+LdsShape lds_shape(const Tables &t, const LdsPlan &p) {
+    const bool orbit = p.zn >= 0 && (!t.zn_k || p.zn_k >= 0) && (!t.bla_on || p.r >= 0);
+    bool all = orbit && (!t.bla_on || p.M >= 0), none = p.dz < 0 && p.dz_e < 0 && p.dc < 0 && p.dc_e < 0;
+    all = all && (!t.dz || p.dz >= 0) && (!t.dz_e || p.dz_e >= 0) && (!t.dc || p.dc >= 0) && (!t.dc_e || p.dc_e >= 0);
+    for (int q = 0; q < 4; q++) {
+        all = all && (!t.bs[q] || p.bs[q] >= 0) && (!t.bs_e[q] || p.bs_e[q] >= 0);
+        none = none && p.bs[q] < 0 && p.bs_e[q] < 0;
+    }
+    return all ? LDS_FULL : orbit && none ? LDS_ORBIT : LDS_PART;
 }
 
 hipError_t launch_tile(const LaunchCfg &cfg, const KArgs &a, hipStream_t stream) {
@@ -341,7 +344,7 @@ hipError_t launch_tile(const LaunchCfg &cfg, const KArgs &a, hipStream_t stream)
         KArgs al = a;
         al.lds = plan_lds(a.t, cfg.kind == KIND_BS ? 8 : 4, max_lds_bytes());
         const int der = (a.calc_dc ? 1 : 0) | (a.calc_dz ? 2 : 0);
-        tile_fn f = al.lds.bytes > 0 ? select_tile_lds(cfg, lds_plan_full(a.t, al.lds), der) : nullptr;
+        tile_fn f = al.lds.bytes > 0 ? select_tile_lds(cfg, lds_shape(a.t, al.lds), der) : nullptr;
         const int fill = f ? fill_blocks(reinterpret_cast<const void *>(f), 1024, al.lds.bytes) : -1;
         if (fill > 0) {
             const int block = tile_block(fill, al);

@@ -33,20 +33,20 @@ tile_fn select_tile_orbit(const LaunchCfg &c) {
 // 1001x667 with dz/dc, from global memory with every step through the recorder
 // and now: 133 -> 119 us at 1e-150, 171 -> 135 at 1e-300; the burning ship with
 // extended range spills here and is faster all the same (1e-800: 421 -> 379).
-template <class Model> static tile_fn fn_lds(bool full) {
-    return full ? k_tile_lds<Model, true> : k_tile_lds<Model, false>;
+template <class Model> static tile_fn fn_lds(LdsShape shape) {
+    return shape == LDS_FULL ? k_tile_lds<Model, LDS_FULL> : k_tile_lds<Model, LDS_PART>;
 }
-template <template <int> class Model> static tile_fn fn_lds_der2(bool full, int der) {
-    return der == 1 ? fn_lds<Model<1>>(full) : der == 3 ? fn_lds<Model<3>>(full) : fn_lds<Model<-1>>(full);
+template <template <int> class Model> static tile_fn fn_lds_der2(LdsShape shape, int der) {
+    return der == 1 ? fn_lds<Model<1>>(shape) : der == 3 ? fn_lds<Model<3>>(shape) : fn_lds<Model<-1>>(shape);
 }
 template <int DER> using M2Xr = HoloXr<KIND_M2, 2, true, DER>;
 template <int DER> using M2Std = HoloStd<KIND_M2, 2, true, DER>;
 
-tile_fn select_tile_orbit_lds(const LaunchCfg &c, bool full, int der) {
-    if (c.kind == KIND_M2) return c.xr ? fn_lds_der2<M2Xr>(full, der) : fn_lds_der2<M2Std>(full, der);
+tile_fn select_tile_orbit_lds(const LaunchCfg &c, LdsShape shape, int der) {
+    if (c.kind == KIND_M2) return c.xr ? fn_lds_der2<M2Xr>(shape, der) : fn_lds_der2<M2Std>(shape, der);
     if (c.kind == KIND_MN) {
         switch (c.degree) {
-#define FSG_MN(D) case D: return c.xr ? fn_lds<HoloXr<KIND_MN, D, true>>(full) : fn_lds<HoloStd<KIND_MN, D, true>>(full);
+#define FSG_MN(D) case D: return c.xr ? fn_lds<HoloXr<KIND_MN, D, true>>(shape) : fn_lds<HoloStd<KIND_MN, D, true>>(shape);
             FSG_MN(2) FSG_MN(3) FSG_MN(4) FSG_MN(5) FSG_MN(6) FSG_MN(7) FSG_MN(8)
 #undef FSG_MN
             default: return nullptr;
@@ -54,7 +54,7 @@ tile_fn select_tile_orbit_lds(const LaunchCfg &c, bool full, int der) {
     }
     if (c.kind == KIND_BS) {
         switch (c.flavor) {
-#define FSG_BS(F) case F: return c.xr ? fn_lds<BsXr<F, true>>(full) : fn_lds<BsStd<F, true>>(full);
+#define FSG_BS(F) case F: return c.xr ? fn_lds<BsXr<F, true>>(shape) : fn_lds<BsStd<F, true>>(shape);
             FSG_BS(1) FSG_BS(2) FSG_BS(3) FSG_BS(4) FSG_BS(5)
 #undef FSG_BS
             default: return nullptr;

@@ -357,9 +357,13 @@ __global__ void __launch_bounds__(256) k_tile(const KArgs a) {
 // radius and coefficients at the lane's own iteration index), and an LDS
 // read answers in a fraction of an L2 hit's time.  One block of up to 1024
 // lanes (tile_block) per CU, or more when they fit, copies the tables once, then runs the loop.
-// FULL: the plan stages every table the launch has, so each table pointer
-// is either null or an LDS address, and the compiler reads the tables with
-// LDS instructions instead of generic (flat) ones
+// SHAPE: LDS_FULL: each table pointer is either null or an LDS address, and the
+// compiler reads the tables with LDS instructions instead of generic (flat)
+// ones.  LDS_ORBIT: the orbit, its codes and the radii are, the derivative paths
+// are global addresses; only the BLA coefficients, staged or not, are generic.
+// A flat load takes a 64-bit address and waits on both counters; LDS_ORBIT
+// instead of LDS_PART: 2048x2048 at 1e-2000 735 -> 702 us, burning ship
+// 1920x1080 at 1e-800 795 -> 752 us, at 1e-60 (1001x667) 187 -> 175 us.
 template <bool FULL, class T>
 __device__ __forceinline__ const T *stage(unsigned char *lds, int32_t off, const T *src, int64_t n) {
     if constexpr (FULL) {
@@ -372,40 +376,43 @@ __device__ __forceinline__ const T *stage(unsigned char *lds, int32_t off, const
     return dst;
 }
 
-template <class Model, bool FULL, int BLOCK = 1024>
+template <class Model, int SHAPE, int BLOCK = 1024>
 __global__ void __launch_bounds__(BLOCK) k_tile_lds(const KArgs a) {
     extern __shared__ __align__(16) unsigned char lds[];
+    constexpr bool FULL = SHAPE == LDS_FULL, ORBIT = SHAPE != LDS_PART;
     const LdsPlan &p = a.lds;
     KArgs al = a;
     Tables &t = al.t;
     const int64_t K = p.K, KB = p.KB;
-    t.Zn = stage<FULL>(lds, p.zn, a.t.Zn, K);
-    t.dc = stage<FULL>(lds, p.dc, a.t.dc, K);
-    t.dc_e = stage<FULL>(lds, p.dc_e, a.t.dc_e, K);
-    if ((FULL || p.dz >= 0) && a.t.dz) {
-        cplx *dz = reinterpret_cast<cplx *>(lds + p.dz);
-        for (int64_t i = threadIdx.x; i < K; i += blockDim.x) dz[i] = a.t.dz[i];
-        if (threadIdx.x == 0) dz[K] = a.t.dz[a.t.L];
-        t.dz = dz;
-    } else if constexpr (FULL) {
-        t.dz = nullptr;
-    }
-    if ((FULL || p.dz_e >= 0) && a.t.dz_e) {
-        int32_t *dze = reinterpret_cast<int32_t *>(lds + p.dz_e);
-        for (int64_t i = threadIdx.x; i < K; i += blockDim.x) dze[i] = a.t.dz_e[i];
-        if (threadIdx.x == 0) dze[K] = a.t.dz_e[a.t.L];
-        t.dz_e = dze;
-    } else if constexpr (FULL) {
-        t.dz_e = nullptr;
-    }
-    for (int q = 0; q < 4; q++) {
-        t.bs[q] = stage<FULL>(lds, p.bs[q], a.t.bs[q], K);
-        t.bs_e[q] = stage<FULL>(lds, p.bs_e[q], a.t.bs_e[q], K);
-    }
-    t.zn_k = stage<FULL>(lds, p.zn_k, a.t.zn_k, K * a.t.zn_k_w);
-    t.rk = stage<FULL>(lds, p.r, a.t.rk, KB);
+    t.Zn = stage<ORBIT>(lds, p.zn, a.t.Zn, K);
+    t.zn_k = stage<ORBIT>(lds, p.zn_k, a.t.zn_k, K * a.t.zn_k_w);
+    t.rk = stage<ORBIT>(lds, p.r, a.t.rk, KB);
     t.M = stage<FULL>(lds, p.M, a.t.M, KB * p.bla_dim);
-    if ((FULL || p.dz >= 0) && a.t.dz) t.L = (int32_t)K;   // the wrapped dZndz value is staged at [K]
+    if constexpr (SHAPE != LDS_ORBIT) {
+        t.dc = stage<FULL>(lds, p.dc, a.t.dc, K);
+        t.dc_e = stage<FULL>(lds, p.dc_e, a.t.dc_e, K);
+        if ((FULL || p.dz >= 0) && a.t.dz) {
+            cplx *dz = reinterpret_cast<cplx *>(lds + p.dz);
+            for (int64_t i = threadIdx.x; i < K; i += blockDim.x) dz[i] = a.t.dz[i];
+            if (threadIdx.x == 0) dz[K] = a.t.dz[a.t.L];
+            t.dz = dz;
+        } else if constexpr (FULL) {
+            t.dz = nullptr;
+        }
+        if ((FULL || p.dz_e >= 0) && a.t.dz_e) {
+            int32_t *dze = reinterpret_cast<int32_t *>(lds + p.dz_e);
+            for (int64_t i = threadIdx.x; i < K; i += blockDim.x) dze[i] = a.t.dz_e[i];
+            if (threadIdx.x == 0) dze[K] = a.t.dz_e[a.t.L];
+            t.dz_e = dze;
+        } else if constexpr (FULL) {
+            t.dz_e = nullptr;
+        }
+        for (int q = 0; q < 4; q++) {
+            t.bs[q] = stage<FULL>(lds, p.bs[q], a.t.bs[q], K);
+            t.bs_e[q] = stage<FULL>(lds, p.bs_e[q], a.t.bs_e[q], K);
+        }
+        if ((FULL || p.dz >= 0) && a.t.dz) t.L = (int32_t)K;   // the wrapped dZndz value is staged at [K]
+    }
     __syncthreads();
     tile_loop<Model>(al);
 }
