@@ -3,7 +3,8 @@
 // onto the GPU.
 //
 // Design.  One scheduler thread per server owns L "lanes" (a HIP stream, a
-// completion event and a small work buffer each) and one copy stream.  A
+// completion event per chunk enqueued on it and a small work buffer each) and
+// one copy stream.  A
 // request is split into chunks of `chunk_px` pixels; every chunk is one
 // launch of the persistent tile kernel on a free lane, capped at 1/L of the
 // GPU's resident waves so that up to L chunks -- from different requests,
@@ -134,6 +135,7 @@ struct Req {
     int64_t off = -1;
     char *dev = nullptr;
     int32_t chunks = 0, dispatched = 0, finished = 0;
+    bool quick = false;       // its last finished chunk took less than QUICK_MS
     hipEvent_t h2d = nullptr, d2h = nullptr;
     int state = PENDING;
     int status = 0;
@@ -143,11 +145,25 @@ struct Req {
     double t_submit = 0, t_admit = 0, t_first = -1, t_done = 0;
 };
 
+// A lane: a stream and the chunks enqueued on it, oldest first.  The scheduler
+// sees the end of a chunk only at its next look, 50 to 100 us on, longer than
+// most chunks run, and a lane of one chunk was idle meanwhile.  A second one keeps
+// the stream busy; the stream's order lets both use the lane's work area.  A burst
+// of 12 requests in chunks of 65536 pixels: one chunk a lane 6.1 ms, two, and
+// looking again after 5 us instead of 40, 4.5; a third gains 4 % more, and every
+// new request would wait for it.  A chunk waits behind another only where that one's
+// request has shown chunks shorter than QUICK_MS: behind a chunk of seconds it
+// would stay while other lanes fall free.
+constexpr int LANE_DEPTH = 2;
+constexpr double QUICK_MS = 1.;
 struct Lane {
     hipStream_t s = nullptr;
-    hipEvent_t ev = nullptr;
     unsigned long long *work = nullptr;
-    Req *req = nullptr;
+    hipEvent_t ev[LANE_DEPTH] = {};
+    Req *req[LANE_DEPTH] = {};
+    int head = 0, count = 0;
+    double t_head = 0;                    // when the oldest chunk came to the front
+    bool room() const { return count == 0 || (count < LANE_DEPTH && req[(head + count - 1) % LANE_DEPTH]->quick); }
 };
 
 }  // namespace
@@ -241,13 +257,19 @@ void fsg_server::loop() {
 
         // chunks that completed
         for (Lane &ln : lanes) {
-            if (!ln.req) continue;
-            const hipError_t q = hipEventQuery(ln.ev);
-            if (q == hipErrorNotReady) continue;
-            if (q != hipSuccess) fail_req(ln.req, FSG_E_HIP, "tile kernel failed");
-            ln.req->finished++;
-            ln.req = nullptr;
-            progress = true;
+            while (ln.count > 0) {
+                const hipError_t q = hipEventQuery(ln.ev[ln.head]);
+                if (q == hipErrorNotReady) break;
+                Req *r = ln.req[ln.head];
+                if (q != hipSuccess) fail_req(r, FSG_E_HIP, "tile kernel failed");
+                r->finished++;
+                const double t = now();
+                r->quick = t - ln.t_head < QUICK_MS;
+                ln.t_head = t;
+                ln.head = (ln.head + 1) % LANE_DEPTH;
+                ln.count--;
+                progress = true;
+            }
         }
         // requests whose chunks are all done: results back to the host
         for (size_t i = 0; i < active.size();) {
@@ -294,9 +316,14 @@ void fsg_server::loop() {
             }
             ++i;
         }
-        // free lanes take the next chunk: fewest chunks dispatched first
-        for (Lane &ln : lanes) {
-            if (ln.req) continue;
+        // lanes with room take the next chunk, the emptiest first: fewest
+        // chunks dispatched first
+        for (size_t turn = 0; turn < lanes.size() * LANE_DEPTH; turn++) {
+            Lane *to = nullptr;
+            for (Lane &x : lanes)
+                if (x.room() && (!to || x.count < to->count)) to = &x;
+            if (!to) break;
+            Lane &ln = *to;
             Req *best = nullptr;
             for (Req *r : active) {
                 if (r->state != ACTIVE || r->dispatched >= r->chunks) continue;
@@ -322,15 +349,18 @@ void fsg_server::loop() {
                                       reinterpret_cast<int32_t *>(d + best->lay.si) + start,
                                       ln.work, ln.s, -(int)lanes.size(), best->grid_w);
             if (rc != 0) fail_req(best, rc, fsg_last_error());
-            (void)hipEventRecord(ln.ev, ln.s);
-            ln.req = best;
+            const int slot = (ln.head + ln.count) % LANE_DEPTH;
+            if (ln.count == 0) ln.t_head = now();
+            (void)hipEventRecord(ln.ev[slot], ln.s);
+            ln.req[slot] = best;
+            ln.count++;
             progress = true;
         }
         if (!progress) {
             std::unique_lock<std::mutex> lk(mu);
             bool busy = !active.empty();
             if (busy)
-                cv_work.wait_for(lk, std::chrono::microseconds(40));
+                cv_work.wait_for(lk, std::chrono::microseconds(5));
             else
                 cv_work.wait_for(lk, std::chrono::milliseconds(5), [&] { return stop || !pending.empty(); });
         }
@@ -358,7 +388,7 @@ int fsg_server_create(const fsg_server_opts *opts, fsg_server **out) {
     auto cleanup = [&](int rc) {
         for (Lane &ln : s->lanes) {
             if (ln.work) (void)hipFree(ln.work);
-            if (ln.ev) (void)hipEventDestroy(ln.ev);
+            for (hipEvent_t e : ln.ev) if (e) (void)hipEventDestroy(e);
             if (ln.s) (void)hipStreamDestroy(ln.s);
         }
         if (s->copy) (void)hipStreamDestroy(s->copy);
@@ -375,9 +405,11 @@ int fsg_server_create(const fsg_server_opts *opts, fsg_server **out) {
     s->lanes.resize((size_t)o.lanes);
     for (Lane &ln : s->lanes) {
         if (hipStreamCreateWithFlags(&ln.s, hipStreamNonBlocking) != hipSuccess ||
-            hipEventCreateWithFlags(&ln.ev, hipEventDisableTiming) != hipSuccess ||
             hipMalloc(reinterpret_cast<void **>(&ln.work), work_words() * sizeof(unsigned long long)) != hipSuccess)
             return cleanup(set_error(FSG_E_HIP, "lane creation failed"));
+        for (hipEvent_t &e : ln.ev)
+            if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
+                return cleanup(set_error(FSG_E_HIP, "lane creation failed"));
     }
     s->th = std::thread([s] { s->loop(); });
     *out = s;
@@ -395,7 +427,7 @@ int fsg_server_destroy(fsg_server *s) {
     for (Lane &ln : s->lanes) {
         (void)hipStreamSynchronize(ln.s);
         (void)hipFree(ln.work);
-        (void)hipEventDestroy(ln.ev);
+        for (hipEvent_t e : ln.ev) (void)hipEventDestroy(e);
         (void)hipStreamDestroy(ln.s);
     }
     (void)hipStreamSynchronize(s->copy);
