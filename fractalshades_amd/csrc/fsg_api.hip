@@ -323,6 +323,8 @@ struct fsg_ctx {
     int32_t *bs_e[4] = {nullptr, nullptr, nullptr, nullptr};
     int32_t *xr_idx = nullptr, *xr_e = nullptr, *zn_k = nullptr;
     int32_t zn_k_w = 0;
+    // their first entries (KArgs)
+    double zn0[2] = {0., 0.}, dz0[2] = {0., 0.};
     double *xr_m = nullptr;
     double *M = nullptr, *r = nullptr;
     int64_t *rk = nullptr;
@@ -444,6 +446,7 @@ int fill_args(fsg_ctx *c, KArgs &a) {
     a.dx_m = c->d.dx_mant; a.dx_e = c->d.dx_exp;
     a.drift_m[0] = c->d.drift_mant[0]; a.drift_m[1] = c->d.drift_mant[1];
     a.drift_e[0] = c->d.drift_exp[0]; a.drift_e[1] = c->d.drift_exp[1];
+    for (int q = 0; q < 2; q++) { a.zn0[q] = c->zn0[q]; a.dz0[q] = c->dz0[q]; }
     a.max_iter = (int32_t)c->d.max_iter;
     a.calc_dc = c->d.calc_dzndc ? 1 : 0;
     a.calc_dz = (c->d.kind != FSG_KIND_BS && c->d.interior_detect) ? 1 : 0;
@@ -722,6 +725,7 @@ int ctx_create(const fsg_ref_desc *desc, fsg_ctx *base, fsg_ctx **out) {
     }
     // the normalisation codes: one load per orbit point, also where the
     // point comes from the register (no search of the sorted indices)
+    c->zn0[0] = desc->Zn_path[0]; c->zn0[1] = desc->Zn_path[1];
     c->zn_k_w = holo ? 1 : 2;
     if (base && base->zn_k && base->zn_k_w == c->zn_k_w) {
         c->zn_k = base->zn_k;
@@ -745,6 +749,7 @@ int ctx_create(const fsg_ref_desc *desc, fsg_ctx *base, fsg_ctx **out) {
         }
         if (c->d.interior_detect) {
             holo_dzndz(h, m, e);
+            c->dz0[0] = m[0].re; c->dz0[1] = m[0].im;
             if ((rc = upload(c, c->dz, m.data(), m.size()))) return cleanup(rc);
             if ((rc = upload(c, c->dz_e, e.data(), e.size()))) return cleanup(rc);
         }

@@ -95,6 +95,9 @@ struct KArgs {
     // filters of the escape and interior tests: |Z + z|^2 > M2 only if a component
     // exceeds esc_lo, |dz/dz|^2 < eps2 only if each component is below eps_hi
     double esc_lo, eps_hi;
+    // the orbit's first point and the binary64 dZndz value there: what the
+    // carried values of a pixel become at a rebase
+    double zn0[2], dz0[2];
     // pixels: complex128 screen offsets in units of dx ("c_pix")
     const double *pix;
     int64_t npts;

@@ -165,19 +165,29 @@ struct HoloStd {
     // Z, A, Zh: as in HoloXr, for z^2 + c
     struct State { cplx z, d, h, c, Z, A, Zh; int32_t w, n, jl; bool dyn, nul; OrbitRec<ORB> orb; };
 
+    // the carried values at w = 0: from the launch arguments, since a pixel near
+    // the critical orbit rebases at every step, each a wait for these otherwise
+    __device__ static void at_start(State &s, const KArgs &a) {
+        s.Z = mk(a.zn0[0], a.zn0[1]);
+        s.A = s.Z + s.z;
+        if (DZ_ON(a)) s.Zh = mk(a.dz0[0], a.dz0[1]);
+    }
+
     __device__ static void init(State &s, const KArgs &a, double px, double py) {
         s.c = to_std(c_from_pix(a, px, py));
         s.z = zc(); s.d = zc(); s.h = zc();
+        if constexpr (KIND == KIND_M2) at_start(s, a);
         s.w = 0; s.n = 0; s.jl = 0; s.dyn = true; s.nul = false;
         s.orb.reset(a.backshift);
     }
 
     __device__ static bool step(State &s, const KArgs &a, Counters &k, int &reason, int32_t) {
         const Tables &t = a.t;
-        if ((KIND == KIND_M2 || t.bla_on) && (s.w & 7) == 0) {
-            int32_t stage = -1, idx;
-            if (t.bla_on) k.looks++;
-            if (t.bla_on) do {
+        if (t.bla_on && (s.w & 7) == 0) {
+            int32_t stage, idx;
+            [[maybe_unused]] const int32_t w0 = s.w;
+            k.looks++;
+            do {
                 stage = bla_lookup(t, s.z.re, s.z.im, s.w, idx);
                 if (stage >= 0) {
                     const int32_t st = 8 << stage;
@@ -193,9 +203,11 @@ struct HoloStd {
                 pin(stage);
             } while (stage >= 0);
             if constexpr (KIND == KIND_M2) {
-                s.Z = t.Zn[s.w];
-                if (DZ_ON(a)) s.Zh = t.dz[s.nul ? 0 : s.w];
-                s.A = s.Z + s.z;
+                if (s.w != w0) {
+                    s.Z = t.Zn[s.w];
+                    if (DZ_ON(a) && !s.nul) s.Zh = t.dz[s.w];
+                    s.A = s.Z + s.z;
+                }
             }
         }
         s.n += 1;
@@ -233,13 +245,16 @@ struct HoloStd {
             const cplx W = mk(__builtin_fma(2., s.Z.re, s.z.re), __builtin_fma(2., s.Z.im, s.z.im));
             pin_after(w1, W.re, W.im);
             Z1 = t.Zn[w1];
-            if (DC_ON(a)) s.d = muls(2., s.A * s.d + Zd * s.z);
+            // dZndz's term first: its value is at hand, and the load that
+            // follows it is then under way before the wait for dZndc's
+            cplx v = zc();
             if (DZ_ON(a)) {
-                const cplx v = s.Zh * s.z;
+                v = s.Zh * s.z;
                 pin_after(wh, v.re, v.im);
                 H1 = t.dz[wh];
-                s.h = muls(2., s.A * s.h + v);
             }
+            if (DC_ON(a)) s.d = muls(2., s.A * s.d + Zd * s.z);
+            if (DZ_ON(a)) s.h = muls(2., s.A * s.h + v);
             s.z = s.z * W + s.c;
         }
         s.w = w1;
@@ -280,7 +295,10 @@ struct HoloStd {
                 s.nul = true;
             }
             s.w = 0;
+            if constexpr (KIND == KIND_M2) at_start(s, a);
             k.reb++;
+        } else if (KIND == KIND_M2 && DZ_ON(a) && edge && !s.nul) {
+            s.Zh = t.dz[s.w];                   // not the wrapped value of the test
         }
         return false;
     }
@@ -522,6 +540,12 @@ struct HoloXr {
             pin(sd); pin(sh);
             pin_after(w1, W.re, W.im);
             Z1 = t.Zn[w1]; k1 = t.zn_k[w1];
+            cplx vh = zc();
+            if (DZ_ON(a)) {                                      // (before dz/dc: HoloStd)
+                vh = mk(Zh.re, Zh.im) * mk(s.z.re, s.z.im);
+                pin_after(wh, vh.re, vh.im);
+                H1 = DZz(t, wh);
+            }
             if (max(sz, max(sd, sh)) > FAR) {
                 if (sz > FAR) { W = mk(ldexp(W.re, -sz), ldexp(W.im, -sz)); s.z.e += sz; sz = 0; }
                 if (sd > FAR) { s.d.re = ldexp(s.d.re, -sd); s.d.im = ldexp(s.d.im, -sd); s.d.e -= sd; sd = 0; }
@@ -533,10 +557,8 @@ struct HoloXr {
                 s.d.re = u.re + ldexp(v.re, sd); s.d.im = u.im + ldexp(v.im, sd);
             }
             if (DZ_ON(a)) {
-                const cplx u = A * mk(s.h.re, s.h.im), v = mk(Zh.re, Zh.im) * z;
-                pin_after(wh, v.re, v.im);
-                H1 = DZz(t, wh);
-                s.h.re = u.re + ldexp(v.re, sh); s.h.im = u.im + ldexp(v.im, sh);
+                const cplx u = A * mk(s.h.re, s.h.im);
+                s.h.re = u.re + ldexp(vh.re, sh); s.h.im = u.im + ldexp(vh.im, sh);
             }
             const cplx u = z * W;
             s.z.re = u.re + ldexp(s.c.re, sz); s.z.im = u.im + ldexp(s.c.im, sz);
