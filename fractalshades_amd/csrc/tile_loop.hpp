@@ -214,7 +214,17 @@ __device__ __forceinline__ void tile_loop(const KArgs &a) {
         const KArgs &g = cold_args();
         int64_t idx = 0;
         unsigned filled = 0;              // lanes [0, filled) have a pixel
-        while (filled < 64u) {
+        // The binary64 pass: a wave takes its share of the unsure pixels at
+        // once, at most 64.  Where they are few they are the longest ones, and
+        // packed into few waves each would pay for the others' branches
+        // (a 24-frame zoom sequence 3.45 -> 2.9 s).
+        unsigned want = 64u;
+        if (g.redo) {
+            const unsigned waves = gridDim.x * (blockDim.x >> 6);
+            const unsigned share = (unsigned)(min(g.work[6], 0xffffffffull - waves) + waves - 1u) / waves;
+            want = min(64u, max(1u, share));
+        }
+        while (filled < want) {
             if (rest == 0ull) {
                 // the next 64 slots, base .. base + 63
                 const unsigned waves = blockDim.x >> 6;
@@ -295,7 +305,7 @@ __device__ __forceinline__ void tile_loop(const KArgs &a) {
                 const auto below = [](unsigned long long m) {
                     return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
                 };
-                const bool goes = ((rest >> __lane_id()) & 1ull) != 0ull && filled + below(rest) < 64u;
+                const bool goes = ((rest >> __lane_id()) & 1ull) != 0ull && filled + below(rest) < want;
                 const unsigned long long sent = __builtin_amdgcn_ballot_w64(goes);
                 const unsigned rank = below(sent), end = filled + (unsigned)__popcll(sent);
                 const int to = (int)(4u * ((goes ? filled + rank : end + __lane_id() - rank) & 63u));
