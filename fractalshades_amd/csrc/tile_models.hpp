@@ -229,15 +229,19 @@ struct HoloStd {
         if (DZ_ON(a) && s.nul) wh = 0;
         cplx Z1, Zd = zc(), H1 = zc();
         if (DC_ON(a)) Zd = t.dc[s.w];
-        if (s.dyn) {
-            pin(w1);
-            Zd = zc();
-        }
+        // after the other loads are out: overwriting Zd waits for its own
+        const auto first_step = [&]() {
+            if (s.dyn) {
+                pin(w1);
+                Zd = zc();
+            }
+        };
         if constexpr (KIND == KIND_MN) {
             const cplx Zr = t.Zn[s.w];
             Z1 = t.Zn[w1];
             cplx Zh = zc();
             if (DZ_ON(a)) { Zh = t.dz[s.nul ? 0 : s.w]; H1 = t.dz[wh]; }
+            first_step();
             s.z = mn_step<DEG>(s.z, Zr, s.c, DC_ON(a), DZ_ON(a), s.d, s.h, s.d, s.h, Zd, Zh,
                                [](cplx u, cplx v) { return u + v; });
         } else {
@@ -253,6 +257,7 @@ struct HoloStd {
                 pin_after(wh, v.re, v.im);
                 H1 = t.dz[wh];
             }
+            first_step();
             if (DC_ON(a)) s.d = muls(2., s.A * s.d + Zd * s.z);
             if (DZ_ON(a)) s.h = muls(2., s.A * s.h + v);
             s.z = s.z * W + s.c;
