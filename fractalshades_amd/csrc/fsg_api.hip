@@ -55,16 +55,16 @@ template <class T> T *dalloc(size_t n, hipError_t &err) {
 // component, scaled into [1, 2); the exponent of zero for a zero value), or
 // INT32_MIN + its Xrange register slot.  Holomorphic: one code per point
 // (the complex value); burning ship: two (x, then y).
-void point_codes(const fsg_ref_desc *d, int w, std::vector<int32_t> &code) {
+void point_codes(const fsg_ref_desc *d, cplx end, int w, std::vector<int32_t> &code) {
     const int64_t L = d->ref_len;
-    code.assign((size_t)(w * L), 0);
+    code.assign((size_t)(w * (L + 1)), 0);
     const auto norm_exp = [](double mx) {
         int k0 = 0;
         if (mx != 0.) (void)std::frexp(mx, &k0);
         return (mx == 0.) ? XL_ZERO_E : k0 - 1;
     };
-    for (int64_t i = 0; i < L; i++) {
-        const double x = std::fabs(d->Zn_path[2 * i]), y = std::fabs(d->Zn_path[2 * i + 1]);
+    for (int64_t i = 0; i <= L; i++) {
+        const double x = std::fabs(i < L ? d->Zn_path[2 * i] : end.re), y = std::fabs(i < L ? d->Zn_path[2 * i + 1] : end.im);
         if (w == 1) {
             code[(size_t)i] = norm_exp(std::max(x, y));
         } else {
@@ -101,6 +101,29 @@ template <class T> void jac_rt(int fl, T x, T y, T J[4]) {
         case 4: bs_jac<4>(x, y, J); break;
         default: bs_jac<5>(x, y, J); break;
     }
+}
+
+// The orbit's entry past its last point, Zn[L].  A jump can land on the last
+// point of an orbit that neither escapes nor closes (div_iter = L); the step
+// from there ends on the next one, and the pixel's results are taken there.
+// Z_L = f(Z_{L-1}) + c in binary64, with c = Z_1 (the burning ship: (a, -b)).
+cplx end_point(const fsg_ref_desc *d) {
+    const int64_t L = d->ref_len;
+    const cplx z = mk(d->Zn_path[2 * L - 2], d->Zn_path[2 * L - 1]), c = mk(d->Zn_path[2], d->Zn_path[3]);
+    if (d->kind != KIND_BS) {
+        cplx r = z;
+        for (int q = 1; q < (d->kind == KIND_M2 ? 2 : d->degree); q++) r = r * z;
+        return r + c;
+    }
+    double x = z.re, y = z.im;
+    switch (d->flavor) {
+        case 1: bs_zn<1>(x, y, 0., 0., c.re, -c.im); break;
+        case 2: bs_zn<2>(x, y, 0., 0., c.re, -c.im); break;
+        case 3: bs_zn<3>(x, y, 0., 0., c.re, -c.im); break;
+        case 4: bs_zn<4>(x, y, 0., 0., c.re, -c.im); break;
+        default: bs_zn<5>(x, y, 0., 0., c.re, -c.im); break;
+    }
+    return mk(x, y);
 }
 
 struct HostRef {
@@ -150,23 +173,26 @@ void zero_codes(const std::vector<double> &m, std::vector<int32_t> &e) {
         if (m[k] == 0.) e[k] = XL_ZERO_E;
 }
 
-// dZndc: D_0 = 0, D_i = f'(Z_{i-1}) D_{i-1} + s, wrapped value at [0] for cycles
+// dZndc: D_0 = 0, D_i = f'(Z_{i-1}) D_{i-1} + s, wrapped value at [0] for
+// cycles; its entry at [L] as the orbit's (end_point)
 void holo_dzndc(const HostRef &h, std::vector<cplx> &m, std::vector<int32_t> &e) {
     const fsg_ref_desc *d = h.d;
     const int64_t L = h.L, valid = std::min<int64_t>(h.L, h.div_iter);
-    m.assign(L, mk(0., 0.)); e.assign(L, 0);
+    m.assign(L + 1, mk(0., 0.)); e.assign(L + 1, 0);
     const xf s = deriv_scale(d);
     if (!d->xr_mode) {
         const double ss = to_std(s);
         for (int64_t i = 1; i < valid; i++) m[i] = dfdz_rt(d->kind, d->degree, h.Z(i - 1)) * m[i - 1] + mk(ss, 0.);
         int64_t i = valid - 1;
+        if (valid == L) m[L] = dfdz_rt(d->kind, d->degree, h.Z(i)) * m[i] + mk(ss, 0.);
         if (i == (int64_t)d->ref_order - 1) m[0] = dfdz_rt(d->kind, d->degree, h.Z(i)) * m[i] + mk(ss, 0.);
     } else {
-        std::vector<xc> D(L, mkc(0., 0., 0));
+        std::vector<xc> D(L + 1, mkc(0., 0., 0));
         for (int64_t i = 1; i < valid; i++) D[i] = dfdz_rt(d->kind, d->degree, h.Zxr(i - 1)) * D[i - 1] + s;
         int64_t i = valid - 1;
+        if (valid == L) D[L] = dfdz_rt(d->kind, d->degree, h.Zxr(i)) * D[i] + s;
         if (i == (int64_t)d->ref_order - 1) D[0] = D[i] * dfdz_rt(d->kind, d->degree, h.Z(i)) + s;
-        for (int64_t k = 0; k < L; k++) { m[k] = mk(D[k].re, D[k].im); e[k] = D[k].e; }
+        for (int64_t k = 0; k <= L; k++) { m[k] = mk(D[k].re, D[k].im); e[k] = D[k].e; }
         zero_codes(m, e);
     }
 }
@@ -192,11 +218,12 @@ void holo_dzndz(const HostRef &h, std::vector<cplx> &m, std::vector<int32_t> &e)
     }
 }
 
-// Burning-ship Jacobian paths (numba_dZndc_path_BS + incr_deriv_ref_BS)
+// Burning-ship Jacobian paths (numba_dZndc_path_BS + incr_deriv_ref_BS), with
+// their entry at [L] as the orbit's (end_point)
 void bs_paths(const HostRef &h, std::vector<double> P[4], std::vector<int32_t> E[4]) {
     const fsg_ref_desc *d = h.d;
     const int64_t L = h.L, valid = std::min<int64_t>(h.L, h.div_iter);
-    for (int q = 0; q < 4; q++) { P[q].assign(L, 0.); E[q].assign(L, 0); }
+    for (int q = 0; q < 4; q++) { P[q].assign(L + 1, 0.); E[q].assign(L + 1, 0); }
     if (!d->calc_dzndc) return;
     const xf s = deriv_scale(d);
     auto incr_std = [&](int64_t from, int64_t to) {
@@ -212,11 +239,12 @@ void bs_paths(const HostRef &h, std::vector<double> P[4], std::vector<int32_t> E
     };
     if (!d->xr_mode) {
         for (int64_t i = 1; i < valid; i++) incr_std(i - 1, i);
+        if (valid == L) incr_std(L - 1, L);
         if (valid - 1 == (int64_t)d->ref_order - 1) incr_std(valid - 1, 0);
         return;
     }
     std::vector<xf> X[4];
-    for (int q = 0; q < 4; q++) X[q].assign(L, mkf(0., 0));
+    for (int q = 0; q < 4; q++) X[q].assign(L + 1, mkf(0., 0));
     auto incr_xr = [&](int64_t from, int64_t to) {
         xf Rx, Ry, J[4];
         h.ZxrBS(from, Rx, Ry);
@@ -228,9 +256,10 @@ void bs_paths(const HostRef &h, std::vector<double> P[4], std::vector<int32_t> E
         X[3][to] = J[2] * xb + J[3] * yb - s;
     };
     for (int64_t i = 1; i < valid; i++) incr_xr(i - 1, i);
+    if (valid == L) incr_xr(L - 1, L);
     if (valid - 1 == (int64_t)d->ref_order - 1) incr_xr(valid - 1, 0);
     for (int q = 0; q < 4; q++) {
-        for (int64_t k = 0; k < L; k++) { P[q][k] = X[q][k].m; E[q][k] = X[q][k].e; }
+        for (int64_t k = 0; k <= L; k++) { P[q][k] = X[q][k].m; E[q][k] = X[q][k].e; }
         zero_codes(P[q], E[q]);
     }
 }
@@ -390,12 +419,14 @@ uint64_t ref_hash_of(const fsg_ref_desc *d) {
     return h;
 }
 
-template <class T> int upload(fsg_ctx *c, T *&dst, const T *src, size_t n, bool shared = false) {
+// end: an entry to follow src's, or null
+template <class T> int upload(fsg_ctx *c, T *&dst, const T *src, size_t n, bool shared = false, const T *end = nullptr) {
     hipError_t err;
-    dst = dalloc<T>(n, err);
+    dst = dalloc<T>(n + (end ? 1 : 0), err);
     if (err != hipSuccess) return fail(FSG_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(err));
     (shared ? c->shared->p : c->owned).push_back(dst);
     if (n) FSG_HIP(hipMemcpy(dst, src, n * sizeof(T), hipMemcpyHostToDevice));
+    if (end) FSG_HIP(hipMemcpy(dst + n, end, sizeof(T), hipMemcpyHostToDevice));
     return 0;
 }
 
@@ -691,6 +722,9 @@ int ctx_create(const fsg_ref_desc *desc, fsg_ctx *base, fsg_ctx **out) {
     c->L = (int32_t)desc->ref_len;
     c->div_iter = (int32_t)desc->ref_div_iter;
     c->order = desc->ref_order > (int64_t)INT32_MAX ? INT32_MAX : (int32_t)desc->ref_order;
+    // an orbit that does not reach its period (a longer max_iter than the one
+    // it was computed for): pixels rebase at its last point
+    if (c->order > c->L) c->div_iter = std::min(c->div_iter, c->L);
     c->first_invalid = std::min(c->L, std::min(c->div_iter, c->order));
     auto cleanup = [&](int code) { delete c; return code; };
 
@@ -712,13 +746,14 @@ int ctx_create(const fsg_ref_desc *desc, fsg_ctx *base, fsg_ctx **out) {
     const int64_t L = c->L;
     const int32_t nx = desc->n_xr;
     const int holo = desc->kind != FSG_KIND_BS;
+    const cplx end = end_point(desc);
     c->ref_hash = h_ref;
     if (base) {
         c->shared = base->shared;
         c->Zn = base->Zn; c->xr_idx = base->xr_idx; c->xr_m = base->xr_m; c->xr_e = base->xr_e;
     } else {
         c->shared = std::make_shared<fsg_ctx::Shared>();
-        if ((rc = upload(c, c->Zn, reinterpret_cast<const cplx *>(desc->Zn_path), (size_t)L, true))) return cleanup(rc);
+        if ((rc = upload(c, c->Zn, reinterpret_cast<const cplx *>(desc->Zn_path), (size_t)L, true, &end))) return cleanup(rc);
         if ((rc = upload(c, c->xr_idx, desc->xr_index, (size_t)nx, true))) return cleanup(rc);
         if ((rc = upload(c, c->xr_m, desc->xr_mant, (size_t)2 * nx, true))) return cleanup(rc);
         if ((rc = upload(c, c->xr_e, desc->xr_exp, (size_t)(holo ? nx : 2 * nx), true))) return cleanup(rc);
@@ -731,7 +766,7 @@ int ctx_create(const fsg_ref_desc *desc, fsg_ctx *base, fsg_ctx **out) {
         c->zn_k = base->zn_k;
     } else {
         std::vector<int32_t> code;
-        point_codes(desc, c->zn_k_w, code);
+        point_codes(desc, end, c->zn_k_w, code);
         if ((rc = upload(c, c->zn_k, code.data(), code.size(), true))) return cleanup(rc);
     }
 
@@ -797,12 +832,12 @@ int ctx_create(const fsg_ref_desc *desc, fsg_ctx *base, fsg_ctx **out) {
     // binary32 copies of the burning-ship orbit and Jacobian paths
     if (c->d.precision == FSG_PREC_FP32X && c->d.kind == FSG_KIND_BS) {
         hipError_t xe;
-        void *p = dalloc<char>((size_t)L * 2 * XSR_BYTES, xe);
+        void *p = dalloc<char>(((size_t)L + 1) * 2 * XSR_BYTES, xe);
         c->owned.push_back(p); c->tx.ZRx = p;
         if (xe != hipSuccess) return cleanup(fail(FSG_E_NOMEM, "hipMalloc FP32X tables"));
         for (int q = 0; q < 4; q++) {
             if (!c->bs[q]) continue;
-            p = dalloc<char>((size_t)L * XSR_BYTES, xe);
+            p = dalloc<char>(((size_t)L + 1) * XSR_BYTES, xe);
             c->owned.push_back(p); c->tx.BSx[q] = p;
             if (xe != hipSuccess) return cleanup(fail(FSG_E_NOMEM, "hipMalloc FP32X tables"));
         }

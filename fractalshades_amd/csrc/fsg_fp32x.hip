@@ -137,10 +137,10 @@ __global__ void k_xs_bla(const double *M, int64_t n, xs *A, xs *B) {
 
 hipError_t build_xs_tables(const Tables &t, int64_t bla_len, TablesX &x, hipStream_t stream) {
     const int tb = 256;
-    hipLaunchKernelGGL(k_xs_orbit, dim3((t.L + tb - 1) / tb), dim3(tb), 0, stream, t.Zn, t.L,
+    hipLaunchKernelGGL(k_xs_orbit, dim3((t.L + tb) / tb), dim3(tb), 0, stream, t.Zn, t.L + 1,
                        t.xr_idx, t.xr_m, t.xr_e, t.n_xr, (xs *)x.Zx);
-    if (t.dc) hipLaunchKernelGGL(k_xs_from_path, dim3((t.L + tb - 1) / tb), dim3(tb), 0, stream,
-                                 (const double *)t.dc, t.dc_e, t.L, (xs *)x.DCx);
+    if (t.dc) hipLaunchKernelGGL(k_xs_from_path, dim3((t.L + tb) / tb), dim3(tb), 0, stream,
+                                 (const double *)t.dc, t.dc_e, t.L + 1, (xs *)x.DCx);
     if (t.dz) hipLaunchKernelGGL(k_xs_from_path, dim3((t.L + tb) / tb), dim3(tb), 0, stream,
                                  (const double *)t.dz, t.dz_e, t.L + 1, (xs *)x.DZx);
     if (t.bla_on && bla_len > 0)
@@ -705,12 +705,12 @@ __global__ void k_xsr_path(const double *m, const int32_t *e, int32_t n, xsr *ou
 
 hipError_t build_xsr_tables(const Tables &t, TablesX &x, hipStream_t stream) {
     const int tb = 256;
-    hipLaunchKernelGGL(k_xsr_orbit, dim3((t.L + tb - 1) / tb), dim3(tb), 0, stream, t.Zn, t.L,
+    hipLaunchKernelGGL(k_xsr_orbit, dim3((t.L + tb) / tb), dim3(tb), 0, stream, t.Zn, t.L + 1,
                        t.xr_idx, t.xr_m, t.xr_e, t.n_xr, (xsr *)x.ZRx);
     for (int q = 0; q < 4; q++)
         if (t.bs[q] && x.BSx[q])
-            hipLaunchKernelGGL(k_xsr_path, dim3((t.L + tb - 1) / tb), dim3(tb), 0, stream,
-                               t.bs[q], t.bs_e[q], t.L, (xsr *)x.BSx[q]);
+            hipLaunchKernelGGL(k_xsr_path, dim3((t.L + tb) / tb), dim3(tb), 0, stream,
+                               t.bs[q], t.bs_e[q], t.L + 1, (xsr *)x.BSx[q]);
     return hipGetLastError();
 }
 
@@ -848,7 +848,7 @@ __global__ void __launch_bounds__(1024) k_tile_lds_bsx(const KArgs a) {
 static LdsPlanX plan_lds_bsx(const Tables &t, int max_bytes) {
     LdsPlanX p;
     std::memset(&p, 0xff, sizeof(p));
-    int64_t K = std::min<int64_t>(t.L, std::min<int64_t>((int64_t)t.div_iter + 1, t.order));
+    int64_t K = std::min<int64_t>((int64_t)t.L + 1, std::min<int64_t>((int64_t)t.div_iter + 1, t.order));
     K = std::max<int64_t>(K, std::min<int64_t>(t.L, 2));
     const int64_t bla_len = 2 * (int64_t)(t.L >> 3);
     const int64_t KB = t.bla_on ? std::min<int64_t>(bla_len, K / 4 + 2) : 0;
@@ -933,7 +933,7 @@ __global__ void __launch_bounds__(1024) k_tile_lds_x(const KArgs a) {
 static LdsPlanX plan_lds_x(const Tables &t, const TablesX &x, int max_bytes) {
     LdsPlanX p;
     std::memset(&p, 0xff, sizeof(p));
-    int64_t K = std::min<int64_t>(t.L, std::min<int64_t>((int64_t)t.div_iter + 1, t.order));
+    int64_t K = std::min<int64_t>((int64_t)t.L + 1, std::min<int64_t>((int64_t)t.div_iter + 1, t.order));
     K = std::max<int64_t>(K, std::min<int64_t>(t.L, 2));
     const int64_t bla_len = 2 * (int64_t)(t.L >> 3);
     const int64_t KB = (t.bla_on && x.Ax) ? std::min<int64_t>(bla_len, K / 4 + 2) : 0;

@@ -24,19 +24,19 @@ constexpr int TILE_STATIC_LDS = 1024;
 
 // Read-only per-reference data, resident in HBM for the life of a context.
 struct Tables {
-    const cplx *Zn;            // [L] reference orbit Z_n rounded to binary64
+    const cplx *Zn;            // [L + 1] reference orbit Z_n rounded to binary64 ([L]: end_point)
     int32_t L, div_iter, order, first_invalid;
-    // holomorphic orbit derivatives: dZn/dc [L], dZn/dz [L+1]; in Xrange
+    // holomorphic orbit derivatives: dZn/dc and dZn/dz [L + 1]; in Xrange
     // mode the exponents sit in the parallel *_e arrays
     const cplx *dc; const int32_t *dc_e;
     const cplx *dz; const int32_t *dz_e;
-    // Burning-ship Jacobian paths dX/da, dX/db, dY/da, dY/db [L]
+    // Burning-ship Jacobian paths dX/da, dX/db, dY/da, dY/db [L + 1]
     const double *bs[4]; const int32_t *bs_e[4];
     // sparse Xrange register of orbit points below 1e-300 (sorted indices)
     int32_t n_xr; int32_t zn_k_w;
     const int32_t *xr_idx; const double *xr_m; const int32_t *xr_e;
     // orbit points in the extended-range kernels' normalised form, zn_k_w
-    // codes per point [zn_k_w L]: holomorphic, one per point (the complex
+    // codes per point [zn_k_w (L + 1)]: holomorphic, one per point (the complex
     // value); burning ship, two (x, then y).  A code k >= ZK_REGISTER: the
     // binary64 value scaled by 2^-k is the normalised mantissa (larger
     // component in [1, 2); k is the exponent of zero for a zero value);

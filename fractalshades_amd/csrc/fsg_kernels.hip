@@ -275,14 +275,14 @@ int max_lds_bytes() {
 
 // Byte offsets of the tables staged in LDS (-1: read from global memory).
 // Entries 0 .. K-1 of each staged table (K = the iterations a pixel can
-// reach, min(L, div_iter + 1, order)), with the wrapped dZndz value at [K].
+// reach, min(L + 1, div_iter + 1, order)), with the wrapped dZndz value at [K].
 // The tables are taken in the order the loop reads them most -- orbit,
 // normalisation codes / Xrange slots, dZndz, dZndc (burning ship: its four paths), BLA radii and
 // coefficients -- as long as they fit; bytes = 0 when not even the orbit does.
 LdsPlan plan_lds(const Tables &t, int bla_dim, int max_bytes) {
     LdsPlan p;
     std::memset(&p, 0xff, sizeof(p));               // every offset -1
-    int64_t K = std::min<int64_t>(t.L, std::min<int64_t>((int64_t)t.div_iter + 1, t.order));
+    int64_t K = std::min<int64_t>((int64_t)t.L + 1, std::min<int64_t>((int64_t)t.div_iter + 1, t.order));
     K = std::max<int64_t>(K, std::min<int64_t>(t.L, 2));   // Zn[1] (orbit finish)
     const int64_t bla_len = 2 * (int64_t)(t.L >> 3);
     const int64_t KB = t.bla_on ? std::min<int64_t>(bla_len, K / 4 + 2) : 0;
