@@ -60,7 +60,7 @@ __device__ __forceinline__ int64_t grid_slot(int64_t s, int64_t n, int64_t w) {
 __device__ __forceinline__ void pin(int32_t &v) { asm("" : "+v"(v)); }
 // the same, not before x and y are known: a load at index v then takes the
 // registers that x and y were made from instead of copying into them later
-__device__ __forceinline__ void pin_after(int32_t &v, double x, double y) { asm("" : "+v"(v) : "v"(x), "v"(y)); }
+template <class T> __device__ __forceinline__ void pin_after(T &v, double x, double y) { asm("" : "+v"(v) : "v"(x), "v"(y)); }
 
 // --------------------------------------------------------------------------
 // BLA stage selection (ref_BLA_get, perturbation.py:2116-2170).  The tree
