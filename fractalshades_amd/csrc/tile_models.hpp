@@ -111,30 +111,23 @@ __device__ __forceinline__ int32_t bla_lookup(const Tables &t, xl z, int32_t w, 
 // The z^d + c step with the derivatives the launch computes (dz/dc when dc,
 // dz/dz when dz): one pass over the shared partial products
 // (p_zn_derivs); Zd / Zh are read only for the derivatives computed.
-// add(a, b) takes the last sum of each result and returns it as an R
-// (binary64: the sum; extended range: the normalised sum).
-template <int DEG, class T, class R, class Add>
-__device__ __forceinline__ R mn_step(T z, T Z, T c, bool dc, bool dz, R &d, R &h, T d0, T h0, T Zd, T Zh,
-                                     Add add) {
+template <int DEG>
+__device__ __forceinline__ cplx mn_step(cplx z, cplx Z, cplx c, bool dc, bool dz, cplx &d, cplx &h, cplx Zd, cplx Zh) {
     if (dc && dz) {
-        const T v[2] = {d0, h0};
-        const T Zv[2] = {Zd, Zh};
-        R o[2];
-        const R r = p_zn_derivs<DEG, 2>(z, Z, c, v, Zv, o, add);
+        const cplx v[2] = {d, h}, Zv[2] = {Zd, Zh};
+        cplx o[2];
+        const cplx r = p_zn_derivs<DEG, 2>(z, Z, c, v, Zv, o);
         d = o[0]; h = o[1];
         return r;
     }
     if (dc || dz) {
-        const T v[1] = {dc ? d0 : h0};
-        const T Zv[1] = {dc ? Zd : Zh};
-        R o[1];
-        const R r = p_zn_derivs<DEG, 1>(z, Z, c, v, Zv, o, add);
+        const cplx v[1] = {dc ? d : h}, Zv[1] = {dc ? Zd : Zh};
+        cplx o[1];
+        const cplx r = p_zn_derivs<DEG, 1>(z, Z, c, v, Zv, o);
         (dc ? d : h) = o[0];
         return r;
     }
-    const T zz[1] = {z};
-    R o[1];
-    return p_zn_derivs<DEG, 0>(z, Z, c, zz, zz, o, add);
+    return p_zn_derivs<DEG, 0, cplx>(z, Z, c, nullptr, nullptr, nullptr);
 }
 
 // ---- pixel -> c (ref_path_c_from_pix + lin_proj_impl, perturbation.py:2214-2230, 2665-2672)
@@ -249,8 +242,7 @@ struct HoloStd {
                 pin(w1);
                 Zd = zc();
             }
-            s.z = mn_step<DEG>(s.z, Zr, s.c, DC_ON(a), DZ_ON(a), s.d, s.h, s.d, s.h, Zd, Zh,
-                               [](cplx u, cplx v) { return u + v; });
+            s.z = mn_step<DEG>(s.z, Zr, s.c, DC_ON(a), DZ_ON(a), s.d, s.h, Zd, Zh);
         } else {
             // mandelbrot_M2.py:607-622: z (z + 2 Z) + c, 2 ((Z + z) d + Zd z)
             const cplx W = mk(__builtin_fma(2., s.Z.re, s.z.re), __builtin_fma(2., s.Z.im, s.z.im));

@@ -159,71 +159,24 @@ FSG_DEV cplx to_std(xl a) {
 }
 FSG_DEV double to_std(xlf a) { return ldexp(a.m, max(a.e, -2200)); }
 
-// ---- lazily normalised intermediates ---------------------------------------
-// Within one iteration, values are combined without renormalising: their
-// mantissas start in [1, 2) (state, orbit point) or within 2^+-100 (the
-// reference's derivative paths) and a few products and sums cannot take
-// them near the binary64 limits, so every operation still rounds exactly
-// as the reference's.  Only a zero result needs care: it takes XL_ZERO_E so
-// that it never sets the exponent of a later sum.  The state is
-// renormalised (xl_of) once per iteration.
+// ---- values used without normalising ----------------------------------------
+// A derivative path's value as it is loaded (its mantissa within 2^+-100) and a
+// state's drifting one: operands of add_n, which aligns them by their exponents
+// and normalises the sum.  A zero carries XL_ZERO_E, so that it never sets the
+// exponent of a sum.
 struct xz { double re, im; int32_t e; };
 
-FSG_DEV xz xz_mk(double re, double im, int32_t e) {
-    xz r;
-    r.re = re; r.im = im;
-    r.e = (amax(re, im) == 0.) ? XL_ZERO_E : e;
-    return r;
-}
 FSG_DEV xz as_z(xl a) { xz r; r.re = a.re; r.im = a.im; r.e = a.e; return r; }
 FSG_DEV xz xz_zero() { xz r; r.re = 0.; r.im = 0.; r.e = XL_ZERO_E; return r; }
 FSG_DEV xl xl_of(xz a) { return xl_n(a.re, a.im, a.e); }
 
-FSG_DEV xz operator+(xz a, xz b) {
+// a + b, normalised.  The normalisation tests the result for zero, so the sum
+// needs no zero test of its own.
+FSG_DEV xl add_n(xz a, xz b) {
     const int32_t E = max(a.e, b.e);
     const int32_t sa = shift_of(a.e, E), sb = shift_of(b.e, E);
-    return xz_mk(ldexp(a.re, sa) + ldexp(b.re, sb), ldexp(a.im, sa) + ldexp(b.im, sb), E);
+    return xl_n(ldexp(a.re, sa) + ldexp(b.re, sb), ldexp(a.im, sa) + ldexp(b.im, sb), E);
 }
-// A product of two values is zero only when a factor is (mantissas stay
-// within 2^+-300, far from underflow), and a zero factor carries the
-// sentinel, so the product's exponent is already below any other: no
-// zero test is needed.  (At most 8 sentinels add up within one iteration --
-// Z^7 times a zero path value -- far from the int32 limit; the state is
-// renormalised after.)
-FSG_DEV xz operator*(xz a, xz b) {
-    const double ac = a.re * b.re, bd = a.im * b.im, ad = a.re * b.im, bc = a.im * b.re;
-    xz r;
-    r.re = ac - bd; r.im = ad + bc; r.e = a.e + b.e;
-    return r;
-}
-FSG_DEV xz operator*(xz a, cplx b) {
-    const double ac = a.re * b.re, bd = a.im * b.im, ad = a.re * b.im, bc = a.im * b.re;
-    return xz_mk(ac - bd, ad + bc, a.e);
-}
-FSG_DEV xz muls(double s, xz a) { xz r; r.re = s * a.re; r.im = s * a.im; r.e = a.e; return r; }   // s != 0
-// 2^f (a + b), normalised: the sum of the last operation of an iteration.
-// The normalisation tests the result for zero, so the sum needs no zero
-// test of its own; the factor 2^f goes to the exponent.
-FSG_DEV xl add_n(xz a, xz b, int32_t f = 0) {
-    const int32_t E = max(a.e, b.e);
-    const int32_t sa = shift_of(a.e, E), sb = shift_of(b.e, E);
-    return xl_n(ldexp(a.re, sa) + ldexp(b.re, sb), ldexp(a.im, sa) + ldexp(b.im, sb), E + f);
-}
-// a b, normalised (the normalisation's zero test replaces the product's)
-FSG_DEV xl mul_n(xz a, cplx b) {
-    const double ac = a.re * b.re, bd = a.im * b.im, ad = a.re * b.im, bc = a.im * b.re;
-    return xl_n(ac - bd, ad + bc, a.e);
-}
-// a + b for a sum that only a comparison reads: a zero result needs no
-// exponent of its own there
-FSG_DEV xz add_raw(xz a, xz b) {
-    const int32_t E = max(a.e, b.e);
-    const int32_t sa = shift_of(a.e, E), sb = shift_of(b.e, E);
-    xz r;
-    r.re = ldexp(a.re, sa) + ldexp(b.re, sb); r.im = ldexp(a.im, sa) + ldexp(b.im, sb); r.e = E;
-    return r;
-}
-FSG_DEV xlf abs2(xz a) { return xlf_n(a.re * a.re + a.im * a.im, 2 * max(a.e, -(1 << 27))); }
 // |a|^2 <= |b|^2 for normalised a, b: le(abs2(a), abs2(b)) without
 // normalising the two squares -- each sum of squares lies in [1, 8) (or is
 // zero), so the aligned larger one is at least 1 and a shift that takes the
@@ -234,13 +187,6 @@ FSG_DEV bool le_abs2(xl a, xl b) {
     const int32_t E = max(ea, eb);
     return ldexp(qa, ea - E) <= ldexp(qb, eb - E);
 }
-// |a|^2 < b for a binary64 b > 0: the mantissa sum rounds as abs2's, and
-// scaling it by 2^(2e) is exact unless the result leaves the normal range,
-// where it lies far on one side of b whichever way it rounds
-FSG_DEV bool abs2_lt(xz a, double b) {
-    return ldexp(a.re * a.re + a.im * a.im, 2 * max(a.e, -(1 << 27))) < b;
-}
-
 // Lazily normalised reals for the burning-ship step (the same argument as
 // xz: mantissas of the operands start in [1, 2), one iteration's products
 // of at most three factors and sums of a few terms stay far inside the
@@ -265,16 +211,6 @@ FSG_DEV xzf operator-(xzf a) { a.m = -a.m; return a; }
 FSG_DEV xzf operator*(xzf a, xzf b) { xzf r; r.m = a.m * b.m; r.e = a.e + b.e; return r; }
 FSG_DEV xzf operator*(double s, xzf a) { xzf r; r.m = s * a.m; r.e = (s == 0.) ? XL_ZERO_E : a.e; return r; }
 FSG_DEV xzf mul_s(double s, xzf a) { return s * a; }
-// s * a for a binary64 s of any magnitude (BLA coefficients): s is split
-// into a mantissa in [1, 2) and an exponent, so that sums of such products
-// stay in range; the product rounds as s * a.m does
-FSG_DEV xzf mul_w(double s, xzf a) {
-    const int32_t k = dexp(s) - 1;
-    xzf r;
-    r.m = ldexp(s, -k) * a.m;
-    r.e = (s == 0.) ? XL_ZERO_E : a.e + k;
-    return r;
-}
 FSG_DEV xzf absv(xzf x) { x.m = fabs(x.m); return x; }
 // comparisons with zero: the sign of the mantissa
 FSG_DEV xzf diffabs(xzf X, xzf x) {
