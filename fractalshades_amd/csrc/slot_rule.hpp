@@ -8,8 +8,9 @@ namespace fsg {
 // The lanes at which a wave stops drawing batches: its part of the launch's
 // unsure pixels, 64 at most.
 FSG_HD unsigned redo_share(uint64_t unsure, unsigned waves) {
-    const uint64_t share = (unsure + waves - 1u) / waves;
-    return share < 1u ? 1u : share > 64u ? 64u : (unsigned)share;
+    if (unsure >= 64ull * waves) return 64u;
+    const unsigned share = ((unsigned)unsure + waves - 1u) / waves;
+    return share < 1u ? 1u : share;
 }
 
 // Whether an unsure slot of a drawn batch, with `before` of the batch's before
