@@ -8,9 +8,10 @@ namespace fsg {
 // The lanes at which a wave stops drawing batches: its part of the launch's
 // unsure pixels, 64 at most.
 FSG_HD unsigned redo_share(uint64_t unsure, unsigned waves) {
-    if (unsure >= 64ull * waves) return 64u;
-    const unsigned share = ((unsigned)unsure + waves - 1u) / waves;
-    return share < 1u ? 1u : share;
+    const uint64_t top = 0xffffffffull - waves;
+    const unsigned share = (unsigned)((unsure < top ? unsure : top) + waves - 1u) / waves;
+    const unsigned some = share > 1u ? share : 1u;
+    return some < 64u ? some : 64u;
 }
 
 // Whether an unsure slot of a drawn batch, with `before` of the batch's before

@@ -220,7 +220,8 @@ __device__ __forceinline__ void tile_loop(const KArgs &a) {
         // Against waves that stopped at their share: 480x270 around the
         // critical orbit, 27050 unsure pixels of 100000 steps, 363 -> 163 ms;
         // 200x200 at 1e-12 and 1e-300 91 -> 72 and 151 -> 94 us.
-        const unsigned want = g.redo ? redo_share(g.work[6], gridDim.x * (blockDim.x >> 6)) : 64u;
+        unsigned want = 64u;
+        if (g.redo) want = redo_share(g.work[6], gridDim.x * (blockDim.x >> 6));
         while (filled < want) {
             if (rest == 0ull) {
                 // the next 64 slots, base .. base + 63
