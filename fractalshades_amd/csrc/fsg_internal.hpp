@@ -132,7 +132,7 @@ hipError_t launch_tile(const LaunchCfg &cfg, const KArgs &a, hipStream_t stream)
 // the calc_orbit instantiations (fsg_orbit.hip) and the LDS-staged ones
 // (fsg_lds.hip, blocks of up to 1024 lanes)
 typedef void (*tile_fn)(const KArgs);
-tile_fn select_tile_orbit(const LaunchCfg &cfg);
+tile_fn select_tile_orbit(const LaunchCfg &cfg, int der);
 tile_fn select_tile_orbit_lds(const LaunchCfg &cfg, LdsShape shape, int der);
 // der: the derivatives the launch computes (bit 0 dz/dc, bit 1 dz/dz)
 tile_fn select_tile_lds(const LaunchCfg &cfg, LdsShape shape, int der);
@@ -143,7 +143,6 @@ LdsShape lds_shape(const Tables &t, const LdsPlan &p);
 hipError_t launch_bla_build(int kind, int degree, int flavor, const cplx *Zn, int32_t L,
                             double kc, double eps, double *M, double *r, int64_t *rk, int32_t stages,
                             hipStream_t stream, bool radii_only = false);
-int tile_kernel_blocks(const LaunchCfg &cfg);
 int grid_fill_blocks(const void *kernel);          // blocks filling the GPU at full occupancy
 int fill_blocks(const void *kernel, int block, int lds_bytes);   // the same for any block / LDS size
 // plan the LDS staging of a launch's tables (bytes = 0 when they do not fit)

@@ -157,9 +157,11 @@ __global__ void k_bla_merge(int32_t comp, int32_t stg, double kc, double eps, do
 // dispatch
 template <class Model> static tile_fn fn_of() { return k_tile<Model>; }
 
-static tile_fn select_tile(const LaunchCfg &c) {
-    if (c.orbit) return select_tile_orbit(c);
-    if (c.kind == KIND_M2) return c.xr ? fn_of<HoloXr<KIND_M2, 2>>() : fn_of<HoloStd<KIND_M2, 2>>();
+// der: the derivatives the launch computes, where a kernel is compiled for them
+static tile_fn select_tile(const LaunchCfg &c, int der) {
+    if (c.orbit) return select_tile_orbit(c, der);
+    if (c.kind == KIND_M2)
+        return c.xr ? fn_of<HoloXr<KIND_M2, 2>>() : der == 3 ? fn_of<HoloStd<KIND_M2, 2, false, 3>>() : fn_of<HoloStd<KIND_M2, 2>>();
     if (c.kind == KIND_MN) {
         switch (c.degree) {
 #define FSG_MN(D) case D: return c.xr ? fn_of<HoloXr<KIND_MN, D>>() : fn_of<HoloStd<KIND_MN, D>>();
@@ -212,12 +214,6 @@ int fill_blocks(const void *fn, int block, int lds) {
 }
 
 int grid_fill_blocks(const void *fn) { return fill_blocks(fn, 256, 0); }
-
-int tile_kernel_blocks(const LaunchCfg &cfg) {
-    tile_fn f = select_tile(cfg);
-    if (!f) return -1;
-    return grid_fill_blocks(reinterpret_cast<const void *>(f));
-}
 
 // blocks that a launch may have, of the fill that the GPU holds
 static int block_cap(int fill, const KArgs &a) {
@@ -340,10 +336,10 @@ hipError_t launch_tile(const LaunchCfg &cfg, const KArgs &a, hipStream_t stream)
     // FSG_TABLES=global keeps the tables in global memory (for comparisons)
     const char *tables = std::getenv("FSG_TABLES");
     const bool no_lds = tables && !std::strcmp(tables, "global");
+    const int der = (a.calc_dc ? 1 : 0) | (a.calc_dz ? 2 : 0);
     if (!no_lds) {
         KArgs al = a;
         al.lds = plan_lds(a.t, cfg.kind == KIND_BS ? 8 : 4, max_lds_bytes());
-        const int der = (a.calc_dc ? 1 : 0) | (a.calc_dz ? 2 : 0);
         tile_fn f = al.lds.bytes > 0 ? select_tile_lds(cfg, lds_shape(a.t, al.lds), der) : nullptr;
         const int fill = f ? fill_blocks(reinterpret_cast<const void *>(f), 1024, al.lds.bytes) : -1;
         if (fill > 0) {
@@ -353,7 +349,7 @@ hipError_t launch_tile(const LaunchCfg &cfg, const KArgs &a, hipStream_t stream)
             return hipGetLastError();
         }
     }
-    tile_fn f = select_tile(cfg);
+    tile_fn f = select_tile(cfg, der);
     if (!f) return hipErrorInvalidValue;
     const int fill = grid_fill_blocks(reinterpret_cast<const void *>(f));
     if (fill <= 0) return hipErrorInvalidValue;

@@ -7,8 +7,9 @@ namespace fsg {
 
 template <class Model> static tile_fn fn_of() { return k_tile<Model>; }
 
-tile_fn select_tile_orbit(const LaunchCfg &c) {
-    if (c.kind == KIND_M2) return c.xr ? fn_of<HoloXr<KIND_M2, 2, true>>() : fn_of<HoloStd<KIND_M2, 2, true>>();
+tile_fn select_tile_orbit(const LaunchCfg &c, int der) {
+    if (c.kind == KIND_M2)
+        return c.xr ? fn_of<HoloXr<KIND_M2, 2, true>>() : der == 3 ? fn_of<HoloStd<KIND_M2, 2, true, 3>>() : fn_of<HoloStd<KIND_M2, 2, true>>();
     if (c.kind == KIND_MN) {
         switch (c.degree) {
 #define FSG_MN(D) case D: return c.xr ? fn_of<HoloXr<KIND_MN, D, true>>() : fn_of<HoloStd<KIND_MN, D, true>>();

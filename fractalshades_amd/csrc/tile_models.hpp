@@ -155,12 +155,17 @@ template <int KIND, int DEG, bool ORB = false, int DER = -1>
 struct HoloStd {
     __device__ static bool DC_ON(const KArgs &a) { if constexpr (DER >= 0) return (DER & 1) != 0; else return a.calc_dc != 0; }
     __device__ static bool DZ_ON(const KArgs &a) { if constexpr (DER >= 0) return (DER & 2) != 0; else return a.calc_dz != 0; }
-    // z^2 + c: Z, A, Zh as in HoloXr; Zd: the dZndc value of the next step, zero
-    // for the first one of the pixel or after a dynamic rebase; first: the plain
-    // steps before that step (a condition that lives across the step is merged in
-    // scalar registers at every join of the tests).  z^d + c: dyn, the next step
-    // is such a first one.  keep: -1, 0 once dZndz is taken at 0 (after a rebase).
-    struct State { cplx z, d, h, c, Z, A, Zh, Zd; int32_t w, n, jl, first, keep; bool dyn; OrbitRec<ORB> orb; };
+    // A pixel around the critical orbit rebases at every step: FLAT has such a
+    // step pass the stop tests by (step).  With dz/dz on only, which waits for
+    // more: without it the other form is no slower for a lone pixel.
+    static constexpr bool FLAT = KIND == KIND_M2 && DER >= 2;
+    // Z, A, Zh: as in HoloXr, for z^2 + c.  FLAT: Zd, the dZndc value of the next
+    // step, zero for the first one (of the pixel or after a dynamic rebase); first,
+    // the plain steps before that step; keep, -1 or, once dZndz is taken at 0
+    // (after a rebase), 0.  The other form has dyn, the next step is a first one,
+    // and nul: conditions that live across the step, merged in scalar registers
+    // at every join of the tests.
+    struct State { cplx z, d, h, c, Z, A, Zh, Zd; int32_t w, n, jl, first, keep; bool dyn, nul; OrbitRec<ORB> orb; };
     static constexpr int32_t NOT_FIRST = -1;
 
     // the carried values at w = 0: from the launch arguments, since a pixel near
@@ -169,7 +174,7 @@ struct HoloStd {
         s.Z = mk(a.zn0[0], a.zn0[1]);
         s.A = s.Z + s.z;
         if (DZ_ON(a)) s.Zh = mk(a.dz0[0], a.dz0[1]);
-        if (DC_ON(a)) {
+        if (FLAT && DC_ON(a)) {
             s.Zd = zc();
             if (s.first == NOT_FIRST) s.Zd = a.t.dc[0];
         }
@@ -178,7 +183,7 @@ struct HoloStd {
     __device__ static void init(State &s, const KArgs &a, double px, double py) {
         s.c = to_std(c_from_pix(a, px, py));
         s.z = zc(); s.d = zc(); s.h = zc();
-        s.w = 0; s.n = 0; s.jl = 0; s.first = 0; s.keep = -1; s.dyn = true;
+        s.w = 0; s.n = 0; s.jl = 0; s.dyn = true; s.nul = false; s.first = 0; s.keep = -1;
         if constexpr (KIND == KIND_M2) at_start(s, a);
         s.orb.reset(a.backshift);
     }
@@ -207,8 +212,8 @@ struct HoloStd {
             if constexpr (KIND == KIND_M2) {
                 if (s.w != w0) {
                     s.Z = t.Zn[s.w];
-                    if (DZ_ON(a) && s.keep) s.Zh = t.dz[s.w];
-                    if (DC_ON(a) && s.n - s.jl != s.first) s.Zd = t.dc[s.w];
+                    if (DZ_ON(a) && (FLAT ? s.keep != 0 : !s.nul)) s.Zh = t.dz[s.w];
+                    if (FLAT && DC_ON(a) && s.n - s.jl != s.first) s.Zd = t.dc[s.w];
                     s.A = s.Z + s.z;
                 }
             }
@@ -229,41 +234,52 @@ struct HoloStd {
             pin(w1);
             if (w1 >= t.order) { w1 = 0; wh = s.n == t.order ? t.L : 0; }
         }
-        if (DZ_ON(a)) wh &= s.keep;
-        cplx Z1, H1 = zc(), D1 = zc();
-        if constexpr (KIND == KIND_MN) {
-            const cplx Zr = t.Zn[s.w];
-            Z1 = t.Zn[w1];
-            cplx Zd = zc(), Zh = zc();
-            if (DC_ON(a)) Zd = t.dc[s.w];
-            if (DZ_ON(a)) { Zh = t.dz[s.w & s.keep]; H1 = t.dz[wh]; }
-            // after the other loads are out: overwriting Zd waits for its own
+        if (FLAT) wh &= s.keep;
+        else if (DZ_ON(a) && s.nul) wh = 0;
+        cplx Z1, Zd = zc(), H1 = zc(), D1 = zc();
+        if (!FLAT && DC_ON(a)) Zd = t.dc[s.w];
+        // after the other loads are out: overwriting Zd waits for its own
+        const auto first_step = [&]() {
             if (s.dyn) {
                 pin(w1);
                 Zd = zc();
             }
+        };
+        if constexpr (KIND == KIND_MN) {
+            const cplx Zr = t.Zn[s.w];
+            Z1 = t.Zn[w1];
+            cplx Zh = zc();
+            if (DZ_ON(a)) { Zh = t.dz[s.nul ? 0 : s.w]; H1 = t.dz[wh]; }
+            first_step();
             s.z = mn_step<DEG>(s.z, Zr, s.c, DC_ON(a), DZ_ON(a), s.d, s.h, Zd, Zh);
         } else {
             // mandelbrot_M2.py:607-622: z (z + 2 Z) + c, 2 ((Z + z) d + Zd z)
             const cplx W = mk(__builtin_fma(2., s.Z.re, s.z.re), __builtin_fma(2., s.Z.im, s.z.im));
             pin_after(w1, W.re, W.im);
             Z1 = t.Zn[w1];
-            cplx u = zc(), v = zc();
+            // dZndz's term first: its value is at hand, and the load that
+            // follows it is then under way before the wait for dZndc's
+            cplx v = zc();
             if (DZ_ON(a)) {
                 v = s.Zh * s.z;
                 pin_after(wh, v.re, v.im);
                 H1 = t.dz[wh];
             }
-            if (DC_ON(a)) {
-                u = s.Zd * s.z;
-                pin_after(w1, u.re, u.im);
-                D1 = t.dc[w1];
-                s.d = muls(2., s.A * s.d + u);
+            if constexpr (FLAT) {
+                if (DC_ON(a)) {
+                    const cplx u = s.Zd * s.z;
+                    pin_after(w1, u.re, u.im);
+                    D1 = t.dc[w1];
+                    s.d = muls(2., s.A * s.d + u);
+                }
+            } else {
+                first_step();
+                if (DC_ON(a)) s.d = muls(2., s.A * s.d + Zd * s.z);
             }
             if (DZ_ON(a)) s.h = muls(2., s.A * s.h + v);
             s.z = s.z * W + s.c;
             // the derivatives before Z + z takes A's registers
-            if (DC_ON(a)) pin_after(Z1.re, s.d.re, s.d.im);
+            if (FLAT && DC_ON(a)) pin_after(Z1.re, s.d.re, s.d.im);
         }
         s.w = w1;
         // The stop and rebase tests are evaluated together: a step that meets
@@ -281,18 +297,16 @@ struct HoloStd {
         const cplx ZZ = s.z + Z1;
         const bool t_esc = amax(ZZ.re, ZZ.im) > a.esc_lo;
         const bool dyn = (fabs(ZZ.re) <= fabs(s.z.re)) && (fabs(ZZ.im) <= fabs(s.z.im));
-        const bool test = s.n >= a.max_iter || t_int || t_esc || edge || s.orb.due(s.n);
-        if constexpr (KIND == KIND_M2) {
-            // Here a step that meets only the rebase's test, each one of a pixel
-            // around the critical orbit, passes the others by too, and the masks
-            // of their branches are not merged step for step.  With the dZndc value
-            // carried (it answers the rebase without a wait), a lone pixel that
-            // rebases at every step takes 318 ns a step with dz/dz, 248 without (514
-            // and 360 before); 512x512 at 1e-40: 42.0 -> 39.8 us.  z^d + c, whose
-            // values are not carried, is slower so (1e-60: 340 -> 346 us).
-            s.Z = Z1; s.A = ZZ; s.Zh = H1; s.Zd = D1;
+        if constexpr (KIND == KIND_M2) { s.Z = Z1; s.A = ZZ; s.Zh = H1; s.Zd = D1; }
+        if constexpr (FLAT) {
+            // Only a step that meets a stop test, the end of the orbit or the recorder
+            // takes these branches; the rebase follows for both, its dZndc value at
+            // hand.  A lone pixel that rebases at every step takes 320 ns a step, 514 in
+            // the other form (1920x1080 at width 4, 1 million steps: 663 -> 405 ms);
+            // 900x900 at 1e-12 with the recorder 122 -> 111 us, 1500x1500 at 1e-12 240 ->
+            // 230 us.
             bool reb = dyn;
-            if (test) {
+            if (s.n >= a.max_iter || t_int || t_esc || edge || s.orb.due(s.n)) {
                 // with the recorder, some lane of the wave is here on most steps: the
                 // bounds are read again rather than held beside its scalar values
                 const KArgs &b = ORB ? cold_args() : a;
@@ -308,8 +322,8 @@ struct HoloStd {
                 if (edge) {
                     if (s.w >= t.div_iter - 1) {
                         reb = true;
-                        if (s.n - 1 - s.jl != s.first) s.first = NOT_FIRST;
-                    } else if (DZ_ON(a) && !dyn && s.keep) {
+                        if (s.n - 1 - s.jl != s.first) s.first = NOT_FIRST;     // not a first step: dZndc at 0
+                    } else if (!dyn && s.keep) {
                         s.Zh = t.dz[s.w];               // not the wrapped value of the test
                     }
                 }
@@ -317,42 +331,42 @@ struct HoloStd {
             if (reb) {
                 s.z = ZZ;
                 if (DC_ON(a)) s.d = s.d + D1;
-                if (DZ_ON(a)) {
-                    if (s.keep) s.h = s.h + H1;         // dZndz at w (at L after a full period)
-                    s.keep = 0;
-                }
+                if (s.keep) s.h = s.h + H1;             // dZndz at w (at L after a full period)
+                s.keep = 0;
                 s.w = 0;
                 at_start(s, a);
                 s.first = s.first == NOT_FIRST ? NOT_FIRST - 1 : s.n - s.jl;
                 k.reb++;
             }
             return false;
-        } else {
-            if (!(test || dyn)) { s.dyn = false; return false; }
-            if (s.n >= a.max_iter) { reason = 0; return true; }
-            if (t_int) {
-                const cplx q = s.h + H1;
-                if (q.re * q.re + q.im * q.im < a.eps2) { reason = 2; return true; }
-            }
-            s.orb.record(s.n, a.backshift, ZZ.re, ZZ.im);
-            if (t_esc && ZZ.re * ZZ.re + ZZ.im * ZZ.im > a.M2) { reason = 1; return true; }
-            bool reb = s.w >= t.div_iter - 1;
-            if (!reb) {
-                s.dyn = dyn;
-                reb = dyn;
-            }
-            if (reb) {
-                s.z = ZZ;
-                if (DC_ON(a)) s.d = s.d + t.dc[s.w];
-                if (DZ_ON(a)) {
-                    if (s.keep) s.h = s.h + H1;
-                    s.keep = 0;
-                }
-                s.w = 0;
-                k.reb++;
-            }
-            return false;
         }
+        if (!(s.n >= a.max_iter || t_int || t_esc || edge || dyn || s.orb.due(s.n))) { s.dyn = false; return false; }
+        if (s.n >= a.max_iter) { reason = 0; return true; }
+        if (t_int) {
+            const cplx q = s.h + H1;
+            if (q.re * q.re + q.im * q.im < a.eps2) { reason = 2; return true; }
+        }
+        s.orb.record(s.n, a.backshift, ZZ.re, ZZ.im);
+        if (t_esc && ZZ.re * ZZ.re + ZZ.im * ZZ.im > a.M2) { reason = 1; return true; }
+        bool reb = s.w >= t.div_iter - 1;
+        if (!reb) {
+            s.dyn = dyn;
+            reb = dyn;
+        }
+        if (reb) {
+            s.z = ZZ;
+            if (DC_ON(a)) s.d = s.d + t.dc[s.w];
+            if (DZ_ON(a)) {
+                if (!s.nul) s.h = s.h + H1;     // dZndz at w (at L after a full period)
+                s.nul = true;
+            }
+            s.w = 0;
+            if constexpr (KIND == KIND_M2) at_start(s, a);
+            k.reb++;
+        } else if (KIND == KIND_M2 && DZ_ON(a) && edge && !s.nul) {
+            s.Zh = t.dz[s.w];                   // not the wrapped value of the test
+        }
+        return false;
     }
 
     __device__ static void finish(const State &s, const KArgs &a, const KArgs &g, int64_t i, int reason) {
