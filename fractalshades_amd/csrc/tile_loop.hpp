@@ -173,7 +173,7 @@ __device__ __forceinline__ void tile_loop(const KArgs &a) {
     typename Model::State s;
     Counters k = {0, 0, 0, 0, 0};
     unsigned unsure = 0;
-    // Slots.  Wave g's first 64 slots are [64 g, 64 g + 64), without an atomic;
+    // Slots.  Each wave has its first 64 slots (first_slot), without an atomic;
     // a launch with no more slots than lanes needs no other.  The slots past
     // those of all waves are handed out, 64 at a draw, by NC pixel cursors,
     // each in its own 128-byte line: an atomic takes 12-15 ns on its address
@@ -230,7 +230,7 @@ __device__ __forceinline__ void tile_loop(const KArgs &a) {
                 const int64_t left = g.npts - held;                          // the cursors' slots
                 int64_t base = -1;
                 if ((hand & HAND_STARTED) == 0u) {
-                    base = 64 * (int64_t)(blockIdx.x * waves + wave);
+                    base = first_slot(blockIdx.x, wave, gridDim.x);
                     hand |= left > 0 ? HAND_STARTED : HAND_DONE;
                 } else {
                     unsigned long long *const cursors = g.work + WORK_CURSORS + (g.redo ? 16 * NC : 0);

@@ -12,6 +12,7 @@ SOURCE = r"""
 #include "bla_key.hpp"
 #include "slot_rule.hpp"
 extern "C" {
+int64_t first_slot(unsigned block, unsigned wave, unsigned blocks) { return fsg::first_slot(block, wave, blocks); }
 unsigned redo_share(uint64_t unsure, unsigned waves) { return fsg::redo_share(unsure, waves); }
 int slot_goes(unsigned filled, unsigned before) { return fsg::slot_goes(filled, before); }
 int64_t radius_key(double r) { return fsg::radius_key(r); }
@@ -31,7 +32,7 @@ def load():
                         "-I", build.CSRC, src, "-o", lib], check=True, capture_output=True)
         f = ctypes.CDLL(lib)
     i64, u32, dbl = ctypes.c_int64, ctypes.c_uint32, ctypes.c_double
-    for name, args, res in (("redo_share", (ctypes.c_uint64, u32), u32), ("slot_goes", (u32, u32), ctypes.c_int),
+    for name, args, res in (("first_slot", (u32, u32, u32), i64), ("redo_share", (ctypes.c_uint64, u32), u32), ("slot_goes", (u32, u32), ctypes.c_int),
                             ("radius_key", (dbl,), i64), ("modulus_key", (dbl, ctypes.c_int32), i64),
                             ("hypot_key", (dbl, dbl), i64)):
         getattr(f, name).argtypes, getattr(f, name).restype = args, res
