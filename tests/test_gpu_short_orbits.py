@@ -43,7 +43,7 @@ def inputs(orbit, degree, dz, dc, backshift):
 @pytest.mark.gpu
 @pytest.mark.parametrize("tables", ["lds", "global"])
 @pytest.mark.parametrize("degree,dz,dc,backshift", [(2, 1, 1, 0), (2, 0, 1, 0), (2, 1, 0, 0), (2, 0, 0, 0), (2, 1, 1, 2),
-                                                    (3, 1, 1, 0), (3, 0, 1, 0), (3, 1, 1, 3)])
+                                                    (3, 1, 1, 0), (3, 0, 1, 0), (3, 1, 1, 3), (3, 0, 1, 3), (3, 1, 0, 3)])
 @pytest.mark.parametrize("orbit", sorted(ORBITS))
 def test_bitexact(orbit, degree, dz, dc, backshift, tables, monkeypatch):
     print(f"case {orbit} d={degree} dz={dz} dc={dc} backshift={backshift} {tables}", flush=True)
