@@ -1,12 +1,12 @@
 // fsg_kernels.hip -- gfx950 kernels for the per-pixel perturbation loop.
 //
-// k_tile: persistent, work-stealing tile kernel.  Each lane owns one pixel at
-// a time and runs the reference's per-pixel loop (BLA jump, perturbation step,
-// max_iter / interior / escape tests, rebasing); when its pixel stops it
-// writes the results and takes the next pixel index from the pixel cursors.
-// Refill is wave-aggregated: one atomic per wave hands out consecutive indices
-// to all lanes that need work (ballot + mbcnt).  The arithmetic is scalar
-// complex recurrences (no MFMA); the kernel is bound by the FP64 VALU rate.
+// k_tile: persistent, work-stealing tile kernel (tile_loop.hpp).  A wave takes 64
+// pixels, one per lane; each runs the reference's per-pixel loop (BLA jumps,
+// perturbation step, max_iter / interior / escape tests, rebasing).  Once the
+// last of them has stopped, and each lane has written its results, the wave takes the
+// next 64.  Its first slots are its own, later ones come 64 at a draw from the
+// pixel cursors.  The arithmetic is scalar complex recurrences (no MFMA); the
+// kernel is bound by the rate at which vector instructions issue.
 //
 // Reference loops restated here:
 //   holomorphic: numba_iterate, src/fractalshades/perturbation.py:1065-1400

@@ -210,10 +210,11 @@ template <bool HOLO> __device__ bool layers_squares(const PostArgs &p, double zr
     return ok;
 }
 
-// Bound by memory: 53 bytes a pixel (69 with a Jacobian) at 5.1 TB/s are 44 us
-// (58) of a 2048 x 2048 frame, which takes 42 (58) us; the general form on
-// every pixel takes 78 (86) us, three 98-instruction logarithms, four moduli
-// and five quotients of binary64 issue.  One kernel per form of derivative:
+// Bound by memory: 53 bytes a pixel (69 with a Jacobian).  4096 x 4096 pixels,
+// 889 MB, take 174 us, 5.1 TB/s, where a copy of 1 GiB reaches 5.2; a 2048 x 2048
+// frame takes 42 (58) us, 5.3 TB/s: its 222 MB stay in part in the 256 MB cache
+// behind the L2s.  The general form on every pixel takes 78 (86) us there, three
+// 98-instruction logarithms, four moduli and five quotients of binary64 issue.  One kernel per form of derivative:
 // its loads are then unconditional and all in flight together.
 template <bool HOLO> __global__ void __launch_bounds__(256) k_postproc(const PostArgs p) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;

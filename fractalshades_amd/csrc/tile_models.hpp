@@ -394,8 +394,11 @@ struct HoloStd {
 // (and the BLA jump and the rebase for what they read); each keeps one
 // exponent, and a sum shifts its other operand -- c, or the path's term -- to
 // that exponent instead of aligning both on the larger one.  z^2 + c: Z + z
-// and z + 2 Z are formed in binary64 from z's binary64 copy: Z is in range,
-// so a z that underflows there is far below the rounding of the sum.
+// and z + 2 Z are formed in binary64 from z's binary64 copy: |Z| is in range,
+// so a z that underflows there is far below the rounding of the sum's modulus.
+// (Where one component of Z is zero, that component of the sum is z's copy, zero
+// or short of digits below 2^-1022.  A component of a result that is itself below
+// 2^-1022 can then lose digits; moduli do not.)
 // z^d + c: the same for the factors of every binomial term.  Two exceptions
 // leave the straight line: an orbit point below 2^LOW_Z (zero, the Xrange
 // register) or above 2^HIGH_Z, with which the factors take the exponent of

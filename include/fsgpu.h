@@ -197,8 +197,8 @@ int fsg_tile_grid_device(fsg_ctx *ctx, const double *d_c_pix, int64_t n, int64_t
  * reference: for callers that cannot allocate device memory (code under HIP
  * graph capture elsewhere in the process, serving loops that forbid
  * allocation after start-up).  The device staging of the inputs and outputs
- * and the pixel cursor and counters live in a static per-device array of
- * FSG_NOALLOC_SCRATCH_BYTES (32 MiB), held by every device the library runs
+ * lives in a static per-device array of FSG_NOALLOC_SCRATCH_BYTES (32 MiB), the
+ * pixel cursors and counters behind it, held by every device the library runs
  * on until the process ends; its address is taken once per device.  A tile
  * needing more staging than that (about 340,000 pixels with three complex
  * fields) is rejected with FSG_E_RANGE.  Calls on one device share the array
